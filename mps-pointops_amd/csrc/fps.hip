@@ -605,6 +605,47 @@ __device__ __forceinline__ void tile_boxes(const float (&px)[PO], const float (&
     }
 }
 
+// A cut below the largest keys of a wave: lane l holds its two largest keys d1
+// >= d2 (running distance bits ^ sign, so that unsigned order is distance
+// order).  Returns the lanes whose d1 and whose d2 reach a threshold that
+// KC - 1 or KC of the 128 keys reach (fewer where ties leave no such cut), or
+// none when no threshold separates 1 to KC keys at distance 0 or above.  The
+// threshold is found by counting: two ballots a probe, the first probe a
+// quarter of an octave below the largest key m, then outwards by factors of 4
+// until more than KC keys are counted, then by bisection -- about 6 probes of
+// ~60 cycles, in place of KC + 1 dependent wave maxima of ~400.
+struct KeyCut {
+    uint64_t first, second;  // lanes whose d1 / d2 is at or above the cut
+};
+template <int KC>
+__device__ __forceinline__ KeyCut cut_top_keys(uint32_t d1, uint32_t d2, uint32_t m) {
+    constexpr uint32_t kZero = 0x80000000u;  // distance +0
+    KeyCut best{0, 0};
+    if (m < kZero) return best;  // only points that are never sampled
+    uint32_t lo = 0, hi = m + 1;  // more than KC keys at lo (0: not known yet), at most KC at hi
+    uint32_t below = 1u << 21;    // largest key less the next outward probe
+    for (;;) {
+        uint32_t t;
+        if (lo == 0) {
+            t = m - kZero > below ? m - below : kZero;
+            below <<= 2;
+        } else {
+            if (hi - lo <= 1) return best;
+            t = lo + (hi - lo) / 2;
+        }
+        const uint64_t a = ballot(d1 >= t);
+        const uint64_t b = ballot(d2 >= t);
+        const int count = __popcll(a) + __popcll(b);
+        if (count > KC) {
+            lo = t;
+        } else {
+            hi = t;
+            best = {a, b};
+            if (count >= KC - 1 || t == kZero) return best;
+        }
+    }
+}
+
 // fps_lead_kernel<P>: the tiled FPS above with the step chain taken by one
 // wave instead of all of them.
 //
@@ -915,48 +956,54 @@ __global__ __launch_bounds__(kLeadThreads) void fps_lead_kernel(
             };
             uint64_t h1, h2;
             top2(false, 0, h1, h2);
-            uint64_t unknown = 0;
-            int ck = 0, cc = 0x7FFFFFFF;
-            int bound = 0;
-#pragma unroll
-            for (int r = 0; r <= KC; ++r) {
-                const uint32_t hh = static_cast<uint32_t>(h1 >> 32);
-                const uint32_t wv = wave_max_u32_l63(hh);
-                const uint64_t at = ballot(hh == wv);
-                int wl = static_cast<int>(__builtin_ctzll(at));
-                uint32_t wlo;
-                if (__popcll(at) > 1) {
-                    wlo = wave_max_u32_l63(hh == wv ? static_cast<uint32_t>(h1) : 0u);
-                    wl = static_cast<int>(__builtin_ctzll(ballot(hh == wv && static_cast<uint32_t>(h1) == wlo)));
-                } else {
-                    wlo = static_cast<uint32_t>(readlane(static_cast<int>(h1), wl));
+            const uint32_t d1 = static_cast<uint32_t>(h1 >> 32);
+            const uint32_t d2 = static_cast<uint32_t>(h2 >> 32);
+            const uint32_t top = wave_max_u32_l63(d1);
+            const KeyCut cut = cut_top_keys<KC>(d1, d2, top);
+            // A candidate's slot: the cut's lanes in lane order, the d1 first.
+            auto put = [&](int slot, uint64_t key) {
+                const int code = static_cast<int>(~static_cast<uint32_t>(key));
+                const float4 c = spts[code & 0x1FFF];
+                cand_pos[parity][fi * KC + slot] = make_float4(c.x, c.y, c.z, i2f(code >> 13));
+                cand_key[parity][fi * KC + slot] = static_cast<int>(static_cast<uint32_t>(key >> 32) ^ 0x80000000u);
+            };
+            if (cut.first != 0) {
+                const int n1 = __popcll(cut.first);
+                const int count = n1 + __popcll(cut.second);
+                const bool has1 = (cut.first >> lane) & 1u;
+                const bool has2 = (cut.second >> lane) & 1u;
+                if (has1) put(lanes_below(cut.first), h1);
+                // The largest key that this lane keeps to itself.
+                uint32_t rest = has1 ? d2 : d1;
+                if (cut.second != 0) {
+                    if (has2) put(n1 + lanes_below(cut.second), h2);
+                    uint64_t h3, h4;
+                    top2(true, h2, h3, h4);
+                    rest = has2 ? static_cast<uint32_t>(h3 >> 32) : rest;
                 }
-                if (r == KC) {
-                    bound = static_cast<int>(wv ^ 0x80000000u);
-                    break;
+                const uint32_t bound = wave_max_u32_l63(rest);
+                // Unfilled slots: the lowest key, which never wins a step.
+                if (lane >= count && lane < KC) {
+                    cand_pos[parity][fi * KC + lane] = make_float4(0.f, 0.f, 0.f, i2f(INT_MAX >> 13));
+                    cand_key[parity][fi * KC + lane] = INT_MIN;
                 }
-                ck = writelane(ck, static_cast<int>(wv ^ 0x80000000u), r);
-                cc = writelane(cc, static_cast<int>(~wlo), r);
-                const bool won = lane == wl;
-                if ((unknown >> wl) & 1u) {
-                    uint64_t n1, n2;
-                    top2(true, (static_cast<uint64_t>(wv) << 32) | wlo, n1, n2);
-                    h1 = won ? n1 : h1;
-                    h2 = won ? n2 : h2;
-                    unknown &= ~(uint64_t(1) << wl);
-                } else {
-                    h1 = won ? h2 : h1;
-                    unknown |= uint64_t(1) << wl;
+                if (lane == 0) bounds[fi] = static_cast<int>(bound ^ 0x80000000u);
+            } else {
+                // No cut (more than KC points share the largest distance, or
+                // none can be sampled): the follower's best point alone, the
+                // smallest index among the largest keys, and the largest key
+                // as the bound: no later step of the run can
+                // take a key at it.
+                const uint32_t wlo = wave_max_u32_l63(d1 == top ? static_cast<uint32_t>(h1) : 0u);
+                if (lane < KC) {
+                    // A padding code (a follower without points) reads any row.
+                    const int code = static_cast<int>(~wlo);
+                    const float4 c = spts[min(code & 0x1FFF, CAP - 1)];
+                    cand_pos[parity][fi * KC + lane] = make_float4(c.x, c.y, c.z, i2f(code >> 13));
+                    cand_key[parity][fi * KC + lane] = lane == 0 ? static_cast<int>(top ^ 0x80000000u) : INT_MIN;
                 }
+                if (lane == 0) bounds[fi] = static_cast<int>(top ^ 0x80000000u);
             }
-            if (lane < KC) {
-                // Padding codes 0x7FFFFFFF: a published padding key never wins a
-                // step, so any in-range position serves.
-                const float4 c = spts[min(cc & 0x1FFF, CAP - 1)];
-                cand_pos[parity][fi * KC + lane] = make_float4(c.x, c.y, c.z, i2f(cc >> 13));
-                cand_key[parity][fi * KC + lane] = ck;
-            }
-            if (lane == 0) bounds[fi] = bound;
         }
         __syncthreads();  // candidates and bounds published; the last run applied
         if (done[parity]) break;  // uniform: written by the leader before this barrier
