@@ -608,27 +608,31 @@ __device__ __forceinline__ void tile_boxes(const float (&px)[PO], const float (&
 // A cut below the largest keys of a wave: lane l holds its two largest keys d1
 // >= d2 (running distance bits ^ sign, so that unsigned order is distance
 // order).  Returns the lanes whose d1 and whose d2 reach a threshold that
-// KC - 1 or KC of the 128 keys reach (fewer where ties leave no such cut), or
+// KC - 2 to KC of the 128 keys reach (fewer where ties leave no such cut), or
 // none when no threshold separates 1 to KC keys at distance 0 or above.  The
-// threshold is found by counting: two ballots a probe, the first probe a
-// quarter of an octave below the largest key m, then outwards by factors of 4
-// until more than KC keys are counted, then by bisection -- about 6 probes of
-// ~60 cycles, in place of KC + 1 dependent wave maxima of ~400.
+// threshold is found by counting, two ballots a probe, in place of KC + 1
+// dependent wave maxima of ~400 cycles each: the first probe as far below the
+// largest key m as the last exchange's threshold was (`guess`), then twice as
+// far until more than KC keys are counted, then by bisection.  At 32 x 4096
+// points, 1024 samples: 338 us with the maxima, 313 us with a first probe a
+// quarter octave below m and KC - 1 or KC keys wanted, 283 us so (fewer keys
+// shorten the runs: KC - 3 288 us; more probes lengthen the exchange: exactly
+// KC 306 us).
 struct KeyCut {
     uint64_t first, second;  // lanes whose d1 / d2 is at or above the cut
 };
 template <int KC>
-__device__ __forceinline__ KeyCut cut_top_keys(uint32_t d1, uint32_t d2, uint32_t m) {
+__device__ __forceinline__ KeyCut cut_top_keys(uint32_t d1, uint32_t d2, uint32_t m, uint32_t& guess) {
     constexpr uint32_t kZero = 0x80000000u;  // distance +0
     KeyCut best{0, 0};
     if (m < kZero) return best;  // only points that are never sampled
     uint32_t lo = 0, hi = m + 1;  // more than KC keys at lo (0: not known yet), at most KC at hi
-    uint32_t below = 1u << 21;    // largest key less the next outward probe
+    uint32_t below = guess;       // largest key less the next outward probe
     for (;;) {
         uint32_t t;
         if (lo == 0) {
             t = m - kZero > below ? m - below : kZero;
-            below <<= 2;
+            below <<= 1;
         } else {
             if (hi - lo <= 1) return best;
             t = lo + (hi - lo) / 2;
@@ -641,7 +645,10 @@ __device__ __forceinline__ KeyCut cut_top_keys(uint32_t d1, uint32_t d2, uint32_
         } else {
             hi = t;
             best = {a, b};
-            if (count >= KC - 1 || t == kZero) return best;
+            if (count >= KC - 2 || t == kZero) {
+                guess = max(m - t, 1u << 12);
+                return best;
+            }
         }
     }
 }
@@ -650,10 +657,10 @@ __device__ __forceinline__ KeyCut cut_top_keys(uint32_t d1, uint32_t d2, uint32_
 // wave instead of all of them.
 //
 // Nine waves: eight followers (waves 0-7) hold the cloud's 64-point tiles
-// (the setup, tiles and exchanges of fps_tiled_kernel with an even split, P
+// (the setup and tiles of fps_tiled_kernel with an even split, P
 // tiles each) and the leader, wave 8, holds none.  After an exchange (every
-// follower publishes its kLeadCand best points and its bound, the next
-// largest running distance) the leader takes the exact steps of the run on
+// follower publishes up to kLeadCand of its best points and its bound, the
+// largest running distance of the others) the leader takes the exact steps of the run on
 // its own over the 64 candidates: largest key, ties to the smallest index,
 // the candidates updated with the points' own arithmetic, until the chosen
 // key is no longer above every bound.  Its step loop is hand-scheduled
@@ -671,9 +678,10 @@ __device__ __forceinline__ KeyCut cut_top_keys(uint32_t d1, uint32_t d2, uint32_
 // without need only takes a no-op minimum), so one ballot gives the tile
 // masks of all four steps; then the masked tile updates.  Updates may be
 // applied in any order before the next exchange, since running distances
-// are minima.  At the end of a run follower 0 turns the ring's lanes into
+// are minima.  At the end of a run the leader turns the ring's lanes into
 // sample indices (64 per lane permute) and stores them, then publishes the
-// progress words.  A run also ends after kLeadRing steps (the ring's size;
+// progress words, while the followers finish and extract (a follower doing
+// it held up the exchange: 300 -> 293 us).  A run also ends after kLeadRing steps (the ring's size;
 // the ring is rewritten only after the next exchange's barrier, which every
 // follower reaches after reading it).  LDS ordering: one wave's LDS
 // operations complete in issue order, so a follower that reads a published
@@ -743,7 +751,7 @@ __global__ __launch_bounds__(kLeadThreads) void fps_lead_kernel(
     const bool sorter = wave < NS;
     const int fi = wave;  // follower number
     const bool follower = !leader;
-    constexpr int kOutWave = 0;  // the first follower stores the samples
+    constexpr int kOutWave = NS;  // the leader stores the samples, while the followers extract
     const int far0 = static_cast<int>(seg.start);
     // With `centres` set, sample s's coordinates also go to
     // centres[3 (out_lo + s) ..], copied from the cloud.
@@ -932,12 +940,15 @@ __global__ __launch_bounds__(kLeadThreads) void fps_lead_kernel(
     const uint32_t lane_shift = 8u * static_cast<uint32_t>(lane >> 4);
 
     if (leader) __builtin_amdgcn_s_setprio(3);
+    uint32_t cut_guess = 1u << 21;
     int64_t step = 1;
     int parity = 0;
     for (;;) {
         if (follower) {
-            // Exchange: this follower's KC best points and its bound (the
-            // (KC+1)-th), as in fps_tiled_kernel.
+            // Exchange: the points above a cut of this follower's keys (KC - 2
+            // to KC of them), and its bound, the largest running distance it
+            // keeps to itself.  Keys as in fps_tiled_kernel; each lane looks
+            // below its two largest only where both are published.
             auto top2 = [&](bool limited, uint64_t lim, uint64_t& a1, uint64_t& a2) {
                 a1 = 0;
                 a2 = 0;
@@ -959,7 +970,7 @@ __global__ __launch_bounds__(kLeadThreads) void fps_lead_kernel(
             const uint32_t d1 = static_cast<uint32_t>(h1 >> 32);
             const uint32_t d2 = static_cast<uint32_t>(h2 >> 32);
             const uint32_t top = wave_max_u32_l63(d1);
-            const KeyCut cut = cut_top_keys<KC>(d1, d2, top);
+            const KeyCut cut = cut_top_keys<KC>(d1, d2, top, cut_guess);
             // A candidate's slot: the cut's lanes in lane order, the d1 first.
             auto put = [&](int slot, uint64_t key) {
                 const int code = static_cast<int>(~static_cast<uint32_t>(key));
@@ -992,8 +1003,7 @@ __global__ __launch_bounds__(kLeadThreads) void fps_lead_kernel(
                 // No cut (more than KC points share the largest distance, or
                 // none can be sampled): the follower's best point alone, the
                 // smallest index among the largest keys, and the largest key
-                // as the bound: no later step of the run can
-                // take a key at it.
+                // as the bound: no later step of the run can take a key at it.
                 const uint32_t wlo = wave_max_u32_l63(d1 == top ? static_cast<uint32_t>(h1) : 0u);
                 if (lane < KC) {
                     // A padding code (a follower without points) reads any row.
@@ -1048,93 +1058,403 @@ __global__ __launch_bounds__(kLeadThreads) void fps_lead_kernel(
                 // the DPP reduction of wave_max_i32_l63.  It stops after 4
                 // steps (st = 0, wv the next step's key), or when the run
                 // ends (st = 1): no steps left, or the next key is not above
-                // every bound.  The s_nop's give the wait states a DPP read
-                // of a VALU result (2), a readlane of a DPP result (1) and a
-                // VALU read of a readlane's SGPR (2) need.
+                // every bound.  The s_nop's (or scalar work in their place)
+                // give the wait states a DPP read of a VALU result (2), a
+                // readlane of a DPP result (1) and a VALU read of a
+                // readlane's SGPR (2) need.
+                //
+                // A block that cannot use up the steps (rem > 4) is the four
+                // steps written out: no shift count, step counter or loop
+                // branch, the tie test behind the readlanes and the next
+                // comparison ahead of the run's end test, so the chain
+                // cmp - ff1 - readlane - update - maximum waits for nothing
+                // else (a branch or a scalar operation in it costs its issue
+                // time: 313 -> 301 us at 32 x 4096 points, 1024 samples).
                 int st, wl, t, fx, fy, fz;
                 uint64_t tt;
                 float t0, t1, t2;
                 int m;
-                asm volatile(
-                    "s_nop 1\n\t"
-                    "s_mov_b32 %[sh], 0\n\t"
-                    "s_mov_b32 %[pk], 0\n"
-                    "1:\n\t"
-                    "v_cmp_eq_u32_e32 vcc, %[wv], %[cmd]\n\t"
-                    "s_ff1_i32_b64 %[wl], vcc\n\t"
-                    "s_bcnt1_i32_b64 %[t], vcc\n\t"
-                    "s_cmp_gt_u32 %[t], 1\n\t"
-                    "s_cbranch_scc1 5f\n"
-                    "2:\n\t"
-                    "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
-                    "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
-                    "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
-                    "s_lshl_b32 %[t], %[wl], %[sh]\n\t"
-                    "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
-                    "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
-                    "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
-                    "s_or_b32 %[pk], %[pk], %[t]\n\t"
-                    "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
-                    "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
-                    "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
-                    "v_add_f32_e32 %[t0], %[t0], %[t1]\n\t"
-                    "s_add_u32 %[sh], %[sh], 8\n\t"
-                    "v_add_f32_e32 %[t0], %[t0], %[t2]\n\t"
-                    "s_sub_u32 %[rem], %[rem], 1\n\t"
-                    "v_min_f32_e32 %[cmd], %[cmd], %[t0]\n\t"
-                    "s_cmp_eq_u32 %[rem], 0\n\t"
-                    "s_cbranch_scc1 8f\n\t"
-                    "v_max_i32_dpp %[m], %[cmd], %[cmd] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-                    "s_nop 1\n\t"
-                    "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-                    "s_nop 1\n\t"
-                    "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
-                    "s_nop 1\n\t"
-                    "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
-                    "s_nop 1\n\t"
-                    "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
-                    "s_nop 1\n\t"
-                    "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
-                    "s_nop 0\n\t"
-                    "v_readlane_b32 %[wv], %[m], 63\n\t"
-                    "s_cmp_le_i32 %[wv], %[maxb]\n\t"
-                    "s_cbranch_scc1 8f\n\t"
-                    "s_cmp_lt_u32 %[sh], 32\n\t"
-                    "s_cbranch_scc1 1b\n\t"
-                    "s_mov_b32 %[st], 0\n\t"
-                    "s_branch 9f\n"
-                    "5:\n\t"
-                    "v_cndmask_b32_e32 %[m], %[imin], %[nidx], vcc\n\t"
-                    "s_nop 1\n\t"
-                    "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-                    "s_nop 1\n\t"
-                    "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-                    "s_nop 1\n\t"
-                    "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
-                    "s_nop 1\n\t"
-                    "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
-                    "s_nop 1\n\t"
-                    "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
-                    "s_nop 1\n\t"
-                    "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
-                    "s_nop 0\n\t"
-                    "v_readlane_b32 %[t], %[m], 63\n\t"
-                    "s_nop 1\n\t"
-                    "v_cmp_eq_u32_e64 %[tt], %[t], %[nidx]\n\t"
-                    "s_and_b64 vcc, vcc, %[tt]\n\t"
-                    "s_ff1_i32_b64 %[wl], vcc\n\t"
-                    "s_branch 2b\n"
-                    "8:\n\t"
-                    "s_mov_b32 %[st], 1\n"
-                    "9:\n\t"
-                    "s_nop 1"
-                    : [cmd] "+v"(cmd), [wv] "+s"(wv), [rem] "+s"(rem), [pk] "=&s"(packed),
-                      [sh] "=&s"(sh), [st] "=&s"(st), [wl] "=&s"(wl), [t] "=&s"(t),
-                      [fx] "=&s"(fx), [fy] "=&s"(fy), [fz] "=&s"(fz), [tt] "=&s"(tt),
-                      [t0] "=&v"(t0), [t1] "=&v"(t1), [t2] "=&v"(t2), [m] "=&v"(m)
-                    : [cx] "v"(ccx), [cy] "v"(ccy), [cz] "v"(ccz), [nidx] "v"(nidx),
-                      [imin] "v"(imin), [maxb] "s"(maxb)
-                    : "vcc", "scc");
+                if (rem > 4) {
+                    asm volatile(
+                        "s_nop 1\n\t"
+                        "v_cmp_eq_u32_e32 vcc, %[wv], %[cmd]\n\t"
+                        "s_ff1_i32_b64 %[wl], vcc\n\t"
+                        "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
+                        "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
+                        "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
+                        "s_bcnt1_i32_b64 %[t], vcc\n\t"
+                        "s_cmp_gt_u32 %[t], 1\n\t"
+                        "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
+                        "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
+                        "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
+                        "s_cbranch_scc1 50f\n\t"
+                        "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
+                        "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
+                        "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
+                        "20:\n\t"
+                        "v_add_f32_e32 %[t0], %[t0], %[t1]\n\t"
+                        "v_add_f32_e32 %[t0], %[t0], %[t2]\n\t"
+                        "v_min_f32_e32 %[cmd], %[cmd], %[t0]\n\t"
+                        "s_mov_b32 %[pk], %[wl]\n\t"
+                        "s_nop 0\n\t"
+                        "v_max_i32_dpp %[m], %[cmd], %[cmd] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+                        "s_nop 0\n\t"
+                        "v_readlane_b32 %[wv], %[m], 63\n\t"
+                        "s_cmp_le_i32 %[wv], %[maxb]\n\t"
+                        "s_nop 0\n\t"
+                        "v_cmp_eq_u32_e32 vcc, %[wv], %[cmd]\n\t"
+                        "s_cbranch_scc1 80f\n\t"
+                        "s_ff1_i32_b64 %[wl], vcc\n\t"
+                        "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
+                        "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
+                        "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
+                        "s_bcnt1_i32_b64 %[t], vcc\n\t"
+                        "s_cmp_gt_u32 %[t], 1\n\t"
+                        "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
+                        "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
+                        "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
+                        "s_cbranch_scc1 51f\n\t"
+                        "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
+                        "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
+                        "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
+                        "21:\n\t"
+                        "v_add_f32_e32 %[t0], %[t0], %[t1]\n\t"
+                        "s_lshl_b32 %[t], %[wl], 8\n\t"
+                        "v_add_f32_e32 %[t0], %[t0], %[t2]\n\t"
+                        "v_min_f32_e32 %[cmd], %[cmd], %[t0]\n\t"
+                        "s_or_b32 %[pk], %[pk], %[t]\n\t"
+                        "s_nop 0\n\t"
+                        "v_max_i32_dpp %[m], %[cmd], %[cmd] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+                        "s_nop 0\n\t"
+                        "v_readlane_b32 %[wv], %[m], 63\n\t"
+                        "s_cmp_le_i32 %[wv], %[maxb]\n\t"
+                        "s_nop 0\n\t"
+                        "v_cmp_eq_u32_e32 vcc, %[wv], %[cmd]\n\t"
+                        "s_cbranch_scc1 81f\n\t"
+                        "s_ff1_i32_b64 %[wl], vcc\n\t"
+                        "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
+                        "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
+                        "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
+                        "s_bcnt1_i32_b64 %[t], vcc\n\t"
+                        "s_cmp_gt_u32 %[t], 1\n\t"
+                        "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
+                        "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
+                        "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
+                        "s_cbranch_scc1 52f\n\t"
+                        "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
+                        "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
+                        "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
+                        "22:\n\t"
+                        "v_add_f32_e32 %[t0], %[t0], %[t1]\n\t"
+                        "s_lshl_b32 %[t], %[wl], 16\n\t"
+                        "v_add_f32_e32 %[t0], %[t0], %[t2]\n\t"
+                        "v_min_f32_e32 %[cmd], %[cmd], %[t0]\n\t"
+                        "s_or_b32 %[pk], %[pk], %[t]\n\t"
+                        "s_nop 0\n\t"
+                        "v_max_i32_dpp %[m], %[cmd], %[cmd] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+                        "s_nop 0\n\t"
+                        "v_readlane_b32 %[wv], %[m], 63\n\t"
+                        "s_cmp_le_i32 %[wv], %[maxb]\n\t"
+                        "s_nop 0\n\t"
+                        "v_cmp_eq_u32_e32 vcc, %[wv], %[cmd]\n\t"
+                        "s_cbranch_scc1 82f\n\t"
+                        "s_ff1_i32_b64 %[wl], vcc\n\t"
+                        "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
+                        "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
+                        "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
+                        "s_bcnt1_i32_b64 %[t], vcc\n\t"
+                        "s_cmp_gt_u32 %[t], 1\n\t"
+                        "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
+                        "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
+                        "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
+                        "s_cbranch_scc1 53f\n\t"
+                        "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
+                        "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
+                        "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
+                        "23:\n\t"
+                        "v_add_f32_e32 %[t0], %[t0], %[t1]\n\t"
+                        "s_lshl_b32 %[t], %[wl], 24\n\t"
+                        "v_add_f32_e32 %[t0], %[t0], %[t2]\n\t"
+                        "v_min_f32_e32 %[cmd], %[cmd], %[t0]\n\t"
+                        "s_or_b32 %[pk], %[pk], %[t]\n\t"
+                        "s_nop 0\n\t"
+                        "v_max_i32_dpp %[m], %[cmd], %[cmd] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+                        "s_nop 0\n\t"
+                        "v_readlane_b32 %[wv], %[m], 63\n\t"
+                        "s_cmp_le_i32 %[wv], %[maxb]\n\t"
+                        "s_cbranch_scc1 83f\n\t"
+                        "s_mov_b32 %[st], 0\n\t"
+                        "s_mov_b32 %[sh], 32\n\t"
+                        "s_branch 9f\n\t"
+                        "50:\n\t"
+                        "v_cndmask_b32_e32 %[m], %[imin], %[nidx], vcc\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_readlane_b32 %[t], %[m], 63\n\t"
+                        "s_nop 1\n\t"
+                        "v_cmp_eq_u32_e64 %[tt], %[t], %[nidx]\n\t"
+                        "s_and_b64 vcc, vcc, %[tt]\n\t"
+                        "s_ff1_i32_b64 %[wl], vcc\n\t"
+                        "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
+                        "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
+                        "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
+                        "s_nop 1\n\t"
+                        "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
+                        "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
+                        "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
+                        "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
+                        "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
+                        "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
+                        "s_branch 20b\n\t"
+                        "51:\n\t"
+                        "v_cndmask_b32_e32 %[m], %[imin], %[nidx], vcc\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_readlane_b32 %[t], %[m], 63\n\t"
+                        "s_nop 1\n\t"
+                        "v_cmp_eq_u32_e64 %[tt], %[t], %[nidx]\n\t"
+                        "s_and_b64 vcc, vcc, %[tt]\n\t"
+                        "s_ff1_i32_b64 %[wl], vcc\n\t"
+                        "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
+                        "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
+                        "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
+                        "s_nop 1\n\t"
+                        "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
+                        "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
+                        "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
+                        "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
+                        "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
+                        "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
+                        "s_branch 21b\n\t"
+                        "52:\n\t"
+                        "v_cndmask_b32_e32 %[m], %[imin], %[nidx], vcc\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_readlane_b32 %[t], %[m], 63\n\t"
+                        "s_nop 1\n\t"
+                        "v_cmp_eq_u32_e64 %[tt], %[t], %[nidx]\n\t"
+                        "s_and_b64 vcc, vcc, %[tt]\n\t"
+                        "s_ff1_i32_b64 %[wl], vcc\n\t"
+                        "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
+                        "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
+                        "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
+                        "s_nop 1\n\t"
+                        "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
+                        "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
+                        "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
+                        "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
+                        "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
+                        "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
+                        "s_branch 22b\n\t"
+                        "53:\n\t"
+                        "v_cndmask_b32_e32 %[m], %[imin], %[nidx], vcc\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_readlane_b32 %[t], %[m], 63\n\t"
+                        "s_nop 1\n\t"
+                        "v_cmp_eq_u32_e64 %[tt], %[t], %[nidx]\n\t"
+                        "s_and_b64 vcc, vcc, %[tt]\n\t"
+                        "s_ff1_i32_b64 %[wl], vcc\n\t"
+                        "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
+                        "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
+                        "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
+                        "s_nop 1\n\t"
+                        "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
+                        "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
+                        "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
+                        "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
+                        "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
+                        "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
+                        "s_branch 23b\n\t"
+                        "80:\n\t"
+                        "s_movk_i32 %[sh], 8\n\t"
+                        "s_branch 88f\n\t"
+                        "81:\n\t"
+                        "s_movk_i32 %[sh], 16\n\t"
+                        "s_branch 88f\n\t"
+                        "82:\n\t"
+                        "s_movk_i32 %[sh], 24\n\t"
+                        "s_branch 88f\n\t"
+                        "83:\n\t"
+                        "s_movk_i32 %[sh], 32\n\t"
+                        "88:\n\t"
+                        "s_mov_b32 %[st], 1\n\t"
+                        "9:\n\t"
+                        "s_nop 1\n\t"
+                        : [cmd] "+v"(cmd), [wv] "+s"(wv), [pk] "=&s"(packed),
+                          [sh] "=&s"(sh), [st] "=&s"(st), [wl] "=&s"(wl), [t] "=&s"(t),
+                          [fx] "=&s"(fx), [fy] "=&s"(fy), [fz] "=&s"(fz), [tt] "=&s"(tt),
+                          [t0] "=&v"(t0), [t1] "=&v"(t1), [t2] "=&v"(t2), [m] "=&v"(m)
+                        : [cx] "v"(ccx), [cy] "v"(ccy), [cz] "v"(ccz), [nidx] "v"(nidx),
+                          [imin] "v"(imin), [maxb] "s"(maxb)
+                        : "vcc", "scc");
+                    rem -= 4;
+                } else {
+                    asm volatile(
+                        "s_nop 1\n\t"
+                        "s_mov_b32 %[sh], 0\n\t"
+                        "s_mov_b32 %[pk], 0\n"
+                        "1:\n\t"
+                        "v_cmp_eq_u32_e32 vcc, %[wv], %[cmd]\n\t"
+                        "s_ff1_i32_b64 %[wl], vcc\n\t"
+                        "s_bcnt1_i32_b64 %[t], vcc\n\t"
+                        "s_cmp_gt_u32 %[t], 1\n\t"
+                        "s_cbranch_scc1 5f\n"
+                        "2:\n\t"
+                        "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
+                        "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
+                        "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
+                        "s_lshl_b32 %[t], %[wl], %[sh]\n\t"
+                        "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
+                        "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
+                        "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
+                        "s_or_b32 %[pk], %[pk], %[t]\n\t"
+                        "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
+                        "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
+                        "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
+                        "v_add_f32_e32 %[t0], %[t0], %[t1]\n\t"
+                        "s_add_u32 %[sh], %[sh], 8\n\t"
+                        "v_add_f32_e32 %[t0], %[t0], %[t2]\n\t"
+                        "s_sub_u32 %[rem], %[rem], 1\n\t"
+                        "v_min_f32_e32 %[cmd], %[cmd], %[t0]\n\t"
+                        "s_cmp_eq_u32 %[rem], 0\n\t"
+                        "s_cbranch_scc1 8f\n\t"
+                        "v_max_i32_dpp %[m], %[cmd], %[cmd] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+                        "s_nop 0\n\t"
+                        "v_readlane_b32 %[wv], %[m], 63\n\t"
+                        "s_cmp_le_i32 %[wv], %[maxb]\n\t"
+                        "s_cbranch_scc1 8f\n\t"
+                        "s_cmp_lt_u32 %[sh], 32\n\t"
+                        "s_cbranch_scc1 1b\n\t"
+                        "s_mov_b32 %[st], 0\n\t"
+                        "s_branch 9f\n"
+                        "5:\n\t"
+                        "v_cndmask_b32_e32 %[m], %[imin], %[nidx], vcc\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+                        "s_nop 1\n\t"
+                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+                        "s_nop 0\n\t"
+                        "v_readlane_b32 %[t], %[m], 63\n\t"
+                        "s_nop 1\n\t"
+                        "v_cmp_eq_u32_e64 %[tt], %[t], %[nidx]\n\t"
+                        "s_and_b64 vcc, vcc, %[tt]\n\t"
+                        "s_ff1_i32_b64 %[wl], vcc\n\t"
+                        "s_branch 2b\n"
+                        "8:\n\t"
+                        "s_mov_b32 %[st], 1\n"
+                        "9:\n\t"
+                        "s_nop 1"
+                        : [cmd] "+v"(cmd), [wv] "+s"(wv), [rem] "+s"(rem), [pk] "=&s"(packed),
+                          [sh] "=&s"(sh), [st] "=&s"(st), [wl] "=&s"(wl), [t] "=&s"(t),
+                          [fx] "=&s"(fx), [fy] "=&s"(fy), [fz] "=&s"(fz), [tt] "=&s"(tt),
+                          [t0] "=&v"(t0), [t1] "=&v"(t1), [t2] "=&v"(t2), [m] "=&v"(m)
+                        : [cx] "v"(ccx), [cy] "v"(ccy), [cz] "v"(ccz), [nidx] "v"(nidx),
+                          [imin] "v"(imin), [maxb] "s"(maxb)
+                        : "vcc", "scc");
+                }
                 taken += static_cast<int>(sh >> 3);
                 if (st != 0) break;
                 // A full block: its row, then the count.  Lane l writes word l
@@ -1154,6 +1474,27 @@ __global__ __launch_bounds__(kLeadThreads) void fps_lead_kernel(
             // never sees an end beyond the count it reads with it).
             __hip_atomic_store(&marks[lane], lane < 2 ? base + taken : 0u, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_WORKGROUP);
+            // The run's samples: lane i of a batch takes step c0 + i, its
+            // chosen lane from the ring's bytes and that candidate's index
+            // by a lane permute (all lanes take part).
+            for (int c0 = 0; c0 < taken; c0 += kWave) {
+                const int si = min(c0 + lane, taken - 1);
+                const int wl = reinterpret_cast<const uint8_t*>(ring[si >> 2])[si & 3];
+                const int idx = __builtin_amdgcn_ds_bpermute(wl << 2, f2i(mine.w));
+                if (c0 + lane < taken) o[run_start + c0 + lane] = seg.base + idx;
+                if (oc != nullptr) {
+                    const int x = __builtin_amdgcn_ds_bpermute(wl << 2, f2i(mine.x));
+                    const int y = __builtin_amdgcn_ds_bpermute(wl << 2, f2i(mine.y));
+                    const int z = __builtin_amdgcn_ds_bpermute(wl << 2, f2i(mine.z));
+                    if (c0 + lane < taken) {
+                        float* c = oc + 3 * (run_start + c0 + lane);
+                        c[0] = i2f(x);
+                        c[1] = i2f(y);
+                        c[2] = i2f(z);
+                    }
+                }
+            }
+            publish(run_start, step);
         } else if (follower) {
             // A block of up to 4 published steps, all box tests at once: lane
             // l takes tile l % 16 (a follower holds at most 16) and step
@@ -1216,32 +1557,9 @@ __global__ __launch_bounds__(kLeadThreads) void fps_lead_kernel(
                     }
                     break;
                 }
-                __builtin_amdgcn_s_sleep(1);
-            }
-            if (wave == kOutWave) {
-                // The run's samples: lane i of a batch takes step c0 + i, its
-                // chosen lane from the ring's bytes and that candidate's index
-                // by a lane permute (all lanes take part).
-                for (int c0 = 0; c0 < a; c0 += kWave) {
-                    const int si = min(c0 + lane, a - 1);
-                    const int wl = reinterpret_cast<const uint8_t*>(ring[si >> 2])[si & 3];
-                    const int idx = __builtin_amdgcn_ds_bpermute(wl << 2, f2i(mine.w));
-                    if (c0 + lane < a) o[run_start + c0 + lane] = seg.base + idx;
-                    if (oc != nullptr) {
-                        const int x = __builtin_amdgcn_ds_bpermute(wl << 2, f2i(mine.x));
-                        const int y = __builtin_amdgcn_ds_bpermute(wl << 2, f2i(mine.y));
-                        const int z = __builtin_amdgcn_ds_bpermute(wl << 2, f2i(mine.z));
-                        if (c0 + lane < a) {
-                            float* c = oc + 3 * (run_start + c0 + lane);
-                            c[0] = i2f(x);
-                            c[1] = i2f(y);
-                            c[2] = i2f(z);
-                        }
-                    }
-                }
+                __builtin_amdgcn_s_sleep(0);
             }
             step = run_start + a;
-            publish(run_start, step);
         }
         parity ^= 1;
     }
