@@ -21,6 +21,9 @@
 //                           64-point tiles so that a step updates only the
 //                           tiles it can change; exact steps over 64
 //                           published candidates between exchanges.
+//   fps_wide_kernel         the leader scheme for clouds of up to 24576 points
+//                           of a batch: running distances in LDS, sorted
+//                           points in a caller-provided scratch array.
 //   fps_global_kernel<T>    one workgroup per cloud for larger clouds of a
 //                           batch: points re-read from L2, running distances
 //                           in a caller-provided scratch array.
@@ -605,9 +608,421 @@ __device__ __forceinline__ void tile_boxes(const float (&px)[PO], const float (&
     }
 }
 
+// Up to 4 steps (one block), as hand-scheduled gfx950 code:
+// the chosen candidate (the lowest lane holding the largest
+// key wv; on a tie, the smallest index by a second wave
+// maximum of -index), its coordinates by readlane, every
+// candidate's key lowered to its distance to them, the lane
+// packed into `packed`, then the next step's largest key by
+// the DPP reduction of wave_max_i32_l63.  It stops after 4
+// steps (st = 0, wv the next step's key), or when the run
+// ends (st = 1): no steps left, or the next key is not above
+// every bound.  The s_nop's (or scalar work in their place)
+// give the wait states a DPP read of a VALU result (2), a
+// readlane of a DPP result (1) and a VALU read of a
+// readlane's SGPR (2) need.
+//
+// A block that cannot use up the steps (rem > 4) is the four
+// steps written out: no shift count, step counter or loop
+// branch, the tie test behind the readlanes and the next
+// comparison ahead of the run's end test, so the chain
+// cmp - ff1 - readlane - update - maximum waits for nothing
+// else (a branch or a scalar operation in it costs its issue
+// time: 313 -> 301 us at 32 x 4096 points, 1024 samples).
+__device__ __forceinline__ int lead_block(int& cmd, int& wv, int& rem, uint32_t& packed, uint32_t& sh,
+                                          float ccx, float ccy, float ccz, int nidx, int maxb) {
+    const int imin = INT_MIN;
+    int st, wl, t, fx, fy, fz;
+    uint64_t tt;
+    float t0, t1, t2;
+    int m;
+    if (rem > 4) {
+        asm volatile(
+            "s_nop 1\n\t"
+            "v_cmp_eq_u32_e32 vcc, %[wv], %[cmd]\n\t"
+            "s_ff1_i32_b64 %[wl], vcc\n\t"
+            "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
+            "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
+            "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
+            "s_bcnt1_i32_b64 %[t], vcc\n\t"
+            "s_cmp_gt_u32 %[t], 1\n\t"
+            "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
+            "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
+            "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
+            "s_cbranch_scc1 50f\n\t"
+            "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
+            "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
+            "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
+            "20:\n\t"
+            "v_add_f32_e32 %[t0], %[t0], %[t1]\n\t"
+            "v_add_f32_e32 %[t0], %[t0], %[t2]\n\t"
+            "v_min_f32_e32 %[cmd], %[cmd], %[t0]\n\t"
+            "s_mov_b32 %[pk], %[wl]\n\t"
+            "s_nop 0\n\t"
+            "v_max_i32_dpp %[m], %[cmd], %[cmd] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+            "s_nop 0\n\t"
+            "v_readlane_b32 %[wv], %[m], 63\n\t"
+            "s_cmp_le_i32 %[wv], %[maxb]\n\t"
+            "s_nop 0\n\t"
+            "v_cmp_eq_u32_e32 vcc, %[wv], %[cmd]\n\t"
+            "s_cbranch_scc1 80f\n\t"
+            "s_ff1_i32_b64 %[wl], vcc\n\t"
+            "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
+            "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
+            "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
+            "s_bcnt1_i32_b64 %[t], vcc\n\t"
+            "s_cmp_gt_u32 %[t], 1\n\t"
+            "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
+            "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
+            "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
+            "s_cbranch_scc1 51f\n\t"
+            "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
+            "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
+            "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
+            "21:\n\t"
+            "v_add_f32_e32 %[t0], %[t0], %[t1]\n\t"
+            "s_lshl_b32 %[t], %[wl], 8\n\t"
+            "v_add_f32_e32 %[t0], %[t0], %[t2]\n\t"
+            "v_min_f32_e32 %[cmd], %[cmd], %[t0]\n\t"
+            "s_or_b32 %[pk], %[pk], %[t]\n\t"
+            "s_nop 0\n\t"
+            "v_max_i32_dpp %[m], %[cmd], %[cmd] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+            "s_nop 0\n\t"
+            "v_readlane_b32 %[wv], %[m], 63\n\t"
+            "s_cmp_le_i32 %[wv], %[maxb]\n\t"
+            "s_nop 0\n\t"
+            "v_cmp_eq_u32_e32 vcc, %[wv], %[cmd]\n\t"
+            "s_cbranch_scc1 81f\n\t"
+            "s_ff1_i32_b64 %[wl], vcc\n\t"
+            "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
+            "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
+            "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
+            "s_bcnt1_i32_b64 %[t], vcc\n\t"
+            "s_cmp_gt_u32 %[t], 1\n\t"
+            "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
+            "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
+            "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
+            "s_cbranch_scc1 52f\n\t"
+            "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
+            "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
+            "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
+            "22:\n\t"
+            "v_add_f32_e32 %[t0], %[t0], %[t1]\n\t"
+            "s_lshl_b32 %[t], %[wl], 16\n\t"
+            "v_add_f32_e32 %[t0], %[t0], %[t2]\n\t"
+            "v_min_f32_e32 %[cmd], %[cmd], %[t0]\n\t"
+            "s_or_b32 %[pk], %[pk], %[t]\n\t"
+            "s_nop 0\n\t"
+            "v_max_i32_dpp %[m], %[cmd], %[cmd] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+            "s_nop 0\n\t"
+            "v_readlane_b32 %[wv], %[m], 63\n\t"
+            "s_cmp_le_i32 %[wv], %[maxb]\n\t"
+            "s_nop 0\n\t"
+            "v_cmp_eq_u32_e32 vcc, %[wv], %[cmd]\n\t"
+            "s_cbranch_scc1 82f\n\t"
+            "s_ff1_i32_b64 %[wl], vcc\n\t"
+            "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
+            "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
+            "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
+            "s_bcnt1_i32_b64 %[t], vcc\n\t"
+            "s_cmp_gt_u32 %[t], 1\n\t"
+            "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
+            "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
+            "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
+            "s_cbranch_scc1 53f\n\t"
+            "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
+            "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
+            "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
+            "23:\n\t"
+            "v_add_f32_e32 %[t0], %[t0], %[t1]\n\t"
+            "s_lshl_b32 %[t], %[wl], 24\n\t"
+            "v_add_f32_e32 %[t0], %[t0], %[t2]\n\t"
+            "v_min_f32_e32 %[cmd], %[cmd], %[t0]\n\t"
+            "s_or_b32 %[pk], %[pk], %[t]\n\t"
+            "s_nop 0\n\t"
+            "v_max_i32_dpp %[m], %[cmd], %[cmd] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+            "s_nop 0\n\t"
+            "v_readlane_b32 %[wv], %[m], 63\n\t"
+            "s_cmp_le_i32 %[wv], %[maxb]\n\t"
+            "s_cbranch_scc1 83f\n\t"
+            "s_mov_b32 %[st], 0\n\t"
+            "s_mov_b32 %[sh], 32\n\t"
+            "s_branch 9f\n\t"
+            "50:\n\t"
+            "v_cndmask_b32_e32 %[m], %[imin], %[nidx], vcc\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_readlane_b32 %[t], %[m], 63\n\t"
+            "s_nop 1\n\t"
+            "v_cmp_eq_u32_e64 %[tt], %[t], %[nidx]\n\t"
+            "s_and_b64 vcc, vcc, %[tt]\n\t"
+            "s_ff1_i32_b64 %[wl], vcc\n\t"
+            "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
+            "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
+            "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
+            "s_nop 1\n\t"
+            "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
+            "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
+            "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
+            "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
+            "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
+            "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
+            "s_branch 20b\n\t"
+            "51:\n\t"
+            "v_cndmask_b32_e32 %[m], %[imin], %[nidx], vcc\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_readlane_b32 %[t], %[m], 63\n\t"
+            "s_nop 1\n\t"
+            "v_cmp_eq_u32_e64 %[tt], %[t], %[nidx]\n\t"
+            "s_and_b64 vcc, vcc, %[tt]\n\t"
+            "s_ff1_i32_b64 %[wl], vcc\n\t"
+            "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
+            "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
+            "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
+            "s_nop 1\n\t"
+            "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
+            "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
+            "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
+            "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
+            "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
+            "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
+            "s_branch 21b\n\t"
+            "52:\n\t"
+            "v_cndmask_b32_e32 %[m], %[imin], %[nidx], vcc\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_readlane_b32 %[t], %[m], 63\n\t"
+            "s_nop 1\n\t"
+            "v_cmp_eq_u32_e64 %[tt], %[t], %[nidx]\n\t"
+            "s_and_b64 vcc, vcc, %[tt]\n\t"
+            "s_ff1_i32_b64 %[wl], vcc\n\t"
+            "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
+            "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
+            "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
+            "s_nop 1\n\t"
+            "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
+            "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
+            "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
+            "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
+            "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
+            "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
+            "s_branch 22b\n\t"
+            "53:\n\t"
+            "v_cndmask_b32_e32 %[m], %[imin], %[nidx], vcc\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_readlane_b32 %[t], %[m], 63\n\t"
+            "s_nop 1\n\t"
+            "v_cmp_eq_u32_e64 %[tt], %[t], %[nidx]\n\t"
+            "s_and_b64 vcc, vcc, %[tt]\n\t"
+            "s_ff1_i32_b64 %[wl], vcc\n\t"
+            "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
+            "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
+            "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
+            "s_nop 1\n\t"
+            "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
+            "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
+            "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
+            "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
+            "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
+            "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
+            "s_branch 23b\n\t"
+            "80:\n\t"
+            "s_movk_i32 %[sh], 8\n\t"
+            "s_branch 88f\n\t"
+            "81:\n\t"
+            "s_movk_i32 %[sh], 16\n\t"
+            "s_branch 88f\n\t"
+            "82:\n\t"
+            "s_movk_i32 %[sh], 24\n\t"
+            "s_branch 88f\n\t"
+            "83:\n\t"
+            "s_movk_i32 %[sh], 32\n\t"
+            "88:\n\t"
+            "s_mov_b32 %[st], 1\n\t"
+            "9:\n\t"
+            "s_nop 1\n\t"
+            : [cmd] "+v"(cmd), [wv] "+s"(wv), [pk] "=&s"(packed),
+              [sh] "=&s"(sh), [st] "=&s"(st), [wl] "=&s"(wl), [t] "=&s"(t),
+              [fx] "=&s"(fx), [fy] "=&s"(fy), [fz] "=&s"(fz), [tt] "=&s"(tt),
+              [t0] "=&v"(t0), [t1] "=&v"(t1), [t2] "=&v"(t2), [m] "=&v"(m)
+            : [cx] "v"(ccx), [cy] "v"(ccy), [cz] "v"(ccz), [nidx] "v"(nidx),
+              [imin] "v"(imin), [maxb] "s"(maxb)
+            : "vcc", "scc");
+        rem -= 4;
+    } else {
+        asm volatile(
+            "s_nop 1\n\t"
+            "s_mov_b32 %[sh], 0\n\t"
+            "s_mov_b32 %[pk], 0\n"
+            "1:\n\t"
+            "v_cmp_eq_u32_e32 vcc, %[wv], %[cmd]\n\t"
+            "s_ff1_i32_b64 %[wl], vcc\n\t"
+            "s_bcnt1_i32_b64 %[t], vcc\n\t"
+            "s_cmp_gt_u32 %[t], 1\n\t"
+            "s_cbranch_scc1 5f\n"
+            "2:\n\t"
+            "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
+            "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
+            "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
+            "s_lshl_b32 %[t], %[wl], %[sh]\n\t"
+            "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
+            "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
+            "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
+            "s_or_b32 %[pk], %[pk], %[t]\n\t"
+            "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
+            "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
+            "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
+            "v_add_f32_e32 %[t0], %[t0], %[t1]\n\t"
+            "s_add_u32 %[sh], %[sh], 8\n\t"
+            "v_add_f32_e32 %[t0], %[t0], %[t2]\n\t"
+            "s_sub_u32 %[rem], %[rem], 1\n\t"
+            "v_min_f32_e32 %[cmd], %[cmd], %[t0]\n\t"
+            "s_cmp_eq_u32 %[rem], 0\n\t"
+            "s_cbranch_scc1 8f\n\t"
+            "v_max_i32_dpp %[m], %[cmd], %[cmd] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+            "s_nop 0\n\t"
+            "v_readlane_b32 %[wv], %[m], 63\n\t"
+            "s_cmp_le_i32 %[wv], %[maxb]\n\t"
+            "s_cbranch_scc1 8f\n\t"
+            "s_cmp_lt_u32 %[sh], 32\n\t"
+            "s_cbranch_scc1 1b\n\t"
+            "s_mov_b32 %[st], 0\n\t"
+            "s_branch 9f\n"
+            "5:\n\t"
+            "v_cndmask_b32_e32 %[m], %[imin], %[nidx], vcc\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+            "s_nop 0\n\t"
+            "v_readlane_b32 %[t], %[m], 63\n\t"
+            "s_nop 1\n\t"
+            "v_cmp_eq_u32_e64 %[tt], %[t], %[nidx]\n\t"
+            "s_and_b64 vcc, vcc, %[tt]\n\t"
+            "s_ff1_i32_b64 %[wl], vcc\n\t"
+            "s_branch 2b\n"
+            "8:\n\t"
+            "s_mov_b32 %[st], 1\n"
+            "9:\n\t"
+            "s_nop 1"
+            : [cmd] "+v"(cmd), [wv] "+s"(wv), [rem] "+s"(rem), [pk] "=&s"(packed),
+              [sh] "=&s"(sh), [st] "=&s"(st), [wl] "=&s"(wl), [t] "=&s"(t),
+              [fx] "=&s"(fx), [fy] "=&s"(fy), [fz] "=&s"(fz), [tt] "=&s"(tt),
+              [t0] "=&v"(t0), [t1] "=&v"(t1), [t2] "=&v"(t2), [m] "=&v"(m)
+            : [cx] "v"(ccx), [cy] "v"(ccy), [cz] "v"(ccz), [nidx] "v"(nidx),
+              [imin] "v"(imin), [maxb] "s"(maxb)
+            : "vcc", "scc");
+    }
+    return st;
+}
+
 // A cut below the largest keys of a wave: lane l holds its two largest keys d1
-// >= d2 (running distance bits ^ sign, so that unsigned order is distance
-// order).  Returns the lanes whose d1 and whose d2 reach a threshold that
+// >= d2 (running distance bits as signed integers: in distance order from 0
+// up, and -inf is negative).  Returns the lanes whose d1 and whose d2 reach a threshold that
 // KC - 2 to KC of the 128 keys reach (fewer where ties leave no such cut), or
 // none when no threshold separates 1 to KC keys at distance 0 or above.  The
 // threshold is found by counting, two ballots a probe, in place of KC + 1
@@ -622,16 +1037,15 @@ struct KeyCut {
     uint64_t first, second;  // lanes whose d1 / d2 is at or above the cut
 };
 template <int KC>
-__device__ __forceinline__ KeyCut cut_top_keys(uint32_t d1, uint32_t d2, uint32_t m, uint32_t& guess) {
-    constexpr uint32_t kZero = 0x80000000u;  // distance +0
+__device__ __forceinline__ KeyCut cut_top_keys(int d1, int d2, int m, uint32_t& guess) {
     KeyCut best{0, 0};
-    if (m < kZero) return best;  // only points that are never sampled
-    uint32_t lo = 0, hi = m + 1;  // more than KC keys at lo (0: not known yet), at most KC at hi
-    uint32_t below = guess;       // largest key less the next outward probe
+    if (m < 0) return best;  // only points that are never sampled
+    int lo = -1, hi = m + 1;  // more than KC keys at lo (-1: not known yet), at most KC at hi
+    uint32_t below = guess;   // largest key less the next outward probe
     for (;;) {
-        uint32_t t;
-        if (lo == 0) {
-            t = m - kZero > below ? m - below : kZero;
+        int t;
+        if (lo < 0) {
+            t = static_cast<uint32_t>(m) > below ? m - static_cast<int>(below) : 0;
             below <<= 1;
         } else {
             if (hi - lo <= 1) return best;
@@ -645,8 +1059,8 @@ __device__ __forceinline__ KeyCut cut_top_keys(uint32_t d1, uint32_t d2, uint32_
         } else {
             hi = t;
             best = {a, b};
-            if (count >= KC - 2 || t == kZero) {
-                guess = max(m - t, 1u << 12);
+            if (count >= KC - 2 || t == 0) {
+                guess = max(static_cast<uint32_t>(m - t), 1u << 12);
                 return best;
             }
         }
@@ -949,71 +1363,56 @@ __global__ __launch_bounds__(kLeadThreads) void fps_lead_kernel(
             // to KC of them), and its bound, the largest running distance it
             // keeps to itself.  Keys as in fps_tiled_kernel; each lane looks
             // below its two largest only where both are published.
-            auto top2 = [&](bool limited, uint64_t lim, uint64_t& a1, uint64_t& a2) {
-                a1 = 0;
-                a2 = 0;
+            int d1 = INT_MIN, d2 = INT_MIN, d3 = INT_MIN, c1 = 0x7FFFFFFF, c2 = 0x7FFFFFFF;
 #pragma unroll
-                for (int k = 0; k < PO; ++k) {
-                    if (k >= my_tiles) break;  // wave-uniform
-                    const uint64_t key =
-                        (static_cast<uint64_t>(static_cast<uint32_t>(f2i(md[k])) ^ 0x80000000u) << 32) |
-                        static_cast<uint32_t>(~pcode[k]);
-                    const bool below = !limited || key < lim;
-                    const bool first = below && key > a1;
-                    const bool second = below && !first && key > a2;
-                    a2 = first ? a1 : (second ? key : a2);
-                    a1 = first ? key : a1;
-                }
-            };
-            uint64_t h1, h2;
-            top2(false, 0, h1, h2);
-            const uint32_t d1 = static_cast<uint32_t>(h1 >> 32);
-            const uint32_t d2 = static_cast<uint32_t>(h2 >> 32);
-            const uint32_t top = wave_max_u32_l63(d1);
+            for (int k = 0; k < PO; ++k) {
+                const int key = f2i(md[k]);
+                d3 = max(d3, min(d2, key));
+                const bool first = key > d1, second = key > d2;
+                c2 = first ? c1 : (second ? pcode[k] : c2);
+                c1 = first ? pcode[k] : c1;
+                d2 = max(d2, min(d1, key));
+                d1 = max(d1, key);
+            }
+            const int top = wave_max_i32_l63(d1);
             const KeyCut cut = cut_top_keys<KC>(d1, d2, top, cut_guess);
-            // A candidate's slot: the cut's lanes in lane order, the d1 first.
-            auto put = [&](int slot, uint64_t key) {
-                const int code = static_cast<int>(~static_cast<uint32_t>(key));
-                const float4 c = spts[code & 0x1FFF];
+            // A padding code (a follower without points) reads any row.
+            auto put = [&](int slot, int key, int code) {
+                const float4 c = spts[min(code & 0x1FFF, CAP - 1)];
                 cand_pos[parity][fi * KC + slot] = make_float4(c.x, c.y, c.z, i2f(code >> 13));
-                cand_key[parity][fi * KC + slot] = static_cast<int>(static_cast<uint32_t>(key >> 32) ^ 0x80000000u);
+                cand_key[parity][fi * KC + slot] = key;
             };
-            if (cut.first != 0) {
+            int count, bound;
+            // A lane that holds the largest distance three times may keep
+            // back its smallest index: then as without a cut.
+            if (cut.first != 0 && ballot(d3 == top) == 0) {
                 const int n1 = __popcll(cut.first);
-                const int count = n1 + __popcll(cut.second);
+                count = n1 + __popcll(cut.second);
                 const bool has1 = (cut.first >> lane) & 1u;
                 const bool has2 = (cut.second >> lane) & 1u;
-                if (has1) put(lanes_below(cut.first), h1);
-                // The largest key that this lane keeps to itself.
-                uint32_t rest = has1 ? d2 : d1;
-                if (cut.second != 0) {
-                    if (has2) put(n1 + lanes_below(cut.second), h2);
-                    uint64_t h3, h4;
-                    top2(true, h2, h3, h4);
-                    rest = has2 ? static_cast<uint32_t>(h3 >> 32) : rest;
-                }
-                const uint32_t bound = wave_max_u32_l63(rest);
-                // Unfilled slots: the lowest key, which never wins a step.
-                if (lane >= count && lane < KC) {
-                    cand_pos[parity][fi * KC + lane] = make_float4(0.f, 0.f, 0.f, i2f(INT_MAX >> 13));
-                    cand_key[parity][fi * KC + lane] = INT_MIN;
-                }
-                if (lane == 0) bounds[fi] = static_cast<int>(bound ^ 0x80000000u);
+                if (has1) put(lanes_below(cut.first), d1, c1);
+                if (has2) put(n1 + lanes_below(cut.second), d2, c2);
+                bound = wave_max_i32_l63(has2 ? d3 : has1 ? d2 : d1);
             } else {
                 // No cut (more than KC points share the largest distance, or
                 // none can be sampled): the follower's best point alone, the
-                // smallest index among the largest keys, and the largest key
-                // as the bound: no later step of the run can take a key at it.
-                const uint32_t wlo = wave_max_u32_l63(d1 == top ? static_cast<uint32_t>(h1) : 0u);
-                if (lane < KC) {
-                    // A padding code (a follower without points) reads any row.
-                    const int code = static_cast<int>(~wlo);
-                    const float4 c = spts[min(code & 0x1FFF, CAP - 1)];
-                    cand_pos[parity][fi * KC + lane] = make_float4(c.x, c.y, c.z, i2f(code >> 13));
-                    cand_key[parity][fi * KC + lane] = lane == 0 ? static_cast<int>(top ^ 0x80000000u) : INT_MIN;
-                }
-                if (lane == 0) bounds[fi] = static_cast<int>(top ^ 0x80000000u);
+                // smallest index among the largest distances, and that
+                // distance as the bound: no later step of the run can take a
+                // key at it.
+                int code = 0x7FFFFFFF;
+#pragma unroll
+                for (int k = 0; k < PO; ++k) code = f2i(md[k]) == top ? min(code, pcode[k]) : code;
+                code = wave_min(code);
+                if (lane == 0) put(0, top, code);
+                count = 1;
+                bound = top;
             }
+            // Unfilled slots: the lowest key, which never wins a step.
+            if (lane >= count && lane < KC) {
+                cand_pos[parity][fi * KC + lane] = make_float4(0.f, 0.f, 0.f, i2f(INT_MAX >> 13));
+                cand_key[parity][fi * KC + lane] = INT_MIN;
+            }
+            if (lane == 0) bounds[fi] = bound;
         }
         __syncthreads();  // candidates and bounds published; the last run applied
         if (done[parity]) break;  // uniform: written by the leader before this barrier
@@ -1046,415 +1445,9 @@ __global__ __launch_bounds__(kLeadThreads) void fps_lead_kernel(
             int wv = wave_max_i32_l63(cmd);  // the first step after an exchange is exact
             int block_key = wv;              // chosen key of the block's first step
             const int nidx = -cidx;
-            const int imin = INT_MIN;
             uint32_t packed = 0, sh = 0;
             for (;;) {
-                // Up to 4 steps (one block), as hand-scheduled gfx950 code:
-                // the chosen candidate (the lowest lane holding the largest
-                // key wv; on a tie, the smallest index by a second wave
-                // maximum of -index), its coordinates by readlane, every
-                // candidate's key lowered to its distance to them, the lane
-                // packed into `packed`, then the next step's largest key by
-                // the DPP reduction of wave_max_i32_l63.  It stops after 4
-                // steps (st = 0, wv the next step's key), or when the run
-                // ends (st = 1): no steps left, or the next key is not above
-                // every bound.  The s_nop's (or scalar work in their place)
-                // give the wait states a DPP read of a VALU result (2), a
-                // readlane of a DPP result (1) and a VALU read of a
-                // readlane's SGPR (2) need.
-                //
-                // A block that cannot use up the steps (rem > 4) is the four
-                // steps written out: no shift count, step counter or loop
-                // branch, the tie test behind the readlanes and the next
-                // comparison ahead of the run's end test, so the chain
-                // cmp - ff1 - readlane - update - maximum waits for nothing
-                // else (a branch or a scalar operation in it costs its issue
-                // time: 313 -> 301 us at 32 x 4096 points, 1024 samples).
-                int st, wl, t, fx, fy, fz;
-                uint64_t tt;
-                float t0, t1, t2;
-                int m;
-                if (rem > 4) {
-                    asm volatile(
-                        "s_nop 1\n\t"
-                        "v_cmp_eq_u32_e32 vcc, %[wv], %[cmd]\n\t"
-                        "s_ff1_i32_b64 %[wl], vcc\n\t"
-                        "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
-                        "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
-                        "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
-                        "s_bcnt1_i32_b64 %[t], vcc\n\t"
-                        "s_cmp_gt_u32 %[t], 1\n\t"
-                        "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
-                        "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
-                        "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
-                        "s_cbranch_scc1 50f\n\t"
-                        "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
-                        "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
-                        "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
-                        "20:\n\t"
-                        "v_add_f32_e32 %[t0], %[t0], %[t1]\n\t"
-                        "v_add_f32_e32 %[t0], %[t0], %[t2]\n\t"
-                        "v_min_f32_e32 %[cmd], %[cmd], %[t0]\n\t"
-                        "s_mov_b32 %[pk], %[wl]\n\t"
-                        "s_nop 0\n\t"
-                        "v_max_i32_dpp %[m], %[cmd], %[cmd] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
-                        "s_nop 0\n\t"
-                        "v_readlane_b32 %[wv], %[m], 63\n\t"
-                        "s_cmp_le_i32 %[wv], %[maxb]\n\t"
-                        "s_nop 0\n\t"
-                        "v_cmp_eq_u32_e32 vcc, %[wv], %[cmd]\n\t"
-                        "s_cbranch_scc1 80f\n\t"
-                        "s_ff1_i32_b64 %[wl], vcc\n\t"
-                        "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
-                        "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
-                        "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
-                        "s_bcnt1_i32_b64 %[t], vcc\n\t"
-                        "s_cmp_gt_u32 %[t], 1\n\t"
-                        "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
-                        "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
-                        "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
-                        "s_cbranch_scc1 51f\n\t"
-                        "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
-                        "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
-                        "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
-                        "21:\n\t"
-                        "v_add_f32_e32 %[t0], %[t0], %[t1]\n\t"
-                        "s_lshl_b32 %[t], %[wl], 8\n\t"
-                        "v_add_f32_e32 %[t0], %[t0], %[t2]\n\t"
-                        "v_min_f32_e32 %[cmd], %[cmd], %[t0]\n\t"
-                        "s_or_b32 %[pk], %[pk], %[t]\n\t"
-                        "s_nop 0\n\t"
-                        "v_max_i32_dpp %[m], %[cmd], %[cmd] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
-                        "s_nop 0\n\t"
-                        "v_readlane_b32 %[wv], %[m], 63\n\t"
-                        "s_cmp_le_i32 %[wv], %[maxb]\n\t"
-                        "s_nop 0\n\t"
-                        "v_cmp_eq_u32_e32 vcc, %[wv], %[cmd]\n\t"
-                        "s_cbranch_scc1 81f\n\t"
-                        "s_ff1_i32_b64 %[wl], vcc\n\t"
-                        "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
-                        "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
-                        "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
-                        "s_bcnt1_i32_b64 %[t], vcc\n\t"
-                        "s_cmp_gt_u32 %[t], 1\n\t"
-                        "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
-                        "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
-                        "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
-                        "s_cbranch_scc1 52f\n\t"
-                        "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
-                        "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
-                        "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
-                        "22:\n\t"
-                        "v_add_f32_e32 %[t0], %[t0], %[t1]\n\t"
-                        "s_lshl_b32 %[t], %[wl], 16\n\t"
-                        "v_add_f32_e32 %[t0], %[t0], %[t2]\n\t"
-                        "v_min_f32_e32 %[cmd], %[cmd], %[t0]\n\t"
-                        "s_or_b32 %[pk], %[pk], %[t]\n\t"
-                        "s_nop 0\n\t"
-                        "v_max_i32_dpp %[m], %[cmd], %[cmd] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
-                        "s_nop 0\n\t"
-                        "v_readlane_b32 %[wv], %[m], 63\n\t"
-                        "s_cmp_le_i32 %[wv], %[maxb]\n\t"
-                        "s_nop 0\n\t"
-                        "v_cmp_eq_u32_e32 vcc, %[wv], %[cmd]\n\t"
-                        "s_cbranch_scc1 82f\n\t"
-                        "s_ff1_i32_b64 %[wl], vcc\n\t"
-                        "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
-                        "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
-                        "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
-                        "s_bcnt1_i32_b64 %[t], vcc\n\t"
-                        "s_cmp_gt_u32 %[t], 1\n\t"
-                        "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
-                        "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
-                        "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
-                        "s_cbranch_scc1 53f\n\t"
-                        "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
-                        "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
-                        "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
-                        "23:\n\t"
-                        "v_add_f32_e32 %[t0], %[t0], %[t1]\n\t"
-                        "s_lshl_b32 %[t], %[wl], 24\n\t"
-                        "v_add_f32_e32 %[t0], %[t0], %[t2]\n\t"
-                        "v_min_f32_e32 %[cmd], %[cmd], %[t0]\n\t"
-                        "s_or_b32 %[pk], %[pk], %[t]\n\t"
-                        "s_nop 0\n\t"
-                        "v_max_i32_dpp %[m], %[cmd], %[cmd] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
-                        "s_nop 0\n\t"
-                        "v_readlane_b32 %[wv], %[m], 63\n\t"
-                        "s_cmp_le_i32 %[wv], %[maxb]\n\t"
-                        "s_cbranch_scc1 83f\n\t"
-                        "s_mov_b32 %[st], 0\n\t"
-                        "s_mov_b32 %[sh], 32\n\t"
-                        "s_branch 9f\n\t"
-                        "50:\n\t"
-                        "v_cndmask_b32_e32 %[m], %[imin], %[nidx], vcc\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_readlane_b32 %[t], %[m], 63\n\t"
-                        "s_nop 1\n\t"
-                        "v_cmp_eq_u32_e64 %[tt], %[t], %[nidx]\n\t"
-                        "s_and_b64 vcc, vcc, %[tt]\n\t"
-                        "s_ff1_i32_b64 %[wl], vcc\n\t"
-                        "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
-                        "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
-                        "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
-                        "s_nop 1\n\t"
-                        "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
-                        "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
-                        "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
-                        "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
-                        "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
-                        "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
-                        "s_branch 20b\n\t"
-                        "51:\n\t"
-                        "v_cndmask_b32_e32 %[m], %[imin], %[nidx], vcc\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_readlane_b32 %[t], %[m], 63\n\t"
-                        "s_nop 1\n\t"
-                        "v_cmp_eq_u32_e64 %[tt], %[t], %[nidx]\n\t"
-                        "s_and_b64 vcc, vcc, %[tt]\n\t"
-                        "s_ff1_i32_b64 %[wl], vcc\n\t"
-                        "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
-                        "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
-                        "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
-                        "s_nop 1\n\t"
-                        "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
-                        "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
-                        "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
-                        "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
-                        "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
-                        "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
-                        "s_branch 21b\n\t"
-                        "52:\n\t"
-                        "v_cndmask_b32_e32 %[m], %[imin], %[nidx], vcc\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_readlane_b32 %[t], %[m], 63\n\t"
-                        "s_nop 1\n\t"
-                        "v_cmp_eq_u32_e64 %[tt], %[t], %[nidx]\n\t"
-                        "s_and_b64 vcc, vcc, %[tt]\n\t"
-                        "s_ff1_i32_b64 %[wl], vcc\n\t"
-                        "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
-                        "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
-                        "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
-                        "s_nop 1\n\t"
-                        "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
-                        "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
-                        "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
-                        "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
-                        "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
-                        "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
-                        "s_branch 22b\n\t"
-                        "53:\n\t"
-                        "v_cndmask_b32_e32 %[m], %[imin], %[nidx], vcc\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_readlane_b32 %[t], %[m], 63\n\t"
-                        "s_nop 1\n\t"
-                        "v_cmp_eq_u32_e64 %[tt], %[t], %[nidx]\n\t"
-                        "s_and_b64 vcc, vcc, %[tt]\n\t"
-                        "s_ff1_i32_b64 %[wl], vcc\n\t"
-                        "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
-                        "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
-                        "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
-                        "s_nop 1\n\t"
-                        "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
-                        "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
-                        "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
-                        "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
-                        "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
-                        "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
-                        "s_branch 23b\n\t"
-                        "80:\n\t"
-                        "s_movk_i32 %[sh], 8\n\t"
-                        "s_branch 88f\n\t"
-                        "81:\n\t"
-                        "s_movk_i32 %[sh], 16\n\t"
-                        "s_branch 88f\n\t"
-                        "82:\n\t"
-                        "s_movk_i32 %[sh], 24\n\t"
-                        "s_branch 88f\n\t"
-                        "83:\n\t"
-                        "s_movk_i32 %[sh], 32\n\t"
-                        "88:\n\t"
-                        "s_mov_b32 %[st], 1\n\t"
-                        "9:\n\t"
-                        "s_nop 1\n\t"
-                        : [cmd] "+v"(cmd), [wv] "+s"(wv), [pk] "=&s"(packed),
-                          [sh] "=&s"(sh), [st] "=&s"(st), [wl] "=&s"(wl), [t] "=&s"(t),
-                          [fx] "=&s"(fx), [fy] "=&s"(fy), [fz] "=&s"(fz), [tt] "=&s"(tt),
-                          [t0] "=&v"(t0), [t1] "=&v"(t1), [t2] "=&v"(t2), [m] "=&v"(m)
-                        : [cx] "v"(ccx), [cy] "v"(ccy), [cz] "v"(ccz), [nidx] "v"(nidx),
-                          [imin] "v"(imin), [maxb] "s"(maxb)
-                        : "vcc", "scc");
-                    rem -= 4;
-                } else {
-                    asm volatile(
-                        "s_nop 1\n\t"
-                        "s_mov_b32 %[sh], 0\n\t"
-                        "s_mov_b32 %[pk], 0\n"
-                        "1:\n\t"
-                        "v_cmp_eq_u32_e32 vcc, %[wv], %[cmd]\n\t"
-                        "s_ff1_i32_b64 %[wl], vcc\n\t"
-                        "s_bcnt1_i32_b64 %[t], vcc\n\t"
-                        "s_cmp_gt_u32 %[t], 1\n\t"
-                        "s_cbranch_scc1 5f\n"
-                        "2:\n\t"
-                        "v_readlane_b32 %[fx], %[cx], %[wl]\n\t"
-                        "v_readlane_b32 %[fy], %[cy], %[wl]\n\t"
-                        "v_readlane_b32 %[fz], %[cz], %[wl]\n\t"
-                        "s_lshl_b32 %[t], %[wl], %[sh]\n\t"
-                        "v_subrev_f32_e32 %[t0], %[fx], %[cx]\n\t"
-                        "v_subrev_f32_e32 %[t1], %[fy], %[cy]\n\t"
-                        "v_subrev_f32_e32 %[t2], %[fz], %[cz]\n\t"
-                        "s_or_b32 %[pk], %[pk], %[t]\n\t"
-                        "v_mul_f32_e32 %[t0], %[t0], %[t0]\n\t"
-                        "v_mul_f32_e32 %[t1], %[t1], %[t1]\n\t"
-                        "v_mul_f32_e32 %[t2], %[t2], %[t2]\n\t"
-                        "v_add_f32_e32 %[t0], %[t0], %[t1]\n\t"
-                        "s_add_u32 %[sh], %[sh], 8\n\t"
-                        "v_add_f32_e32 %[t0], %[t0], %[t2]\n\t"
-                        "s_sub_u32 %[rem], %[rem], 1\n\t"
-                        "v_min_f32_e32 %[cmd], %[cmd], %[t0]\n\t"
-                        "s_cmp_eq_u32 %[rem], 0\n\t"
-                        "s_cbranch_scc1 8f\n\t"
-                        "v_max_i32_dpp %[m], %[cmd], %[cmd] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
-                        "s_nop 0\n\t"
-                        "v_readlane_b32 %[wv], %[m], 63\n\t"
-                        "s_cmp_le_i32 %[wv], %[maxb]\n\t"
-                        "s_cbranch_scc1 8f\n\t"
-                        "s_cmp_lt_u32 %[sh], 32\n\t"
-                        "s_cbranch_scc1 1b\n\t"
-                        "s_mov_b32 %[st], 0\n\t"
-                        "s_branch 9f\n"
-                        "5:\n\t"
-                        "v_cndmask_b32_e32 %[m], %[imin], %[nidx], vcc\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_mirror row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
-                        "s_nop 1\n\t"
-                        "v_max_i32_dpp %[m], %[m], %[m] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
-                        "s_nop 0\n\t"
-                        "v_readlane_b32 %[t], %[m], 63\n\t"
-                        "s_nop 1\n\t"
-                        "v_cmp_eq_u32_e64 %[tt], %[t], %[nidx]\n\t"
-                        "s_and_b64 vcc, vcc, %[tt]\n\t"
-                        "s_ff1_i32_b64 %[wl], vcc\n\t"
-                        "s_branch 2b\n"
-                        "8:\n\t"
-                        "s_mov_b32 %[st], 1\n"
-                        "9:\n\t"
-                        "s_nop 1"
-                        : [cmd] "+v"(cmd), [wv] "+s"(wv), [rem] "+s"(rem), [pk] "=&s"(packed),
-                          [sh] "=&s"(sh), [st] "=&s"(st), [wl] "=&s"(wl), [t] "=&s"(t),
-                          [fx] "=&s"(fx), [fy] "=&s"(fy), [fz] "=&s"(fz), [tt] "=&s"(tt),
-                          [t0] "=&v"(t0), [t1] "=&v"(t1), [t2] "=&v"(t2), [m] "=&v"(m)
-                        : [cx] "v"(ccx), [cy] "v"(ccy), [cz] "v"(ccz), [nidx] "v"(nidx),
-                          [imin] "v"(imin), [maxb] "s"(maxb)
-                        : "vcc", "scc");
-                }
+                const int st = lead_block(cmd, wv, rem, packed, sh, ccx, ccy, ccz, nidx, maxb);
                 taken += static_cast<int>(sh >> 3);
                 if (st != 0) break;
                 // A full block: its row, then the count.  Lane l writes word l
@@ -1565,6 +1558,392 @@ __global__ __launch_bounds__(kLeadThreads) void fps_lead_kernel(
     }
 }
 
+// fps_wide_kernel: the leader scheme for clouds of up to kWideMaxPoints
+// points, more than a workgroup's registers hold.
+//
+// The same nine waves, runs, candidates and step chain as fps_lead_kernel;
+// only where the points live differs.  The running distances and the points'
+// original indices stay in LDS by sorted position (6 bytes a point, dynamic
+// LDS), the sorted coordinates in a caller-provided scratch array (16 bytes a
+// point, read through the XCD's L2).  A follower holds up to 48 tiles of 64
+// sorted points and lane t the box of its tile t, so a step's tiles come from
+// one box test and ballot; the tiles of a block of 4 steps are loaded
+// together, 4 tiles at a time, and each point is read once for all its steps.
+//
+// What bounds it: the leader's step chain and the exchanges, as in
+// fps_lead_kernel; the whole cloud is only read in the first few runs.  The
+// kernel it replaces (one workgroup, every point re-read from L2 in every
+// step) was bound by that read: 17.8 ms for 8 x 16384 points, 4096 samples
+// (4.35 us a step).
+constexpr int kWideMaxTiles = 48;  // tiles per follower: 6 bytes x 24576 points of LDS
+constexpr int64_t kWideMaxPoints = int64_t(kWideMaxTiles) * kLeadFollowers * kWave;
+constexpr int kWideBatch = 4;      // tiles loaded together
+// Clouds of at most this many samples are left to fps_global_kernel, which
+// needs no sort: 8 x 16384 points, 32 samples 140 us against 175 (64 samples
+// 280 against 231); 2 x 24576, 64 samples 370 against 333.
+constexpr int kWideFew = 48;
+
+__global__ __launch_bounds__(kLeadThreads) void fps_wide_kernel(
+    const float* __restrict__ xyz, const int64_t* __restrict__ ptr,
+    const int64_t* __restrict__ out_ptr, const int64_t* __restrict__ starts,
+    int64_t* __restrict__ out, float4* __restrict__ sorted, int cap, int64_t N, int64_t npoint,
+    int64_t start, int skip, int few) {
+    constexpr int NF = kLeadFollowers;
+    constexpr int KC = kLeadCand;
+    constexpr int TS = NF * kWave;  // threads of the sort
+    constexpr int kCells = 4096;
+    // Running distances of the sorted positions (the sort's cell counts
+    // before that), then their original indices.  `cap` (a multiple of
+    // 64 NF, at least kCells) covers the largest cloud of the launch.
+    extern __shared__ float wide_lds[];
+    float* const md = wide_lds;
+    uint16_t* const index_of = reinterpret_cast<uint16_t*>(wide_lds + cap);
+    int* const cell_count = reinterpret_cast<int*>(wide_lds);
+    __shared__ float red[6][NF];
+    __shared__ int wave_sum[NF];
+    __shared__ float4 cand_pos[2][kWave];
+    __shared__ int cand_key[2][kWave];
+    __shared__ int bounds[NF];
+    // Per 4 steps the packed lanes and the chosen key of the first of them;
+    // the leader's other lanes write the padding behind the rows, so that
+    // one store without an exec mask hits distinct addresses.
+    __shared__ uint32_t ring[kLeadRing / 4 * 2 + kWave];
+    __shared__ __align__(8) uint32_t marks[kWave];
+    __shared__ int done[2];
+
+    const Segment seg = segment_of(blockIdx.x, ptr, out_ptr, starts, N, npoint, start);
+    if (seg.cnt <= few) return;  // uniform over the workgroup, before any barrier
+    const float* p = xyz + 3 * seg.in_lo;
+    float4* const spts = sorted + seg.in_lo;
+    int64_t* o = out + seg.out_lo;
+    const int n = static_cast<int>(seg.n);
+    const int tid = threadIdx.x;
+    const int wave = uniform(tid / kWave);
+    const int lane = tid % kWave;
+    const bool leader = wave == NF;
+    const int far0 = static_cast<int>(seg.start);
+    if (leader && lane == 0) o[0] = seg.base + far0;
+    if (n <= 0) return;
+
+    // ---- setup by the followers: bounding box, cell counts, scan, scatter
+    if (tid == 0) {
+        marks[0] = marks[1] = 1u;
+        done[0] = done[1] = 0;
+    }
+    if (!leader) {
+        for (int c = tid; c < kCells; c += TS) cell_count[c] = 0;
+        float v[6];
+        v[0] = v[1] = v[2] = v[3] = v[4] = v[5] = INFINITY;
+        for (int j = tid; j < n; j += TS) {
+            const float x = p[3 * j], y = p[3 * j + 1], z = p[3 * j + 2];
+            v[0] = fminf(v[0], x); v[3] = fminf(v[3], -x);
+            v[1] = fminf(v[1], y); v[4] = fminf(v[4], -y);
+            v[2] = fminf(v[2], z); v[5] = fminf(v[5], -z);
+        }
+        fold_min<6, kWave / 2>(v, lane);
+        if (lane == 0) {
+#pragma unroll
+            for (int a = 0; a < 3; ++a) red[a][wave] = v[a];
+        }
+        if (lane == kWave / 2) {
+#pragma unroll
+            for (int a = 0; a < 3; ++a) red[3 + a][wave] = -v[a];
+        }
+    }
+    __syncthreads();  // box partials, cleared counters, marks
+    float lo[3], scale[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        float mn = red[a][0], mx = red[3 + a][0];
+#pragma unroll
+        for (int w = 1; w < NF; ++w) {
+            mn = fminf(mn, red[a][w]);
+            mx = fmaxf(mx, red[3 + a][w]);
+        }
+        lo[a] = mn;
+        const float ext = mx - mn;
+        scale[a] = (ext > 0.f && ext < INFINITY) ? 16.f / ext : 0.f;
+    }
+    auto cell_of = [&](float x, float y, float z) {
+        const float c3[3] = {x, y, z};
+        uint32_t q[3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a)  // NaN goes to cell 0, infinities to the edges
+            q[a] = static_cast<uint32_t>(fminf(fmaxf((c3[a] - lo[a]) * scale[a], 0.f), 15.f));
+        return morton12(q[0], q[1], q[2]);
+    };
+    if (!leader)
+        for (int j = tid; j < n; j += TS)
+            atomicAdd(&cell_count[cell_of(p[3 * j], p[3 * j + 1], p[3 * j + 2])], 1);
+    __syncthreads();  // counts complete
+    {
+        constexpr int CPT = kCells / TS;
+        int run = 0;
+        if (!leader) {
+#pragma unroll
+            for (int c = 0; c < CPT; ++c) {
+                const int v = cell_count[tid * CPT + c];
+                cell_count[tid * CPT + c] = run;
+                run += v;
+            }
+        }
+        int incl = run;
+#pragma unroll
+        for (int d = 1; d < kWave; d <<= 1) {
+            const int up = __shfl_up(incl, d, kWave);
+            if (lane >= d) incl += up;
+        }
+        if (!leader && lane == kWave - 1) wave_sum[wave] = incl;
+        __syncthreads();  // wave totals
+        int before = incl - run;
+        for (int w = 0; w < wave && w < NF; ++w) before += wave_sum[w];
+        if (!leader) {
+#pragma unroll
+            for (int c = 0; c < CPT; ++c) cell_count[tid * CPT + c] += before;
+        }
+    }
+    __syncthreads();  // offsets complete
+    // Tiles per follower, and its first sorted position.
+    const int tiles = (n + TS - 1) / TS;
+    const int pos0 = wave * tiles * kWave;
+    if (!leader) {
+        for (int j = tid; j < n; j += TS) {
+            const float x = p[3 * j], y = p[3 * j + 1], z = p[3 * j + 2];
+            const int q = atomicAdd(&cell_count[cell_of(x, y, z)], 1);  // < n: the counts sum to n
+            spts[q] = make_float4(x, y, z, 0.f);
+            index_of[q] = static_cast<uint16_t>(j);
+        }
+        // Positions without a point: an index above every point's.
+        for (int q = n + tid; q < tiles * TS; q += TS) index_of[q] = 0xFFFFu;
+    }
+    __syncthreads();  // sorted points written (and, behind the barrier, visible to the workgroup)
+    // ---- running distances and tile boxes (lane t: tile t; [+inf, +inf],
+    // which no test selects, where there is none or it holds no point)
+    float tlo[3] = {INFINITY, INFINITY, INFINITY}, thi[3] = {INFINITY, INFINITY, INFINITY};
+    if (!leader) {
+        const int f = min(max(far0, 0), n - 1);
+        const float cx = p[3 * f], cy = p[3 * f + 1], cz = p[3 * f + 2];
+        for (int t = 0; t < tiles; ++t) {
+            const int q = pos0 + t * kWave + lane;
+            const bool valid = q < n;
+            const float4 s = spts[min(q, n - 1)];
+            float d = valid ? initial_running(skip, s.x, s.y, s.z) : -INFINITY;
+            d = running_min(d, sqdist3(s.x, s.y, s.z, cx, cy, cz));
+            md[q] = d;
+            float v[6];
+            v[0] = valid ? s.x : INFINITY; v[3] = valid ? -s.x : INFINITY;
+            v[1] = valid ? s.y : INFINITY; v[4] = valid ? -s.y : INFINITY;
+            v[2] = valid ? s.z : INFINITY; v[5] = valid ? -s.z : INFINITY;
+            fold_min<6, kWave / 2>(v, lane);
+            float blo[3], bhi[3];
+            bool has = lane == t;
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                blo[a] = i2f(readlane(f2i(v[a]), 0));
+                bhi[a] = -i2f(readlane(f2i(v[a]), kWave / 2));
+                has = has && blo[a] <= bhi[a];
+            }
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                tlo[a] = has ? blo[a] : tlo[a];
+                thi[a] = has ? bhi[a] : thi[a];
+            }
+        }
+    }
+
+    if (leader) __builtin_amdgcn_s_setprio(3);
+    // The leader's ring store: lanes 0 and 1 the row, the others the padding.
+    const int ring_at = lane < 2 ? lane : kLeadRing / 4 * 2 + lane - 2;
+    const int ring_row = lane < 2 ? 2 : 0;
+    uint32_t cut_guess = 1u << 21;
+    int64_t step = 1;
+    int parity = 0;
+    for (;;) {
+        if (!leader) {
+            // Exchange: each lane's three largest running distances, the
+            // tiles of the first two, and the follower's cut.
+            int d1 = INT_MIN, d2 = INT_MIN, d3 = INT_MIN, t1 = 0, t2 = 0;
+#pragma unroll 8
+            for (int t = 0; t < tiles; ++t) {
+                const int key = f2i(md[pos0 + t * kWave + lane]);
+                d3 = max(d3, min(d2, key));
+                const bool first = key > d1, second = key > d2;
+                t2 = first ? t1 : (second ? t : t2);
+                t1 = first ? t : t1;
+                d2 = max(d2, min(d1, key));
+                d1 = max(d1, key);
+            }
+            const int top = wave_max_i32_l63(d1);
+            // The points that the cut will probably take, requested now so
+            // that the search hides their latency.
+            const int q1 = pos0 + t1 * kWave + lane, q2 = pos0 + t2 * kWave + lane;
+            const int likely = max(top - static_cast<int>(min(cut_guess, 1u << 29) << 1), 0);
+            float4 c1 = make_float4(0.f, 0.f, 0.f, 0.f), c2 = c1;
+            if (d1 >= likely) c1 = spts[min(q1, n - 1)];
+            if (d2 >= likely) c2 = spts[min(q2, n - 1)];
+            const KeyCut cut = cut_top_keys<KC>(d1, d2, top, cut_guess);
+            auto put = [&](int slot, int key, float4 c, int j) {
+                cand_pos[parity][wave * KC + slot] = make_float4(c.x, c.y, c.z, i2f(j));
+                cand_key[parity][wave * KC + slot] = key;
+            };
+            const bool has1 = (cut.first >> lane) & 1u;
+            const bool has2 = (cut.second >> lane) & 1u;
+            int count, bound;
+            // A lane that holds the largest distance three times may keep
+            // back its smallest index: then as without a cut.
+            if (cut.first != 0 && ballot(d3 == top) == 0) {
+                const int n1 = __popcll(cut.first);
+                count = n1 + __popcll(cut.second);
+                if (has1) {
+                    if (d1 < likely) c1 = spts[q1];
+                    put(lanes_below(cut.first), d1, c1, index_of[q1]);
+                }
+                if (has2) {
+                    if (d2 < likely) c2 = spts[q2];
+                    put(n1 + lanes_below(cut.second), d2, c2, index_of[q2]);
+                }
+                bound = wave_max_i32_l63(has2 ? d3 : has1 ? d2 : d1);
+            } else {
+                // No cut (more than KC points share the largest distance, or
+                // none can be sampled): the follower's best point alone, the
+                // smallest index among the largest distances, and that
+                // distance as the bound: no later step of the run can take a
+                // key at it.
+                int j = INT_MAX;
+                for (int t = 0; t < tiles; ++t) {
+                    const int q = pos0 + t * kWave + lane;
+                    j = f2i(md[q]) == top ? min(j, static_cast<int>(index_of[q])) : j;
+                }
+                j = wave_min(j);
+                const int f = min(j, n - 1);  // a follower without points: any point
+                if (lane == 0) put(0, top, make_float4(p[3 * f], p[3 * f + 1], p[3 * f + 2], 0.f), j);
+                count = 1;
+                bound = top;
+            }
+            if (lane >= count && lane < KC)  // unfilled slots never win a step
+                put(lane, INT_MIN, make_float4(0.f, 0.f, 0.f, 0.f), INT_MAX);
+            if (lane == 0) bounds[wave] = bound;
+        }
+        __syncthreads();  // candidates and bounds published; the last run applied
+        if (done[parity]) break;  // uniform: written by the leader before this barrier
+        const int64_t run_start = step;
+        const float4 mine = cand_pos[parity][lane];  // w: the point index
+        if (leader) {
+            int maxb_v = bounds[0];
+#pragma unroll
+            for (int w = 1; w < NF; ++w) maxb_v = max(maxb_v, bounds[w]);
+            int cmd = cand_key[parity][lane];
+            const int cidx = f2i(mine.w);
+            // A non-finite candidate limits the run to one step (see
+            // fps_lead_kernel).
+            const bool odd = cmd >= 0 && !(isfinite(mine.x) && isfinite(mine.y) && isfinite(mine.z));
+            const int maxb = ballot(odd) ? INT_MAX : max(uniform(maxb_v), 0);
+            const int64_t rest = seg.cnt - step;
+            int rem = uniform(static_cast<int>(rest < kLeadRing ? rest : kLeadRing));  // steps left
+            const uint32_t base = static_cast<uint32_t>(run_start);
+            int taken = 0;
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): no wait for it in the loop
+            int wv = wave_max_i32_l63(cmd);  // the first step after an exchange is exact
+            int block_key = wv;              // chosen key of the block's first step
+            uint32_t packed = 0, sh = 0;
+            for (;;) {
+                const int st = lead_block(cmd, wv, rem, packed, sh, mine.x, mine.y, mine.z, -cidx, maxb);
+                taken += static_cast<int>(sh >> 3);
+                if (st != 0) break;
+                ring[ring_at + ((taken >> 2) - 1) * ring_row] = lane == 0 ? packed : static_cast<uint32_t>(block_key);
+                __atomic_signal_fence(__ATOMIC_SEQ_CST);  // the row is issued before the count
+                __hip_atomic_store(&marks[lane == 0 ? 0 : lane + (lane == 1)], base + taken,
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                block_key = wv;
+            }
+            // The last block's row (full or partial), then the count and the
+            // run's end in one store.
+            ring[ring_at + ((taken - 1) >> 2) * ring_row] = lane == 0 ? packed : static_cast<uint32_t>(block_key);
+            step += taken;
+            done[parity ^ 1] = step >= seg.cnt ? 1 : 0;  // read by every wave after the next barrier
+            __atomic_signal_fence(__ATOMIC_SEQ_CST);
+            __hip_atomic_store(&marks[lane], lane < 2 ? base + taken : 0u, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WORKGROUP);
+            // The run's samples: lane i of a batch takes step c0 + i.
+            for (int c0 = 0; c0 < taken; c0 += kWave) {
+                const int si = min(c0 + lane, taken - 1);
+                const int wl = static_cast<int>((ring[(si >> 2) * 2] >> (8 * (si & 3))) & 63u);
+                const int idx = __builtin_amdgcn_ds_bpermute(wl << 2, cidx);
+                if (c0 + lane < taken) o[run_start + c0 + lane] = seg.base + idx;
+            }
+        } else {
+            // A block of up to 4 published steps: each step's centroid (this
+            // wave's copy of the candidates), the tiles whose box it may
+            // reach within the block's first chosen key, and the updates of
+            // the union of those tiles.
+            auto block = [&](uint32_t lanes4, float M1, int cnt) {
+                float fx[4], fy[4], fz[4];
+                uint64_t hit[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int wl = static_cast<int>((lanes4 >> (8 * j)) & 63u);
+                    fx[j] = i2f(readlane(f2i(mine.x), wl));
+                    fy[j] = i2f(readlane(f2i(mine.y), wl));
+                    fz[j] = i2f(readlane(f2i(mine.z), wl));
+                    const float gx = fx[j] - __builtin_amdgcn_fmed3f(fx[j], tlo[0], thi[0]);
+                    const float gy = fy[j] - __builtin_amdgcn_fmed3f(fy[j], tlo[1], thi[1]);
+                    const float gz = fz[j] - __builtin_amdgcn_fmed3f(fz[j], tlo[2], thi[2]);
+                    float lb = gx * gx;
+                    lb = lb + gy * gy;
+                    lb = lb + gz * gz;
+                    hit[j] = j < cnt ? ballot(lb < M1) : 0;
+                }
+                uint64_t todo = hit[0] | hit[1] | hit[2] | hit[3];
+                while (todo != 0) {
+                    // The batch's loads first (a repeated last tile where
+                    // fewer are left), then its updates.
+                    int tile[kWideBatch];
+                    float4 pt[kWideBatch];
+                    float d[kWideBatch];
+                    int last = 0;
+#pragma unroll
+                    for (int i = 0; i < kWideBatch; ++i) {
+                        tile[i] = todo != 0 ? static_cast<int>(__builtin_ctzll(todo)) : -1;
+                        last = todo != 0 ? tile[i] : last;
+                        todo &= todo - 1;
+                        const int q = pos0 + last * kWave + lane;
+                        pt[i] = spts[min(q, n - 1)];
+                        d[i] = md[q];
+                    }
+#pragma unroll
+                    for (int i = 0; i < kWideBatch; ++i) {
+                        if (tile[i] < 0) break;  // wave-uniform
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+                            if ((hit[j] >> tile[i]) & 1u)
+                                d[i] = running_min(d[i], sqdist3(pt[i].x, pt[i].y, pt[i].z, fx[j], fy[j], fz[j]));
+                        md[pos0 + tile[i] * kWave + lane] = d[i];
+                    }
+                }
+            };
+            int a = 0;  // steps of this run applied (a multiple of 4 until the run ends)
+            for (;;) {
+                const uint64_t m = __hip_atomic_load(reinterpret_cast<uint64_t*>(marks), __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_WORKGROUP);
+                __atomic_signal_fence(__ATOMIC_SEQ_CST);  // ring reads after the mark
+                const int pub = uniform(static_cast<int>(m)) - static_cast<int>(run_start);
+                const int end = uniform(static_cast<int>(m >> 32)) - static_cast<int>(run_start);
+                while (a + 4 <= pub || (end > 0 && pub >= end && a < end)) {
+                    const int cnt = end > 0 && pub >= end ? min(4, end - a) : 4;
+                    const uint32_t* row = ring + (a >> 2) * 2;
+                    block(static_cast<uint32_t>(uniform(static_cast<int>(row[0]))),
+                          i2f(uniform(static_cast<int>(row[1]))), cnt);
+                    a += cnt;
+                }
+                if (end > 0 && pub >= end) break;
+                __builtin_amdgcn_s_sleep(0);
+            }
+            step = run_start + a;
+        }
+        parity ^= 1;
+    }
+}
+
 template <int T>
 __global__ __launch_bounds__(T) void fps_global_kernel(const float* __restrict__ xyz,
                                                        const int64_t* __restrict__ ptr,
@@ -1572,11 +1951,12 @@ __global__ __launch_bounds__(T) void fps_global_kernel(const float* __restrict__
                                                        const int64_t* __restrict__ starts,
                                                        int64_t* __restrict__ out,
                                                        float* __restrict__ scratch, int64_t N,
-                                                       int64_t npoint, int64_t start, int skip) {
+                                                       int64_t npoint, int64_t start, int skip,
+                                                       int64_t most) {
     constexpr int NW = T / kWave;
     __shared__ int2 slots[2][NW];
     const Segment seg = segment_of(blockIdx.x, ptr, out_ptr, starts, N, npoint, start);
-    if (seg.cnt <= 0) return;
+    if (seg.cnt <= 0 || seg.cnt > most) return;
     const float* p = xyz + 3 * seg.in_lo;
     float* md = scratch + seg.in_lo;
     int64_t* o = out + seg.out_lo;
@@ -2230,6 +2610,12 @@ hipError_t launch_regs(const float* xyz, const int64_t* ptr, const int64_t* out_
     return hipGetLastError();
 }
 
+// Scratch of launch_fps above kRegsMaxPoints, by the largest cloud: the sorted
+// coordinates of fps_wide_kernel, or fps_global_kernel's running distances.
+size_t fps_scratch_bytes_per_point(int64_t max_len) {
+    return max_len <= kWideMaxPoints ? sizeof(float4) : sizeof(float);
+}
+
 hipError_t launch_fps(const float* xyz, const int64_t* ptr, const int64_t* out_ptr,
                       const int64_t* starts, int64_t* out, float* scratch, int64_t blocks,
                       int64_t max_len, int64_t N, int64_t npoint, int64_t start, int skip,
@@ -2245,9 +2631,27 @@ hipError_t launch_fps(const float* xyz, const int64_t* ptr, const int64_t* out_p
     if (max_len <= 16 * kRegsThreads)
         return launch_regs<16>(xyz, ptr, out_ptr, starts, out, blocks, N, npoint, start, skip, stream);
     if (scratch == nullptr) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((fps_global_kernel<kGlobalThreads>), dim3(static_cast<uint32_t>(blocks)),
-                       dim3(kGlobalThreads), 0, stream, xyz, ptr, out_ptr, starts, out, scratch,
-                       N, npoint, start, skip);
+    // Up to kWideMaxPoints the wide kernel takes the clouds of more than
+    // kWideFew samples and the global kernel the others; a dense launch is all
+    // one or all the other, a ragged one may hold both, so it runs both (in
+    // turn on the stream: the second may reuse the first's scratch).
+    const bool wide = max_len <= kWideMaxPoints;
+    if (!wide || ptr != nullptr || npoint <= kWideFew) {
+        hipLaunchKernelGGL((fps_global_kernel<kGlobalThreads>), dim3(static_cast<uint32_t>(blocks)),
+                           dim3(kGlobalThreads), 0, stream, xyz, ptr, out_ptr, starts, out, scratch,
+                           N, npoint, start, skip, wide ? int64_t(kWideFew) : INT64_MAX);
+        const hipError_t err = hipGetLastError();
+        if (err != hipSuccess || !wide || ptr == nullptr) return err;
+    }
+    constexpr int kRow = kLeadFollowers * kWave;
+    const int cap = static_cast<int>((max_len + kRow - 1) / kRow) * kRow;
+    const int lds = cap * static_cast<int>(sizeof(float) + sizeof(uint16_t));
+    const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(&fps_wide_kernel),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (err != hipSuccess) return err;
+    hipLaunchKernelGGL(fps_wide_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kLeadThreads),
+                       static_cast<size_t>(lds), stream, xyz, ptr, out_ptr, starts, out,
+                       reinterpret_cast<float4*>(scratch), cap, N, npoint, start, skip, kWideFew);
     return hipGetLastError();
 }
 
@@ -2413,7 +2817,7 @@ extern "C" {
 
 size_t pointops_fps_dense_scratch_bytes(int64_t B, int64_t N) {
     if (B <= 0 || N <= kRegsMaxPoints) return 0;
-    return static_cast<size_t>(B) * static_cast<size_t>(N) * sizeof(float);
+    return static_cast<size_t>(B) * static_cast<size_t>(N) * fps_scratch_bytes_per_point(N);
 }
 
 hipError_t pointops_fps_dense(const float* xyz, int64_t* out, void* scratch, int64_t B, int64_t N,
@@ -2430,7 +2834,7 @@ hipError_t pointops_fps_dense(const float* xyz, int64_t* out, void* scratch, int
 
 size_t pointops_fps_flat_scratch_bytes(int64_t total_n, int64_t max_len) {
     if (max_len <= kRegsMaxPoints || total_n <= 0) return 0;
-    return static_cast<size_t>(total_n) * sizeof(float);
+    return static_cast<size_t>(total_n) * fps_scratch_bytes_per_point(max_len);
 }
 
 hipError_t pointops_fps_flat(const float* x, const int64_t* ptr, const int64_t* out_ptr,

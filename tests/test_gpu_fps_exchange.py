@@ -32,7 +32,7 @@ def _cloud(kind: str, n: int) -> torch.Tensor:
 
 
 @pytest.mark.parametrize("kind", ["lattice", "repeated", "one", "octaves", "never"])
-@pytest.mark.parametrize("n", [9, 511, 1024, 1025, 4096])
+@pytest.mark.parametrize("n", [9, 511, 1024, 1025, 4096, 8193, 24576])
 def test_fps_with_hard_cuts_matches_oracle(cuda_device, kind, n):
     import mps_pointops as mp
 
@@ -41,3 +41,20 @@ def test_fps_with_hard_cuts_matches_oracle(cuda_device, kind, n):
     skip = kind == "never"
     got = mp.furthest_point_sample(xyz.cuda(), npoint, 3, skip, strategy="single")
     np.testing.assert_array_equal(got.cpu().numpy(), O.fps(xyz, npoint, 3, skip))
+
+
+@pytest.mark.parametrize("sizes", [[8193, 1, 64, 700, 0, 4097], [24576, 24575, 513, 2], [9000, 512, 16384]])
+def test_ragged_fps_with_a_large_cloud_matches_oracle(cuda_device, sizes):
+    """Clouds of every size in one launch of the kernel the largest needs."""
+    from mps_pointops import flat
+
+    g = torch.Generator().manual_seed(len(sizes))
+    x = torch.randn(sum(sizes), 3, generator=g)
+    ptr = [0] + torch.tensor(sizes).cumsum(0).tolist()
+    got = flat.fps(x.cuda(), ratio=0.02, random_start=False, ptr=ptr).cpu().numpy()
+    want = []
+    for a, b in zip(ptr, ptr[1:]):
+        count = int(np.ceil(np.float32(b - a) * np.float32(0.02)))
+        if count:
+            want.append(a + O.fps(x[None, a:b], count, 0)[0])
+    np.testing.assert_array_equal(got, np.concatenate(want))
