@@ -124,12 +124,10 @@ hipError_t pointops_nearest3_grid(const float *query, const float *ref, float *d
                                   hipStream_t stream);
 
 /* The same search (identical results) for clouds of 1 <= N <= 8192
- * references, M <= 16384 queries and 1 <= K <= 32, faster: one workgroup per
- * cloud counting-sorts the references by Morton cell into `workspace`
- * (pointops_knn3_windowed_workspace_bytes(B, M, N) bytes, no initialisation
- * needed), and each query starts from a limit taken from the references
- * around its own cell in that order, so that only references at least that
- * near are buffered and merged.  Replaces ops.py:195-199
+ * references, M <= 16384 queries and 1 <= K <= 32, faster: screened on the
+ * matrix cores (pointops_knn_screen), the references' operands made once into
+ * `workspace` (pointops_knn3_windowed_workspace_bytes(B, M, N) bytes, 16-byte
+ * aligned, no initialisation needed).  Replaces ops.py:195-199
  * (kernels/knn.metal:32-140), like pointops_knn3. */
 size_t pointops_knn3_windowed_workspace_bytes(int64_t B, int64_t M, int64_t N);
 hipError_t pointops_knn3_windowed(const float *query, const float *ref, float *dist, int64_t *idx,
@@ -143,6 +141,18 @@ hipError_t pointops_knn_feat(const float *query, const float *ref, float *dist, 
                              int64_t B, int64_t M, int64_t N, int64_t D, int64_t K,
                              hipStream_t stream);
 
+/* The dense search (identical results: pointops_knn3 for D = 3, else
+ * pointops_knn_feat) screened on the matrix cores: products of operands split
+ * into bfloat16 parts, with a bound on their error, rule out all but about K
+ * references of each query, whose distances are then computed and ranked as
+ * the other entry points do.  D <= 128, K <= 64.  `workspace`:
+ * pointops_knn_screen_workspace_bytes(B, N, D) bytes, 16-byte aligned, no
+ * initialisation needed.  Replaces ops.py:195-204 like those entry points. */
+size_t pointops_knn_screen_workspace_bytes(int64_t B, int64_t N, int64_t D);
+hipError_t pointops_knn_screen(const float *query, const float *ref, float *dist, int64_t *idx,
+                               void *workspace, int64_t B, int64_t M, int64_t N, int64_t D,
+                               int64_t K, hipStream_t stream);
+
 /* Flat (ragged) kNN, global x indices padded with -1, (Q,K).  Replaces
  * _flat_search_mps.py:96-107 (kernels/flat_search.metal:44-154 for D = 3,
  * kernels/feature_knn.metal:166-199 otherwise).  y (Q,D) queries, x (Nx,D)
@@ -150,6 +160,15 @@ hipError_t pointops_knn_feat(const float *query, const float *ref, float *dist, 
 hipError_t pointops_knn_flat(const float *y, const float *x, const int64_t *ptr_y,
                              const int64_t *ptr_x, int64_t *out, int64_t Q, int64_t batch,
                              int64_t D, int64_t K, hipStream_t stream);
+/* The same flat search (identical results) screened as pointops_knn_screen;
+ * D <= 128, K <= 64; total_x is x's row count, ptr_x[batch] at most that.
+ * `workspace`: pointops_knn_flat_screen_workspace_bytes(total_x, batch, D)
+ * bytes, 16-byte aligned, no initialisation needed. */
+size_t pointops_knn_flat_screen_workspace_bytes(int64_t total_x, int64_t batch, int64_t D);
+hipError_t pointops_knn_flat_screen(const float *y, const float *x, const int64_t *ptr_y,
+                                    const int64_t *ptr_x, int64_t *out, void *workspace, int64_t Q,
+                                    int64_t total_x, int64_t batch, int64_t D, int64_t K,
+                                    hipStream_t stream);
 
 /* ----------------------------------------------------------- ball query */
 

@@ -1570,11 +1570,12 @@ __global__ __launch_bounds__(kLeadThreads) void fps_lead_kernel(
 // one box test and ballot; the tiles of a block of 4 steps are loaded
 // together, 4 tiles at a time, and each point is read once for all its steps.
 //
-// What bounds it: the leader's step chain and the exchanges, as in
-// fps_lead_kernel; the whole cloud is only read in the first few runs.  The
-// kernel it replaces (one workgroup, every point re-read from L2 in every
-// step) was bound by that read: 17.8 ms for 8 x 16384 points, 4096 samples
-// (4.35 us a step).
+// What bounds it: the exchanges.  At 8 x 16384 points, 4096 samples the leader
+// takes 320 cycles a step and an exchange (160 of them) 17600, of which the
+// followers' scan, cut and candidates are 4000 and the rest the slowest one's
+// lag (8 tile reads a step over the followers, each behind an L2 latency).
+// 1.9 ms; the kernel it replaces, which re-read the cloud from L2 in every
+// step, took 17.8 ms (4.35 us a step).
 constexpr int kWideMaxTiles = 48;  // tiles per follower: 6 bytes x 24576 points of LDS
 constexpr int64_t kWideMaxPoints = int64_t(kWideMaxTiles) * kLeadFollowers * kWave;
 constexpr int kWideBatch = 4;      // tiles loaded together

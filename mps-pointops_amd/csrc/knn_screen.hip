@@ -1,0 +1,974 @@
+// Exact kNN for gfx950, screened on the matrix cores.
+//
+// The searches define every rounding of a distance (knn.hip), which a matrix
+// product cannot reproduce, but it can tell which references cannot be among
+// the K nearest.  Each block serves 64 queries of one cloud; its four waves
+// split the cloud's tiles of 32 references and twice compute, for all pairs,
+//
+//     s = |r|^2 - 2 q.r     (the squared distance less |q|^2)
+//
+// on the matrix cores.  For D = 3 the operands are split into two bf16 parts
+// and all the products and a three-part norm are the 16 slots of one
+// v_mfma_f32_32x32x16_bf16; other widths take the coordinates, relative to a
+// centre and scaled, in f16.  |s + |q|^2 - d| <= E, with d the exact kernels'
+// rounded squared distance and E = err (|q| + max |r|)^2 (see screen_error).
+//
+// Pass 1 keeps, per query, the minima of 128 groups of references: one
+// v_min3 for two pairs.  K groups hold K distinct references, so the K-th
+// smallest minimum T bounds the K-th smallest d by T + |q|^2 + E, and every
+// neighbour has s <= T + 2E.  Pass 2 repeats the products and lists the
+// references at or below that (about K + K^2 / 256 of them, plus those within
+// 2E).  The listed references' distances are then computed as the searches
+// define them, and ranked by (distance, index): the results are the other
+// kernels' bit for bit.  Consecutive references fall into different groups,
+// so an order that puts neighbours next to each other does not spoil T.
+//
+// A query that the screen cannot serve (more than kScreenCap references
+// listed, as among many copies of one point; a coordinate that is not finite
+// or beyond 2^50 in its cloud) is searched by one wave over all references,
+// inside the same launch.
+//
+// What bounds it: not the products (134 M pairs at config 2 are 5500 cycles a
+// block) but the phases around them, in cycles of a block at 32 x 1024 queries
+// x 4096 references, k = 16: prologue 4200, pass 1 5300, limits 7000, pass 2
+// 21000 (the hits' masks and appends), exact distances and ranks 10500; at 8 x
+// 2048 x 2048, D = 64, k = 20: 11200, 14000, 14000, 16500, 33000 (each listed
+// row is 256 bytes from L2).  Measured: config 2 98 -> 43 us, 16 x 512 x 1024
+// 41 -> 18 us, D = 64 359 -> 53 us, D = 128 590 -> 75 us (one lane per query,
+// every pair's distance as defined), 3 ragged clouds of 20000, k = 16 1000 ->
+// 190 us (one wave per query).  Eight waves a block, since four left every
+// phase waiting on its own latency (65 against 43 us at config 2); bfloat16 in
+// three products instead of f16 in one took 61 us for D = 64.
+#include <type_traits>
+
+#include "knn_wave.hpp"
+#include "pointops_common.hpp"
+#include "pointops_hip.h"
+
+namespace pointops {
+namespace {
+
+constexpr int kScreenThreads = 512;
+constexpr int kScreenWaves = kScreenThreads / kWave;
+constexpr int kPrepThreads = 256;
+constexpr int kScreenQueries = 64;  // per block
+constexpr int kTileRefs = 32;       // references per tile: the rows of one product
+constexpr int kScreenGroups = 128;  // minima per query
+constexpr int kScreenCap = 128;     // listed references per query
+constexpr int kScreenMaxK = 64;
+constexpr int kGroupStride = 72;    // floats between groups: 8 groups x 8 queries hit 64 banks
+constexpr float kScreenMaxSq = 1.2676506e30f;  // 2^100: squares of sums stay finite
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+struct ScreenLayout {
+    uint4* frag;    // per tile and k-step: 64 lanes x 8 bf16 or f16
+    float* norm;    // D != 3: |r|^2 per tile row (+inf behind the last reference)
+    float* far_sq;  // per tile: largest |r|^2 (+inf: not to be screened)
+};
+
+// Tiles are numbered by segment: segment b's begin at lo / 32 + b, where lo is
+// its first row, which leaves room for a partial tile per segment.
+__host__ __device__ inline int64_t screen_tiles(int64_t rows, int64_t batch) {
+    return rows / kTileRefs + batch;
+}
+
+// k-steps of 16 dimensions.
+__host__ __device__ inline int screen_steps(int64_t D) { return D == 3 ? 1 : static_cast<int>((D + 15) / 16); }
+
+size_t screen_layout(int64_t rows, int64_t batch, int64_t D, ScreenLayout* L, char* base) {
+    const int64_t tiles = screen_tiles(rows, batch);
+    const size_t frag = static_cast<size_t>(tiles) * screen_steps(D) * kWave * sizeof(uint4);
+    const size_t norm = D == 3 ? 0 : static_cast<size_t>(tiles) * kTileRefs * sizeof(float);
+    if (L != nullptr) {
+        L->frag = reinterpret_cast<uint4*>(base);
+        L->norm = reinterpret_cast<float*>(base + frag);
+        L->far_sq = reinterpret_cast<float*>(base + frag + norm);
+    }
+    return frag + norm + static_cast<size_t>(tiles) * sizeof(float);
+}
+
+// The relative error of the screen, against (|q| + max |r|)^2, which is at
+// least |q - r|^2 and four times |q| |r|.
+// D = 3: a two-part operand is within 2^-16 of the float (relative), so the
+// doubled products of a pair are within 4 x 2^-16 |q| |r|, a quarter of which
+// counts: 2^-16; 16 terms summed in float32, 2^-23 each (allowing for
+// truncation), the norms and the exact kernels' own rounding add 2^-18.
+// Others: an f16 operand is within 2^-11, so the doubled products are within
+// 4 x 2^-11 |q| |r|: 2^-11; D terms at 2^-23 and 2 (D + 6) 2^-24 for the norms
+// and the exact chain.  (Coordinates below f16's normal range lose at most
+// 2^-25 of the scaled unit each: screen_slack.)
+__host__ __device__ inline float screen_error(int D) {
+    return D == 3 ? 2.3e-5f : 4.8828125e-4f * 1.02f + static_cast<float>(D + 6) * 3.6e-7f;
+}
+// Absolute slack, in the scale of s: operands and products below the normal
+// ranges, and exact distances (of unscaled coordinates) below float32's, each
+// of whose roundings may be off by 2^-149.
+__host__ __device__ inline float screen_slack(int D, float span, float scale) {
+    if (D == 3) return 1e-30f;
+    const float tiny = scale * 5.3e-23f;  // 2^-74
+    return 1e-30f + span * static_cast<float>(D) * 1.2e-7f + static_cast<float>(2 * D) * (tiny * tiny);
+}
+
+// bf16 parts of a float, rounded to nearest: v = hi + lo to 2^-18.
+__device__ __forceinline__ uint32_t bf16_bits(float v) {
+    const uint32_t u = static_cast<uint32_t>(f2i(v));
+    return (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
+}
+__device__ __forceinline__ float bf16_value(uint32_t bits) { return i2f(static_cast<int>(bits << 16)); }
+__device__ __forceinline__ void bf16_split(float v, uint32_t& hi, uint32_t& lo) {
+    hi = bf16_bits(v);
+    lo = bf16_bits(v - bf16_value(hi));
+}
+
+__device__ __forceinline__ uint4 pack8(const uint32_t (&v)[8]) {
+    return make_uint4(v[0] | v[1] << 16, v[2] | v[3] << 16, v[4] | v[5] << 16, v[6] | v[7] << 16);
+}
+
+__device__ __forceinline__ bf16x8 as_bf16(uint4 v) { return __builtin_bit_cast(bf16x8, v); }
+__device__ __forceinline__ f16x8 as_f16(uint4 v) { return __builtin_bit_cast(f16x8, v); }
+
+// Eight floats rounded to f16 (to nearest; infinite beyond its range).
+__device__ __forceinline__ uint4 f16_frag(const float (&f)[8]) {
+    f16x8 v;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = static_cast<_Float16>(f[i]);
+    return __builtin_bit_cast(uint4, v);
+}
+
+// Centre of a 3-D segment for the screen (its coordinates are taken relative
+// to it, which keeps E small for clouds far from the origin): the mean of 8
+// points spread over it.  Any point serves; 0 if a coordinate is not finite.
+__device__ __forceinline__ void screen_centre(const float* __restrict__ ref, int64_t n, float (&c)[3]) {
+    float s[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float* p = ref + 3 * ((n * i) >> 3);
+        s[0] += p[0];
+        s[1] += p[1];
+        s[2] += p[2];
+    }
+#pragma unroll
+    for (int a = 0; a < 3; ++a) c[a] = isfinite(s[a]) ? s[a] * 0.125f : 0.f;
+}
+
+// Eight dimensions from d0 of a row (0 behind the last).
+__device__ __forceinline__ void load8(const float* __restrict__ r, int d0, int D, bool vec, float (&f)[8]) {
+    if (vec) {
+        // Unconditional loads (of dimension 0 behind the last), so that a
+        // row's are all in flight together.
+        const bool in_a = d0 < D, in_b = d0 + 4 < D;
+        const float4 a = *reinterpret_cast<const float4*>(r + (in_a ? d0 : 0));
+        const float4 b = *reinterpret_cast<const float4*>(r + (in_b ? d0 + 4 : 0));
+        f[0] = in_a ? a.x : 0.f; f[1] = in_a ? a.y : 0.f; f[2] = in_a ? a.z : 0.f; f[3] = in_a ? a.w : 0.f;
+        f[4] = in_b ? b.x : 0.f; f[5] = in_b ? b.y : 0.f; f[6] = in_b ? b.z : 0.f; f[7] = in_b ? b.w : 0.f;
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) f[i] = d0 + i < D ? r[d0 + i] : 0.f;
+    }
+}
+
+// Centre and scale of a feature segment, from 8 rows spread over it: their
+// mean (any point serves; 0 where it is not finite) to centre[], 0 behind D, and the
+// power of two that takes the largest difference between their coordinates to
+// [4, 8).  f16 reaches 8000 times further, and a row beyond that is not
+// screened.  One wave, lane l for dimensions l and l + 64; every wave of a
+// launch computes the same values for a segment.
+constexpr int kScreenMaxD = 128;
+__device__ __forceinline__ float screen_frame(const float* __restrict__ ref, int64_t n, int D, int lane,
+                                              float* centre) {
+    float most = 0.f;
+    for (int t = lane; t < D; t += kWave) {
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = ref[((n * i) >> 3) * D + t];
+        float sum = v[0];
+#pragma unroll
+        for (int i = 1; i < 8; ++i) {
+            sum = sum + v[i];
+            most = fmaxf(most, fabsf(v[i] - v[0]));
+        }
+        centre[t] = isfinite(sum) ? sum * 0.125f : 0.f;
+    }
+    for (int t = D + lane; t < kScreenMaxD; t += kWave) centre[t] = 0.f;
+    most = wave_max(most);  // (NaN is ignored here and found in its own row)
+    if (!(most > 1e-25f && most < 1e25f)) return 1.f;
+    const int e = ((f2i(most) >> 23) & 0xFF) - 127;  // most in [2^e, 2^(e+1))
+    return i2f((2 - e + 127) << 23);
+}
+
+// Segment of the references (rows) or queries of tile / block t.
+struct ScreenSegment {
+    int64_t b;    // cloud
+    int64_t lo;   // its first row
+    int64_t n;    // its rows
+    int64_t at;   // first row of this tile / block within it
+};
+
+// Tile or block `t` of `per` rows in the numbering of screen_tiles.
+__device__ __forceinline__ ScreenSegment screen_segment(const int64_t* __restrict__ ptr, int64_t batch,
+                                                        int64_t t, int per) {
+    int64_t lo = 0, hi = batch - 1;
+    while (lo < hi) {  // the last segment that begins at or before t
+        const int64_t mid = lo + (hi - lo + 1) / 2;
+        if (ptr[mid] / per + mid <= t) lo = mid;
+        else hi = mid - 1;
+    }
+    ScreenSegment s;
+    s.b = lo;
+    s.lo = ptr[lo];
+    s.n = ptr[lo + 1] - s.lo;
+    s.at = (t - (s.lo / per + lo)) * per;
+    return s;
+}
+
+// Half (lane / 32) of a 3-D reference's slots, its coordinates relative to the
+// centre: h, h, l, l of the coordinates, then the norm; a row behind the last
+// reference is 0 with an infinite norm.  `sq`: its squared norm.
+__device__ __forceinline__ uint4 ref_frag3(float x, float y, float z, bool valid, int half, float& sq) {
+    sq = x * x + y * y + z * z;
+    uint32_t h[3], l[3], nh, nm, nl;
+    bf16_split(x, h[0], l[0]);
+    bf16_split(y, h[1], l[1]);
+    bf16_split(z, h[2], l[2]);
+    nh = bf16_bits(sq);
+    bf16_split(sq - bf16_value(nh), nm, nl);
+    uint32_t v[8] = {h[0], h[1], h[2], h[0], h[1], h[2], l[0], l[1]};
+    const uint32_t w[8] = {l[2], l[0], l[1], l[2], nh, nm, nl, 0};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        v[i] = half ? w[i] : v[i];
+        v[i] = valid ? v[i] : (half && i == 4 ? 0x7F80u : 0u);
+    }
+    return pack8(v);
+}
+
+// A valid row's part in its tile's or cloud's largest squared norm: +inf where
+// it is not to be screened (NaN compares false).
+__device__ __forceinline__ float far_of(float sq, bool valid) {
+    return valid ? (sq < kScreenMaxSq ? sq : INFINITY) : 0.f;
+}
+
+// One wave per tile: the references' fragments, norms and largest norm.
+// Lane l holds row l % 32 and dimensions 8 (l / 32) .. + 7 of each k-step.
+template <bool D3, bool FLAT>
+__global__ __launch_bounds__(kPrepThreads) void screen_prep_kernel(
+    const float* __restrict__ ref, const int64_t* __restrict__ ptr, ScreenLayout L, int64_t batch,
+    int64_t N, int64_t tiles, int D, int steps) {
+    const int lane = lane_id();
+    const int64_t t = static_cast<int64_t>(blockIdx.x) * (kPrepThreads / kWave) + uniform(threadIdx.x / kWave);
+    if (t >= tiles) return;
+    ScreenSegment s;
+    if constexpr (FLAT) {
+        s = screen_segment(ptr, batch, t, kTileRefs);
+    } else {  // every cloud has the same number of tiles here
+        const int64_t per = (N + kTileRefs - 1) / kTileRefs;
+        s.b = t / per;
+        s.lo = s.b * N;
+        s.n = N;
+        s.at = (t - s.b * per) * kTileRefs;
+    }
+    if (s.at >= s.n) return;  // a number no segment uses
+    const int row = lane & 31, half = lane >> 5;
+    const bool valid = s.at + row < s.n;
+    const float* r = ref + (s.lo + (valid ? s.at + row : 0)) * D;
+    float sq = 0.f;
+    if constexpr (D3) {
+        float c[3];
+        screen_centre(ref + 3 * s.lo, s.n, c);
+        L.frag[t * kWave + lane] = ref_frag3(r[0] - c[0], r[1] - c[1], r[2] - c[2], valid, half, sq);
+    } else {
+        // Coordinates relative to the segment's centre, scaled.
+        const bool vec = D % 4 == 0 && reinterpret_cast<uintptr_t>(ref) % 16 == 0;
+        __shared__ __align__(16) float centres[kPrepThreads / kWave][kScreenMaxD];
+        float* const centre = centres[uniform(threadIdx.x / kWave)];
+        const float scale = screen_frame(ref + s.lo * D, s.n, D, lane, centre);
+        __builtin_amdgcn_wave_barrier();
+        for (int k = 0; k < steps; ++k) {
+            const int d0 = 16 * k + 8 * half;
+            float f[8], o[8];
+            load8(r, d0, D, vec, f);
+            load8(centre, d0, kScreenMaxD, true, o);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                f[i] = valid ? (f[i] - o[i]) * scale : 0.f;  // (0 behind D)
+                sq = sq + f[i] * f[i];
+                if (!(fabsf(f[i]) < 65000.f)) sq = INFINITY;  // beyond f16, or NaN
+            }
+            L.frag[(t * steps + k) * kWave + lane] = f16_frag(f);
+        }
+        sq = sq + __shfl_xor(sq, 32, kWave);
+        if (half == 0) L.norm[t * kTileRefs + row] = valid ? sq : INFINITY;
+    }
+    const float most = wave_max(far_of(sq, valid));
+    if (lane == 0) L.far_sq[t] = most;
+}
+
+struct ScreenArgs {
+    const float* query;
+    const float* ref;
+    const int64_t* ptr_y;  // FLAT: segment offsets of the queries and references
+    const int64_t* ptr_x;
+    float* dist;           // dense outputs
+    int64_t* idx;          // dense or flat indices
+    ScreenLayout L;
+    int64_t batch, M, N, QS;  // dense: queries of a cloud lie QS rows apart
+    int D, K;
+};
+
+// KS k-steps (D <= 16 KS); D3: one fragment holds everything.  Eight waves,
+// each with an eighth of the tiles against all 64 queries (two columns of 32).
+// PREP: the fragments come from screen_prep_kernel; otherwise (D3 only) each
+// wave makes them from the coordinates as it goes, twice, which for small
+// clouds costs less than a launch.
+template <int KS, bool D3, bool FLAT, bool PREP>
+__global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(const ScreenArgs a) {
+    constexpr int kBatch = D3 ? 4 : KS <= 4 ? 2 : 1;  // tiles in flight
+    constexpr int kU = 2;               // columns of 32 queries
+    constexpr int kFold = kScreenWaves * kTileRefs / kScreenGroups;  // rows of a lane per group
+    // Pass 1's minima (and the rows of the exact phase).
+    __shared__ __align__(16) float groups[kScreenGroups * kGroupStride + 1024];
+    __shared__ __align__(16) uint32_t listed[kScreenQueries * kScreenCap];
+    __shared__ __align__(16) uint32_t own_keys[D3 ? 4 : kScreenQueries * kScreenCap];
+    __shared__ int count[kScreenQueries];
+    __shared__ float limit[kScreenQueries];
+    __shared__ float norm_q[kScreenQueries];
+    __shared__ float far_red[kScreenWaves];
+    __shared__ __align__(16) float centres[kScreenWaves][D3 ? 4 : kScreenMaxD];  // a copy per wave: no barrier
+    // The exact phase: the listed references' keys (where the minima were, for
+    // D3), and each wave's rows of 16 dimensions (where the minima were).
+    uint32_t* const keys = D3 ? reinterpret_cast<uint32_t*>(groups) : own_keys;
+    static_assert(kScreenGroups * kGroupStride >= kScreenQueries * kScreenCap, "keys fit");
+
+    const int tid = threadIdx.x;
+    const int lane = tid % kWave;
+    const int wave = uniform(tid / kWave);
+    const int col = lane & 31, half = lane >> 5;
+    const int D = a.D;
+    // This block's queries and their cloud's references.
+    int64_t row0, ref0, n, tile0, out0, b;
+    int nq;
+    if constexpr (FLAT) {
+        const ScreenSegment s = screen_segment(a.ptr_y, a.batch, blockIdx.x, kScreenQueries);
+        if (s.at >= s.n) return;  // a number no segment uses (uniform)
+        b = s.b;
+        row0 = out0 = s.lo + s.at;
+        nq = static_cast<int>(min<int64_t>(kScreenQueries, s.n - s.at));
+        ref0 = a.ptr_x[b];
+        n = a.ptr_x[b + 1] - ref0;
+        tile0 = ref0 / kTileRefs + b;
+    } else {
+        const CloudBlock cb = cloud_block(static_cast<uint32_t>((a.M + kScreenQueries - 1) / kScreenQueries));
+        b = cb.b;
+        const int64_t m0 = static_cast<int64_t>(cb.x) * kScreenQueries;
+        row0 = out0 = b * a.QS + m0;
+        nq = static_cast<int>(min<int64_t>(kScreenQueries, a.M - m0));
+        ref0 = b * a.N;
+        n = a.N;
+        tile0 = b * ((n + kTileRefs - 1) / kTileRefs);
+    }
+    const int tiles = static_cast<int>((n + kTileRefs - 1) / kTileRefs);
+    const int K = static_cast<int>(min<int64_t>(a.K, n));
+
+    // ---- the queries' fragments, of -2 q (exact), and norms
+    uint4 bq[kU][KS];
+    float c[3] = {0.f, 0.f, 0.f};
+    if constexpr (D3) {
+        if (n > 0) screen_centre(a.ref + 3 * ref0, n, c);
+    }
+    const bool vec = D % 4 == 0 && reinterpret_cast<uintptr_t>(a.query) % 16 == 0;
+    const bool vec_rows = vec && reinterpret_cast<uintptr_t>(a.ref) % 16 == 0;
+    float scale = 1.f;
+    if constexpr (!D3) {
+        if (n > 0) scale = screen_frame(a.ref + ref0 * D, n, D, lane, centres[wave]);
+        else for (int t = lane; t < kScreenMaxD; t += kWave) centres[wave][t] = 0.f;
+        __builtin_amdgcn_wave_barrier();
+    }
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+        const int qi = 32 * u + col;
+        const float* q = a.query + (row0 + (qi < nq ? qi : 0)) * D;
+        float sq = 0.f;
+        if constexpr (D3) {
+            const float x = q[0] - c[0], y = q[1] - c[1], z = q[2] - c[2];
+            sq = x * x + y * y + z * z;
+            uint32_t h[3], l[3];
+            bf16_split(-2.f * x, h[0], l[0]);
+            bf16_split(-2.f * y, h[1], l[1]);
+            bf16_split(-2.f * z, h[2], l[2]);
+            // Slots: h, l, h, l against the references' h, h, l, l; 1 against the norm's parts.
+            uint32_t v[8] = {h[0], h[1], h[2], l[0], l[1], l[2], h[0], h[1]};
+            const uint32_t w[8] = {h[2], l[0], l[1], l[2], 0x3F80u, 0x3F80u, 0x3F80u, 0};
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = half ? w[i] : v[i];
+            bq[u][0] = pack8(v);
+        } else {
+#pragma unroll
+            for (int k = 0; k < KS; ++k) {
+                const int d0 = 16 * k + 8 * half;
+                float f[8], o[8];
+                load8(q, d0, D, vec, f);
+                load8(centres[wave], d0, kScreenMaxD, true, o);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    f[i] = (f[i] - o[i]) * scale;  // (0 behind D)
+                    sq = sq + f[i] * f[i];
+                    if (!(fabsf(f[i]) < 32000.f)) sq = INFINITY;  // -2 f beyond f16, or NaN
+                    f[i] = -2.f * f[i];
+                }
+                bq[u][k] = f16_frag(f);
+            }
+            sq = sq + __shfl_xor(sq, 32, kWave);
+        }
+        if (wave == 0 && half == 0) norm_q[qi] = sq;
+    }
+    if (tid < kScreenQueries) count[tid] = 0;
+    float my_far = 0.f;  // without PREP: of the rows this lane has seen
+    if constexpr (PREP) {
+        float far_sq = 0.f;
+        for (int i = tid; i < tiles; i += kScreenThreads) far_sq = fmaxf(far_sq, a.L.far_sq[tile0 + i]);
+        far_sq = wave_max(far_sq);
+        if (lane == 0) far_red[wave] = far_sq;
+    }
+
+    // The screen of one tile against the wave's queries: acc[u][i] is
+    // s of reference 8 (i / 4) + 4 half + i % 4 and query 32 (u0 + u) + col.
+    auto load = [&](int t, uint4 (&f)[KS], float4 (&nr)[D3 ? 1 : 4]) {
+        if constexpr (!PREP) {  // the coordinates, for as_fragment
+            const float* r = a.ref + 3 * (ref0 + min<int64_t>(t * kTileRefs + col, n - 1));
+            f[0] = make_uint4(f2i(r[0]), f2i(r[1]), f2i(r[2]), 0);
+            return;
+        }
+        const uint4* src = a.L.frag + (tile0 + t) * KS * kWave + lane;
+#pragma unroll
+        for (int k = 0; k < KS; ++k) f[k] = src[k * kWave];
+        if constexpr (!D3) {
+            const float* nrm = a.L.norm + (tile0 + t) * kTileRefs + 4 * half;
+#pragma unroll
+            for (int g = 0; g < 4; ++g) nr[g] = *reinterpret_cast<const float4*>(nrm + 8 * g);
+        }
+    };
+    auto as_fragment = [&](int t, uint4& f) {
+        if constexpr (!PREP) {
+            const bool valid = t * kTileRefs + col < n;
+            float sq;
+            f = ref_frag3(i2f(f.x) - c[0], i2f(f.y) - c[1], i2f(f.z) - c[2], valid, half, sq);
+            my_far = fmaxf(my_far, far_of(sq, valid));
+        }
+    };
+    auto screen = [&](const uint4 (&f)[KS], const float4 (&nr)[D3 ? 1 : 4], f32x16 (&acc)[kU]) {
+        if constexpr (D3) {
+            const f32x16 zero = {};
+#pragma unroll
+            for (int u = 0; u < kU; ++u)
+                acc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16(f[0]), as_bf16(bq[u][0]), zero, 0, 0, 0);
+        } else {
+#pragma unroll
+            for (int u = 0; u < kU; ++u)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    acc[u][4 * g] = nr[g].x;
+                    acc[u][4 * g + 1] = nr[g].y;
+                    acc[u][4 * g + 2] = nr[g].z;
+                    acc[u][4 * g + 3] = nr[g].w;
+                }
+#pragma unroll
+            for (int k = 0; k < KS; ++k)
+#pragma unroll
+                for (int u = 0; u < kU; ++u)
+                    acc[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16(f[k]), as_f16(bq[u][k]), acc[u], 0, 0, 0);
+        }
+    };
+    // The wave's tiles, kBatch at a time (the next ones requested before the
+    // current ones are used): use(j, t, acc) for t = t0 + kScreenWaves j, then
+    // flush(t0), for every batch.  Tiles behind the last are replaced by the
+    // wave's first; use() sees t.
+    auto walk = [&](auto use, auto flush) {
+        if (wave >= tiles) return;
+        uint4 f[kBatch][KS];
+        float4 nr[kBatch][D3 ? 1 : 4];
+        auto fetch = [&](int t0) {
+#pragma unroll
+            for (int j = 0; j < kBatch; ++j) {
+                const int t = t0 + j * kScreenWaves;
+                load(t < tiles ? t : wave, f[j], nr[j]);
+            }
+        };
+        fetch(wave);
+        for (int t0 = wave; t0 < tiles; t0 += kBatch * kScreenWaves) {
+            uint4 cf[kBatch][KS];
+            float4 cn[kBatch][D3 ? 1 : 4];
+#pragma unroll
+            for (int j = 0; j < kBatch; ++j) {
+#pragma unroll
+                for (int k = 0; k < KS; ++k) cf[j][k] = f[j][k];
+#pragma unroll
+                for (int g = 0; g < (D3 ? 1 : 4); ++g) cn[j][g] = nr[j][g];
+            }
+            fetch(t0 + kBatch * kScreenWaves);
+#pragma unroll
+            for (int j = 0; j < kBatch; ++j) {
+                f32x16 acc[kU];
+                const int t = t0 + j * kScreenWaves;
+                as_fragment(t < tiles ? t : wave, cf[j][0]);
+                screen(cf[j], cn[j], acc);
+                use(j, t, acc);
+            }
+            flush(t0);
+        }
+    };
+
+    // ---- pass 1: group minima
+    {
+        float m[kU][16];
+#pragma unroll
+        for (int u = 0; u < kU; ++u)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) m[u][i] = INFINITY;
+        walk([&](int, int, const f32x16 (&acc)[kU]) {  // (a tile again changes no minimum)
+#pragma unroll
+            for (int u = 0; u < kU; ++u)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) m[u][i] = fminf(m[u][i], acc[u][i]);
+        }, [](int) {});
+#pragma unroll
+        for (int u = 0; u < kU; ++u)
+#pragma unroll
+            for (int i = 0; i < 16 / kFold; ++i) {
+                float v = m[u][i];
+                if constexpr (kFold == 2) v = fminf(v, m[u][i + 8]);  // 16 references on
+                groups[((2 * wave + half) * (16 / kFold) + i) * kGroupStride + 32 * u + col] = v;
+            }
+    }
+    if constexpr (!PREP) {
+        my_far = wave_max(my_far);
+        if (lane == 0) far_red[wave] = my_far;
+    }
+    __syncthreads();  // minima, norms, largest norms, cleared counts
+    float far_sq = far_red[0];
+#pragma unroll
+    for (int w = 1; w < kScreenWaves; ++w) far_sq = fmaxf(far_sq, far_red[w]);
+
+    // ---- the limit of each query: eight lanes per query, 16 groups each,
+    // searched for the K-th smallest minimum.  Any threshold that K groups
+    // reach serves; the search ends at one that few more reach.
+    {
+        const int qi = wave * 8 + (lane >> 3), part = lane & 7;
+        const float nq_sq = norm_q[qi];
+        float v[kScreenGroups / 8];
+        float lo = INFINITY, hi = 0.f, sum = 0.f, some = 0.f;
+#pragma unroll
+        for (int k = 0; k < kScreenGroups / 8; ++k) {
+            // fmaxf maps NaN to 0: such a query is not served by the screen.
+            v[k] = fmaxf(groups[(8 * k + part) * kGroupStride + qi] + nq_sq, 0.f);
+            const bool real = v[k] < INFINITY;  // the group holds a reference
+            lo = fminf(lo, v[k]);
+            hi = fmaxf(hi, real ? v[k] : 0.f);
+            sum = sum + (real ? v[k] : 0.f);
+            some = some + (real ? 1.f : 0.f);
+        }
+        auto dpp_f = [](float x, auto ctrl) { return i2f(dpp<decltype(ctrl)::value>(f2i(x))); };
+        auto eight = [&](float x, auto op) {  // over the query's eight lanes
+            x = op(x, dpp_f(x, std::integral_constant<int, kDppQuadXor1>{}));
+            x = op(x, dpp_f(x, std::integral_constant<int, kDppQuadXor2>{}));
+            return op(x, dpp_f(x, std::integral_constant<int, kDppRowHalfMirror>{}));
+        };
+        const float least = eight(lo, [](float x, float y) { return fminf(x, y); });
+        hi = eight(hi, [](float x, float y) { return fmaxf(x, y); });  // every such group is within hi
+        sum = eight(sum, [](float x, float y) { return x + y; });
+        some = eight(some, [](float x, float y) { return x + y; });
+        lo = least;
+        // The first guess takes the minima as exponentially distributed above
+        // the least; then the count says on which side, interpolating.
+        float guess = least + (sum / some - least) * -__logf(1.f - fminf(static_cast<float>(K) / some, 0.99f));
+        float reach_lo = 0.f, reach_hi = some;
+        if (some < static_cast<float>(K)) hi = 3e38f;  // everything finite is listed
+        const int most = K + 2 + K / 8;
+        bool done = some <= static_cast<float>(most);
+        for (int it = 0; it < 12 && ballot(!done) != 0; ++it) {
+            if (!(guess > lo && guess < hi) || it > 6) guess = 0.5f * (lo + hi);
+            float reach = 0.f;
+#pragma unroll
+            for (int k = 0; k < kScreenGroups / 8; ++k) reach += v[k] <= guess ? 1.f : 0.f;
+            reach = eight(reach, [](float x, float y) { return x + y; });
+            if (!done) {
+                if (reach >= K) {
+                    hi = guess;
+                    reach_hi = reach;
+                } else {
+                    lo = guess;
+                    reach_lo = reach;
+                }
+                done = reach >= K && reach <= most;
+                guess = lo + (hi - lo) * ((K + 1 - reach_lo) / (reach_hi - reach_lo));
+            }
+        }
+        if (part == 0) {
+            const float span = sqrtf(nq_sq) + sqrtf(far_sq);
+            const float e = screen_error(D) * (span * span) + screen_slack(D, span, scale);
+            // (In the coordinates' own scale, so that no distance overflows.)
+            const float back = 1.f / scale;
+            const bool served = qi < nq && nq_sq * back * back < kScreenMaxSq &&
+                                far_sq * back * back < kScreenMaxSq;
+            // (Finite, so that the rows behind the last, at +inf, are not listed.)
+            limit[qi] = served ? fminf(hi + 2.f * e - nq_sq, 3e38f) : -INFINITY;
+            if (qi < nq && !served) count[qi] = kScreenCap + 1;
+        }
+    }
+    __syncthreads();  // limits
+
+    // ---- pass 2: the references within each query's limit
+    {
+        float lim[kU];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) lim[u] = limit[32 * u + col];
+        // A batch's hits, 16 bits a tile, appended together: one atomic per
+        // lane and column with hits.
+        constexpr int kWords = (kBatch + 1) / 2;
+        uint32_t hit[kU][kWords] = {};
+        walk([&](int j, int t, const f32x16 (&acc)[kU]) {
+            const bool real = t < tiles;
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+                float least = acc[u][0];
+#pragma unroll
+                for (int i = 1; i < 16; ++i) least = fminf(least, acc[u][i]);
+                uint32_t h = 0;
+                if (ballot(least <= lim[u]) != 0 && real) {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) h |= acc[u][i] <= lim[u] ? 1u << i : 0u;
+                }
+                hit[u][j / 2] |= h << (16 * (j & 1));
+            }
+        }, [&](int t0) {
+            int at[kU];
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+                int n_hit = 0;
+#pragma unroll
+                for (int w = 0; w < kWords; ++w) n_hit += __popc(hit[u][w]);
+                at[u] = 0;
+                if (n_hit != 0) at[u] = atomicAdd(&count[32 * u + col], n_hit);
+            }
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+                uint32_t* list = listed + (32 * u + col) * kScreenCap;
+#pragma unroll
+                for (int w = 0; w < kWords; ++w)
+                    while (hit[u][w] != 0) {
+                        const int i = __builtin_ctz(hit[u][w]);
+                        hit[u][w] &= hit[u][w] - 1;
+                        // (Rows behind the last are at +inf, above every limit.)
+                        const int t = t0 + (2 * w + (i >> 4)) * kScreenWaves;
+                        if (at[u] < kScreenCap) list[at[u]] = t * kTileRefs + 8 * ((i >> 2) & 3) + 4 * half + (i & 3);
+                        ++at[u];
+                    }
+            }
+        });
+    }
+    __syncthreads();  // lists
+
+    // ---- exact distances: the wave's eight queries' lists end to end, a lane
+    // per listed reference
+    constexpr int kMine = kScreenQueries / kScreenWaves;
+    const int q0 = wave * kMine;
+    int first[kMine + 1];  // where each query's list begins
+    first[0] = 0;
+#pragma unroll
+    for (int i = 0; i < kMine; ++i) {
+        const int m = q0 + i < nq ? uniform(count[q0 + i]) : 0;
+        first[i + 1] = first[i] + (m > kScreenCap ? 0 : m);  // (longer: left over)
+    }
+    for (int e0 = 0; e0 < first[kMine]; e0 += kWave) {
+        const int e = e0 + lane;
+        const bool valid = e < first[kMine];
+        int i = 0, base = 0;
+#pragma unroll
+        for (int o = 1; o < kMine; ++o) {
+            const bool in = valid && e >= first[o];
+            i = in ? o : i;
+            base = in ? first[o] : base;
+        }
+        const int slot = (q0 + i) * kScreenCap + (valid ? e - base : 0);
+        const int64_t r = ref0 + (valid ? listed[slot] : 0);
+        const float* q = a.query + (row0 + q0 + i) * D;
+        float d;
+        if constexpr (D3) {
+            const float* rr = a.ref + 3 * r;
+            d = sqdist3(rr[0], rr[1], rr[2], q[0], q[1], q[2]);
+        } else if (vec_rows) {
+            // The 64 rows, 16 dimensions at a time, through LDS: four lanes
+            // read a row's 64 bytes together (a lane reading its own row
+            // would fetch each of its cache lines once per 16 bytes).
+            constexpr int kRow = 20;  // floats between rows: no bank conflicts
+            float4* const rows = reinterpret_cast<float4*>(groups + wave * kWave * kRow);
+            static_assert(kScreenWaves * kWave * kRow <= kScreenGroups * kGroupStride + 1024, "rows fit");
+            d = 0.f;  // 0 + d0^2 = d0^2
+            const int part = lane & 3;
+            float4 next[4], qn[4];
+            const float* src[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                qn[k] = 4 * k < D ? *reinterpret_cast<const float4*>(q + 4 * k) : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int64_t other = __shfl(r, 16 * k + (lane >> 2), kWave);
+                src[k] = a.ref + other * D + 4 * part;
+                next[k] = 4 * part < D ? *reinterpret_cast<const float4*>(src[k]) : make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+            for (int d0 = 0; d0 < D; d0 += 16) {
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int k = 0; k < 4; ++k) rows[(16 * k + (lane >> 2)) * (kRow / 4) + part] = next[k];
+                __builtin_amdgcn_wave_barrier();
+                float4 qc[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    qc[k] = qn[k];
+                    if (d0 + 16 + 4 * part < D) next[k] = *reinterpret_cast<const float4*>(src[k] + d0 + 16);
+                    if (d0 + 16 + 4 * k < D) qn[k] = *reinterpret_cast<const float4*>(q + d0 + 16 + 4 * k);
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    if (d0 + 4 * k >= D) break;
+                    const float4 x = rows[lane * (kRow / 4) + k];
+                    const float4 y = qc[k];
+                    const float x0 = x.x - y.x, x1 = x.y - y.y, x2 = x.z - y.z, x3 = x.w - y.w;
+                    d = d + x0 * x0;
+                    d = d + x1 * x1;
+                    d = d + x2 * x2;
+                    d = d + x3 * x3;
+                }
+            }
+        } else {
+            d = sqdist_nd(a.ref + r * D, q, D);
+        }
+        if (valid) keys[slot] = static_cast<uint32_t>(f2i(d));
+    }
+    __builtin_amdgcn_wave_barrier();
+
+    // ---- ranks: half a wave per query
+    for (int i = half; i < kMine; i += 2) {
+        const int qi = q0 + i;
+        if (qi >= nq || count[qi] > kScreenCap) continue;
+        const int m = count[qi];
+        const uint4* list4 = reinterpret_cast<const uint4*>(listed + qi * kScreenCap);
+        const uint4* key4 = reinterpret_cast<const uint4*>(keys + qi * kScreenCap);
+        for (int e = col; e < m; e += 32) {
+            const uint32_t key = keys[qi * kScreenCap + e], at = listed[qi * kScreenCap + e];
+            const uint64_t mine = static_cast<uint64_t>(key) << 32 | at;
+            int rank = 0;
+            auto before_mine = [&](uint32_t k, uint32_t r, int o) {
+                const uint64_t other = static_cast<uint64_t>(o < m ? k : 0xFFFFFFFFu) << 32 | r;
+                return other < mine ? 1 : 0;
+            };
+#pragma unroll 2
+            for (int o = 0; o < m; o += 4) {  // (entries behind the list are read, not counted)
+                const uint4 k = key4[o >> 2], l = list4[o >> 2];
+                rank += before_mine(k.x, l.x, o) + before_mine(k.y, l.y, o + 1) +
+                        before_mine(k.z, l.z, o + 2) + before_mine(k.w, l.w, o + 3);
+            }
+            if (rank < K) {
+                const int64_t slot = (out0 + qi) * a.K + rank;
+                if constexpr (FLAT) {
+                    a.idx[slot] = ref0 + at;
+                } else {
+                    a.dist[slot] = sqrtf(i2f(static_cast<int>(key)));
+                    a.idx[slot] = at;
+                }
+            }
+        }
+        if constexpr (FLAT)  // a segment of fewer than K references
+            for (int s = K + col; s < a.K; s += 32) a.idx[(out0 + qi) * a.K + s] = -1;
+    }
+
+    // ---- the queries left over: one wave each, over every reference
+    for (int qi = wave; qi < nq; qi += kScreenWaves) {
+        if (uniform(count[qi]) <= kScreenCap) continue;
+        const float* q = a.query + (row0 + qi) * D;
+        float ld[1] = {INFINITY};
+        int li[1] = {-1};
+        bool ok = true;
+        if constexpr (!D3 || FLAT)  // dense 3-D queries match at infinite distances
+            for (int t = 0; t < D; ++t) ok = ok && isfinite(q[t]);
+        if (ok)
+            scan_refs<1, D3, !D3 || FLAT>(q, a.ref + ref0 * D, static_cast<int>(n), D, a.K, lane, ld, li);
+        if (lane < a.K) {
+            const int64_t slot = (out0 + qi) * a.K + lane;
+            if constexpr (FLAT) {
+                a.idx[slot] = li[0] < 0 ? int64_t(-1) : ref0 + li[0];
+            } else {
+                a.dist[slot] = sqrtf(ld[0]);
+                a.idx[slot] = D3 ? static_cast<int64_t>(static_cast<uint32_t>(li[0]))
+                                 : (li[0] < 0 ? int64_t(-1) : int64_t(li[0]));
+            }
+        }
+    }
+}
+
+template <int KS, bool D3, bool FLAT, bool PREP = true>
+hipError_t launch_search(const ScreenArgs& a, int64_t blocks, hipStream_t stream) {
+    hipLaunchKernelGGL((knn_screen_kernel<KS, D3, FLAT, PREP>), dim3(static_cast<uint32_t>(blocks)),
+                       dim3(kScreenThreads), 0, stream, a);
+    return hipGetLastError();
+}
+
+// k-steps of the kernel that serves D dimensions.
+int screen_kernel_steps(int64_t D) {
+    const int s = screen_steps(D);
+    return D == 3 ? 1 : s <= 2 ? 2 : s <= 4 ? 4 : s <= 6 ? 6 : 8;
+}
+
+size_t screen_workspace(int64_t rows, int64_t batch, int64_t D, ScreenLayout* L = nullptr, void* base = nullptr) {
+    return screen_layout(rows, batch, D == 3 ? 3 : 16 * screen_kernel_steps(D), L, static_cast<char*>(base));
+}
+
+// The references' fragments (into a.L), which depend on the references alone.
+template <bool FLAT>
+hipError_t launch_prep(const ScreenArgs& a, int64_t ref_rows, hipStream_t stream) {
+    const int64_t tiles = FLAT ? screen_tiles(ref_rows, a.batch) : a.batch * ((a.N + kTileRefs - 1) / kTileRefs);
+    constexpr int kPrepWaves = kPrepThreads / kWave;
+    const dim3 grid(static_cast<uint32_t>((tiles + kPrepWaves - 1) / kPrepWaves));
+    if (a.D == 3)
+        hipLaunchKernelGGL((screen_prep_kernel<true, FLAT>), grid, dim3(kPrepThreads), 0, stream, a.ref,
+                           a.ptr_x, a.L, a.batch, a.N, tiles, a.D, 1);
+    else
+        hipLaunchKernelGGL((screen_prep_kernel<false, FLAT>), grid, dim3(kPrepThreads), 0, stream, a.ref,
+                           a.ptr_x, a.L, a.batch, a.N, tiles, a.D, screen_kernel_steps(a.D));
+    return hipGetLastError();
+}
+
+template <bool FLAT>
+hipError_t launch_blocks(const ScreenArgs& a, int64_t blocks, hipStream_t stream) {
+    switch (screen_kernel_steps(a.D)) {
+        case 1: return launch_search<1, true, FLAT>(a, blocks, stream);
+        case 2: return launch_search<2, false, FLAT>(a, blocks, stream);
+        case 4: return launch_search<4, false, FLAT>(a, blocks, stream);
+        case 6: return launch_search<6, false, FLAT>(a, blocks, stream);
+        default: return launch_search<8, false, FLAT>(a, blocks, stream);
+    }
+}
+
+template <bool FLAT>
+hipError_t launch_screen(ScreenArgs a, void* workspace, int64_t ref_rows, int64_t blocks,
+                         hipStream_t stream) {
+    screen_workspace(ref_rows, a.batch, a.D, &a.L, workspace);
+    const hipError_t err = launch_prep<FLAT>(a, ref_rows, stream);
+    return err != hipSuccess ? err : launch_blocks<FLAT>(a, blocks, stream);
+}
+
+int64_t screen_blocks(int64_t M, int64_t B) { return (M + kScreenQueries - 1) / kScreenQueries * B; }
+
+bool screen_fits(int64_t blocks, int64_t ref_rows, int64_t batch) {
+    return blocks <= INT32_MAX && screen_tiles(ref_rows, batch) <= INT32_MAX / 2;
+}
+
+}  // namespace
+}  // namespace pointops
+
+namespace pointops {
+
+// The dense 3-D search in two launches: knn3_screen_prepare (the references'
+// fragments into `workspace`, pointops_knn_screen_workspace_bytes(B, N, 3)
+// bytes) and knn3_screen_rows (the queries -- M rows per cloud whose rows,
+// queries and both outputs, lie QS rows apart -- over a workspace filled for
+// the same references, B and N, or without one).
+hipError_t knn3_screen_prepare(const float* ref, void* workspace, int64_t B, int64_t N, hipStream_t stream) {
+    if (B < 1 || N < 1 || workspace == nullptr || N > INT32_MAX - kWave || !screen_fits(B, B * N, B))
+        return hipErrorInvalidValue;
+    ScreenArgs a{};
+    a.ref = ref;
+    a.batch = B;
+    a.N = N;
+    a.D = 3;
+    screen_workspace(B * N, B, 3, &a.L, workspace);
+    return launch_prep<false>(a, B * N, stream);
+}
+
+hipError_t knn3_screen_rows(const float* query, const float* ref, float* dist, int64_t* idx,
+                            void* workspace, int64_t B, int64_t M, int64_t QS, int64_t N, int64_t K,
+                            hipStream_t stream) {
+    if (B < 1 || M < 1 || QS < M || K < 1 || K > kScreenMaxK || K > N || N > INT32_MAX - kWave ||
+        !screen_fits(screen_blocks(M, B), B * N, B))
+        return hipErrorInvalidValue;
+    ScreenArgs a{};
+    a.query = query;
+    a.ref = ref;
+    a.dist = dist;
+    a.idx = idx;
+    a.batch = B;
+    a.M = M;
+    a.N = N;
+    a.QS = QS;
+    a.D = 3;
+    a.K = static_cast<int>(K);
+    if (workspace == nullptr) return launch_search<1, true, false, false>(a, screen_blocks(M, B), stream);
+    screen_workspace(B * N, B, 3, &a.L, workspace);
+    return launch_blocks<false>(a, screen_blocks(M, B), stream);
+}
+
+}  // namespace pointops
+
+using namespace pointops;
+
+extern "C" {
+
+size_t pointops_knn_screen_workspace_bytes(int64_t B, int64_t N, int64_t D) {
+    if (B <= 0 || N <= 0 || D < 1 || D > 128) return 0;
+    return screen_workspace(B * N, B, D);
+}
+
+hipError_t pointops_knn_screen(const float* query, const float* ref, float* dist, int64_t* idx,
+                               void* workspace, int64_t B, int64_t M, int64_t N, int64_t D,
+                               int64_t K, hipStream_t stream) {
+    if (B < 0 || M < 0 || N < 0 || D < 1 || D > 128 || K < 0 || K > kScreenMaxK || K > N)
+        return hipErrorInvalidValue;
+    if (B == 0 || M == 0 || K == 0) return hipSuccess;
+    const int64_t blocks = screen_blocks(M, B);
+    if (workspace == nullptr || N > INT32_MAX - kWave || !screen_fits(blocks, B * N, B))
+        return hipErrorInvalidValue;
+    ScreenArgs a{};
+    a.query = query;
+    a.ref = ref;
+    a.dist = dist;
+    a.idx = idx;
+    a.batch = B;
+    a.M = M;
+    a.N = N;
+    a.QS = M;
+    a.D = static_cast<int>(D);
+    a.K = static_cast<int>(K);
+    return launch_screen<false>(a, workspace, B * N, blocks, stream);
+}
+
+size_t pointops_knn_flat_screen_workspace_bytes(int64_t total_x, int64_t batch, int64_t D) {
+    if (total_x < 0 || batch <= 0 || D < 1 || D > 128) return 0;
+    return screen_workspace(total_x, batch, D);
+}
+
+hipError_t pointops_knn_flat_screen(const float* y, const float* x, const int64_t* ptr_y,
+                                    const int64_t* ptr_x, int64_t* out, void* workspace, int64_t Q,
+                                    int64_t total_x, int64_t batch, int64_t D, int64_t K,
+                                    hipStream_t stream) {
+    if (Q < 0 || total_x < 0 || batch < 0 || D < 1 || D > 128 || K < 0 || K > kScreenMaxK)
+        return hipErrorInvalidValue;
+    if (Q == 0 || K == 0) return hipSuccess;
+    const int64_t blocks = Q / kScreenQueries + batch;
+    if (batch == 0 || workspace == nullptr || total_x > INT32_MAX - kWave ||
+        !screen_fits(blocks, total_x, batch))
+        return hipErrorInvalidValue;
+    ScreenArgs a{};
+    a.query = y;
+    a.ref = x;
+    a.ptr_y = ptr_y;
+    a.ptr_x = ptr_x;
+    a.idx = out;
+    a.batch = batch;
+    a.D = static_cast<int>(D);
+    a.K = static_cast<int>(K);
+    return launch_screen<true>(a, workspace, total_x, blocks, stream);
+}
+
+}  // extern "C"

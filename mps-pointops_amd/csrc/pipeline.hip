@@ -47,11 +47,11 @@ namespace pointops {
 hipError_t fps_dense_progress(const float* xyz, int64_t* out, int64_t B, int64_t N,
                               int64_t npoint, int64_t start, int skip, uint64_t* progress,
                               uint64_t tag, int64_t chunk, float* centres, hipStream_t stream);
-hipError_t knn3_window_sort(const float* ref, void* workspace, int64_t B, int64_t M, int64_t N,
+hipError_t knn3_screen_prepare(const float* ref, void* workspace, int64_t B, int64_t N,
+                               hipStream_t stream);
+hipError_t knn3_screen_rows(const float* query, const float* ref, float* dist, int64_t* idx,
+                            void* workspace, int64_t B, int64_t M, int64_t QS, int64_t N, int64_t K,
                             hipStream_t stream);
-hipError_t knn3_windowed_rows(const float* query, const float* ref, float* dist, int64_t* idx,
-                              void* workspace, int64_t B, int64_t M, int64_t QS, int64_t N,
-                              int64_t K, hipStream_t stream);
 
 namespace {
 
@@ -170,7 +170,7 @@ size_t pointops_fps_query_pipeline_workspace_bytes(int64_t B, int64_t N, int64_t
     if (B <= 0 || N <= 0 || npoint <= 0 || chunk <= 0) return 0;
     return align_up(static_cast<size_t>(B) * sizeof(uint64_t)) +
            align_up(static_cast<size_t>(B * npoint * 3) * sizeof(float)) +
-           pointops_knn3_windowed_workspace_bytes(B, npoint, N);
+           pointops_knn_screen_workspace_bytes(B, N, 3);
 }
 
 hipError_t pointops_fps_query_pipeline_f32(
@@ -209,10 +209,10 @@ hipError_t pointops_fps_query_pipeline_f32(
     err = fps_dense_progress(xyz, samples, B, N, npoint, start_idx, skip_near_origin != 0,
                              progress, 0, chunk, staged, fps_stream);
     if (err != hipSuccess) return err;
-    // kNN's sort of the references needs the cloud only: it runs first on
-    // the query stream, beside FPS.
+    // kNN's fragments of the references need the cloud only: they are made
+    // first on the query stream, beside FPS.
     if (knn_k > 0) {
-        err = knn3_window_sort(xyz, knn_ws, B, npoint, N, query_stream);
+        err = knn3_screen_prepare(xyz, knn_ws, B, N, query_stream);
         if (err != hipSuccess) return err;
     }
     for (int64_t c = 0; c < chunks; ++c) {
@@ -239,8 +239,8 @@ hipError_t pointops_fps_query_pipeline_f32(
         }
     }
     if (knn_k > 0) {  // after the last gate: every centre is in place
-        err = knn3_windowed_rows(centres, xyz, knn_dist, knn_idx, knn_ws, B, npoint, npoint, N,
-                                 knn_k, query_stream);
+        err = knn3_screen_rows(centres, xyz, knn_dist, knn_idx, knn_ws, B, npoint, npoint, N, knn_k,
+                               query_stream);
         if (err != hipSuccess) return err;
     }
     // Work queued on fps_stream after this call sees every output.

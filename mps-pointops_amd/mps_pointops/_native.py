@@ -37,6 +37,8 @@ _SIGNATURES: dict[str, list] = {
     "pointops_knn3_grid": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp],
     "pointops_knn3_windowed": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp],
     "pointops_knn_feat": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _vp],
+    "pointops_knn_screen": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _vp],
+    "pointops_knn_flat_screen": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _vp],
     "pointops_knn_flat": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp],
     "pointops_ball_query_f32": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _f32, _vp],
     "pointops_ball_query_multi_f32": [_vp, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp],
@@ -75,6 +77,8 @@ _SIZE_QUERIES: dict[str, list] = {
     "pointops_fps_flat_scratch_bytes": [_i64, _i64],
     "pointops_knn3_grid_workspace_bytes": [_i64, _i64, _i64],
     "pointops_knn3_windowed_workspace_bytes": [_i64, _i64, _i64],
+    "pointops_knn_screen_workspace_bytes": [_i64, _i64, _i64],
+    "pointops_knn_flat_screen_workspace_bytes": [_i64, _i64, _i64],
     "pointops_three_interpolate_backward_workspace_bytes": [_i64, _i64, _i64],
     "pointops_ball_query_grid_workspace_bytes": [_i64, _i64, _i64],
     "pointops_ball_query_backward_workspace_bytes": [_i64, _i64],

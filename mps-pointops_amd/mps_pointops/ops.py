@@ -34,14 +34,33 @@ _KNN_GRID_MAX_K = 32
 _KNN_GRID_MIN_N = 32_768
 _KNN_GRID_MIN_PAIRS = 1 << 26
 # 3-D kNN with at most 32 neighbours over clouds of 2048 to 8192 references
-# (and at most 16384 queries per cloud) first sorts each cloud by Morton cell
-# and starts every query from a limit set by its neighbours in that order
-# (pointops_knn3_windowed): same results, about 15% faster at config 2's
-# shape; below 2048 references the extra launch does not pay.
+# (and at most 16384 queries per cloud) goes to pointops_knn3_windowed: same
+# results; below 2048 references the launch that prepares them does not pay.
 _KNN_WINDOW_MAX_K = 32
 _KNN_WINDOW_MIN_N = 2048
 _KNN_WINDOW_MAX_N = 8192
 _KNN_WINDOW_MAX_M = 16384
+# Other searches of at most 128 dimensions and 64 neighbours are screened on
+# the matrix cores (pointops_knn_screen), same results, from the sizes at which
+# that pays for its two launches (_screened below).
+_KNN_SCREEN_MAX_D = 128
+_KNN_SCREEN_MAX_K = 64
+_KNN_SCREEN_MIN_PAIRS = 1 << 20
+
+
+def _screened(B: int, M: int, N: int, D: int, k: int) -> bool:
+    """Whether a dense search takes the screened entry point with its own
+    workspace.  D = 3 does where neither the windowed entry nor pointops_knn3
+    (which screens clouds of up to 16384 references without one) serves it
+    better.  Other D, measured against the scan: 2 x 512 x 512 (D = 33, k = 10)
+    39 against 35 us, 8 x 256 x 256 (D = 68, k = 20) 38 against 28, 8 x 600 x
+    600 (D = 40, k = 20) 44 against 53, 4 x 1000 x 1000 (D = 100, k = 40) 79
+    against 129."""
+    if D > _KNN_SCREEN_MAX_D or k > _KNN_SCREEN_MAX_K:
+        return False
+    if D == 3:
+        return N >= _KNN_WINDOW_MIN_N
+    return B * M * N >= _KNN_SCREEN_MIN_PAIRS
 
 
 def _check_large_status(workspace: Tensor) -> None:
@@ -171,6 +190,11 @@ def knn(query: Tensor, ref: Tensor, k: int) -> tuple[Tensor, Tensor]:
         workspace = torch.empty(size, dtype=torch.uint8, device=query.device)
         _native.call("pointops_knn3_windowed", query.data_ptr(), ref.data_ptr(), dist.data_ptr(),
                      idx.data_ptr(), workspace.data_ptr(), B, M, N, k, stream)
+    elif _screened(B, M, N, D, k):
+        size = _native.size_query("pointops_knn_screen_workspace_bytes", B, N, D)
+        workspace = torch.empty(size, dtype=torch.uint8, device=query.device)
+        _native.call("pointops_knn_screen", query.data_ptr(), ref.data_ptr(), dist.data_ptr(),
+                     idx.data_ptr(), workspace.data_ptr(), B, M, N, D, k, stream)
     elif D == 3:
         _native.call("pointops_knn3", query.data_ptr(), ref.data_ptr(), dist.data_ptr(),
                      idx.data_ptr(), B, M, N, k, stream)
