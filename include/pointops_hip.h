@@ -170,6 +170,29 @@ hipError_t pointops_knn_flat_screen(const float *y, const float *x, const int64_
                                     int64_t total_x, int64_t batch, int64_t D, int64_t K,
                                     hipStream_t stream);
 
+/* The finish of a flat 3-D kNN (pointcept.py:150-172): int32 indices and
+ * Euclidean distances, (M,K), of the int64 rows idx (into x, -1 missing);
+ * distances are recomputed in the searches' order of operations, and a
+ * neighbour whose squared distance is not below `ceiling` is missing: -1 and
+ * `pad`. */
+hipError_t pointops_knn_finish(const float *y, const float *x, const int64_t *idx, int32_t *out,
+                               float *dist, int64_t M, int64_t K, float ceiling, float pad,
+                               hipStream_t stream);
+
+/* Row-major grouping (pointcept.py:175-210): out (M,K,W) holds feat's rows
+ * (N,C) at idx (M,K; int32 or int64, -1 gives zeros), W = C; with xyz (N,3)
+ * and centres (M,3) set, W = 3 + C and xyz[idx] - centre comes first.  The
+ * backward ADDS g (M,K,W) into grad_feat (N,C) and grad_xyz (N,3) with float
+ * atomics (the caller zero-fills them) and writes grad_centres (M,3), minus
+ * each query's sum; NULL outputs are skipped. */
+hipError_t pointops_group_rows(const float *feat, const float *xyz, const float *centres,
+                               const void *idx, int32_t idx_bits, float *out, int64_t M, int64_t K,
+                               int64_t C, hipStream_t stream);
+hipError_t pointops_group_rows_backward(const float *g, const void *idx, int32_t idx_bits,
+                                        float *grad_feat, float *grad_xyz, float *grad_centres,
+                                        int64_t M, int64_t K, int64_t C, int32_t with_xyz,
+                                        hipStream_t stream);
+
 /* ----------------------------------------------------------- ball query */
 
 /* Dense first-K ball query (PyTorch3D convention).  Replaces

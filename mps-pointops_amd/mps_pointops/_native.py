@@ -63,6 +63,9 @@ _SIGNATURES: dict[str, list] = {
     "pointops_group_points": [_vp, _vp, _i32, _vp, _i64, _i64, _i64, _i64, _vp],
     "pointops_group_points_backward": [_vp, _i64, _vp, _i32, _vp, _vp, _i64, _i64, _i64, _i64, _vp],
     "pointops_group_points_rel": [_vp, _vp, _vp, _vp, _i32, _vp, _i64, _i64, _i64, _i64, _i64, _vp],
+    "pointops_knn_finish": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _f32, _f32, _vp],
+    "pointops_group_rows": [_vp, _vp, _vp, _vp, _i32, _vp, _i64, _i64, _i64, _vp],
+    "pointops_group_rows_backward": [_vp, _vp, _i32, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp],
     "pointops_chamfer_nearest_f32": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i32, _vp],
     "pointops_chamfer_nearest_f64": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i32, _vp],
     "pointops_chamfer_backward_f32": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i32, _vp],

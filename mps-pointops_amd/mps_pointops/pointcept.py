@@ -76,6 +76,86 @@ def _gather_rows(table: Tensor, idx: Tensor) -> Tensor:
     return rows.where((idx >= 0)[..., None], 0.0)
 
 
+def _zeros_unless(t: Tensor | None, shape, like: Tensor) -> Tensor:
+    return torch.zeros(shape, dtype=like.dtype, device=like.device) if t is None else t
+
+
+class _GroupRows(torch.autograd.Function):
+    """(M, K, C) rows of ``feat`` at ``idx``, after the positions relative to
+    ``centres`` where ``xyz`` is given, in one launch.  Linear in all three;
+    the adjoint is _ScatterRows, so gradients of any order exist."""
+
+    @staticmethod
+    def forward(ctx, feat, xyz, centres, idx):
+        M, K = idx.shape
+        C = feat.shape[1]
+        out = torch.empty((M, K, C + (0 if xyz is None else 3)), dtype=feat.dtype,
+                          device=feat.device)
+        feat = feat.contiguous()
+        xyz = None if xyz is None else xyz.contiguous()
+        centres = None if centres is None else centres.contiguous()
+        _native.call("pointops_group_rows", feat.data_ptr(), _native.ptr(xyz),
+                     _native.ptr(centres), idx.data_ptr(), 8 * idx.element_size(), out.data_ptr(),
+                     M, K, C, _native.stream(feat.device))
+        ctx.save_for_backward(idx)
+        ctx.rows, ctx.with_xyz = len(feat), xyz is not None
+        return out
+
+    @staticmethod
+    def backward(ctx, grad):
+        (idx,) = ctx.saved_tensors
+        want = ctx.needs_input_grad[:3]
+        if grad is None or not any(want):
+            return None, None, None, None
+        grads = _ScatterRows.apply(grad, idx, ctx.rows, ctx.with_xyz, want)
+        return (*(g if w else None for g, w in zip(grads, want)), None)
+
+
+class _ScatterRows(torch.autograd.Function):
+    """The adjoint of _GroupRows: (feat, xyz, centres) gradients of (M, K, W)
+    rows, an empty tensor for each that ``want`` leaves out."""
+
+    @staticmethod
+    def forward(ctx, grad, idx, rows, with_xyz, want):
+        M, K, W = grad.shape
+        C = W - (3 if with_xyz else 0)
+        grad = grad.contiguous()
+        feat = grad.new_zeros((rows, C) if want[0] else 0)
+        xyz = grad.new_zeros((rows, 3) if want[1] else 0)
+        centres = grad.new_empty((M, 3) if want[2] else 0)
+        _native.call("pointops_group_rows_backward", grad.data_ptr(), idx.data_ptr(),
+                     8 * idx.element_size(), feat.data_ptr() if want[0] and C else None,
+                     xyz.data_ptr() if want[1] else None, centres.data_ptr() if want[2] else None,
+                     M, K, C, int(with_xyz), _native.stream(grad.device))
+        ctx.save_for_backward(idx)
+        ctx.rows, ctx.with_xyz, ctx.want, ctx.width = rows, with_xyz, want, C
+        return feat, xyz, centres
+
+    @staticmethod
+    def backward(ctx, feat, xyz, centres):
+        if not ctx.needs_input_grad[0]:
+            return None, None, None, None, None
+        (idx,) = ctx.saved_tensors
+        like = next(t for t in (feat, xyz, centres) if t is not None)
+        feat = _zeros_unless(feat if ctx.want[0] else None, (ctx.rows, ctx.width), like)
+        if ctx.with_xyz:
+            xyz = _zeros_unless(xyz if ctx.want[1] else None, (ctx.rows, 3), like)
+            centres = _zeros_unless(centres if ctx.want[2] else None, (len(idx), 3), like)
+        else:
+            xyz = centres = None
+        return _GroupRows.apply(feat, xyz, centres, idx), None, None, None, None
+
+
+def _native_rows(*tensors: Tensor) -> bool:
+    """Whether the row kernels serve these inputs: float32 on one GPU, outside
+    function transforms and forward-mode differentiation (which go through the
+    tensor operations)."""
+    return (all(t.device.type == "cuda" and t.dtype == torch.float32 for t in tensors)
+            and len({t.device for t in tensors}) == 1
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and torch.autograd.forward_ad._current_level < 0)
+
+
 def farthest_point_sampling(xyz: Tensor, offset: Tensor, new_offset: Tensor) -> Tensor:
     """Global int32 FPS indices, starting at each batch's first point
     (pointcept.py:80-104): one ragged launch for every batch."""
@@ -129,14 +209,12 @@ def knn_query(nsample: int, xyz: Tensor, offset: Tensor, new_xyz: Tensor | None 
         idx = flat.knn_indices(x, y, ptr_x, ptr_y, nsample)
         # The ceiling is applied to the squared distance recomputed from the
         # selected coordinates, in the kernels' order ((dx^2 + dy^2) + dz^2).
-        valid = idx >= 0
-        delta = y[:, None, :] - x[torch.where(valid, idx, 0)]
-        squared = delta[..., 0] * delta[..., 0]
-        squared = squared + delta[..., 1] * delta[..., 1]
-        squared = squared + delta[..., 2] * delta[..., 2]
-        valid = valid & (squared < _PAD_SQUARED_DISTANCE)
-        dist = torch.where(valid, torch.sqrt(squared), _PAD_DISTANCE)
-        return torch.where(valid, idx, -1).to(torch.int32), dist
+        neighbours = torch.empty((M, nsample), dtype=torch.int32, device=x.device)
+        dist = torch.empty((M, nsample), dtype=torch.float32, device=x.device)
+        _native.call("pointops_knn_finish", y.data_ptr(), x.data_ptr(), idx.data_ptr(),
+                     neighbours.data_ptr(), dist.data_ptr(), M, nsample, _PAD_SQUARED_DISTANCE,
+                     _PAD_DISTANCE, _native.stream(x.device))
+        return neighbours, dist
 
 
 def grouping(idx: Tensor, feat: Tensor, xyz: Tensor, new_xyz: Tensor | None = None,
@@ -153,13 +231,23 @@ def grouping(idx: Tensor, feat: Tensor, xyz: Tensor, new_xyz: Tensor | None = No
         raise ValueError("idx must be on the xyz device")
     if bool(((idx < -1) | (idx >= len(xyz))).any().item()):
         raise ValueError("idx contains an out-of-range point index")
-    grouped = _gather_rows(feat, idx)
+    return _grouped(idx, feat, xyz, new_xyz, with_xyz)
+
+
+def _grouped(idx: Tensor, feat: Tensor, xyz: Tensor, new_xyz: Tensor | None,
+             with_xyz: bool) -> Tensor:
+    """grouping for indices that are known to be in range."""
     if not with_xyz:
-        return grouped
+        if len(feat) and _native_rows(feat):
+            return _GroupRows.apply(feat, None, None, idx.contiguous())
+        return _gather_rows(feat, idx)
     centres = xyz if new_xyz is None else new_xyz
     _points(centres, "new_xyz")
     if centres.device != xyz.device or len(centres) != len(idx):
         raise ValueError("new_xyz must have one row per idx row on the xyz device")
+    if len(feat) and _native_rows(feat, xyz, centres):
+        return _GroupRows.apply(feat, xyz, centres, idx.contiguous())
+    grouped = _gather_rows(feat, idx)
     relative = (_gather_rows(xyz, idx) - centres[:, None, :]).where((idx >= 0)[..., None], 0.0)
     return torch.cat((relative, grouped), dim=-1)
 
@@ -173,6 +261,8 @@ def knn_query_and_group(feat: Tensor, xyz: Tensor, offset: Tensor | None = None,
         if offset is None or nsample is None:
             raise ValueError("offset and nsample are required when idx is absent")
         idx, _ = knn_query(nsample, xyz, offset, new_xyz, new_offset)
+        _check_features(feat, xyz)
+        return _grouped(idx, feat, xyz, new_xyz, with_xyz), idx
     return grouping(idx, feat, xyz, new_xyz, with_xyz), idx
 
 
