@@ -2620,7 +2620,7 @@ size_t fps_scratch_bytes_per_point(int64_t max_len) {
 hipError_t launch_fps(const float* xyz, const int64_t* ptr, const int64_t* out_ptr,
                       const int64_t* starts, int64_t* out, float* scratch, int64_t blocks,
                       int64_t max_len, int64_t N, int64_t npoint, int64_t start, int skip,
-                      hipStream_t stream) {
+                      hipStream_t stream, bool sorted = true) {
     if (max_len <= 1 * kRegsThreads)
         return launch_regs<1>(xyz, ptr, out_ptr, starts, out, blocks, N, npoint, start, skip, stream);
     if (max_len <= 2 * kRegsThreads)
@@ -2636,7 +2636,8 @@ hipError_t launch_fps(const float* xyz, const int64_t* ptr, const int64_t* out_p
     // kWideFew samples and the global kernel the others; a dense launch is all
     // one or all the other, a ragged one may hold both, so it runs both (in
     // turn on the stream: the second may reuse the first's scratch).
-    const bool wide = max_len <= kWideMaxPoints;
+    // (`sorted`: the scratch has room for the wide kernel's points.)
+    const bool wide = sorted && max_len <= kWideMaxPoints;
     if (!wide || ptr != nullptr || npoint <= kWideFew) {
         hipLaunchKernelGGL((fps_global_kernel<kGlobalThreads>), dim3(static_cast<uint32_t>(blocks)),
                            dim3(kGlobalThreads), 0, stream, xyz, ptr, out_ptr, starts, out, scratch,
@@ -2835,12 +2836,28 @@ hipError_t pointops_fps_dense(const float* xyz, int64_t* out, void* scratch, int
 
 size_t pointops_fps_flat_scratch_bytes(int64_t total_n, int64_t max_len) {
     if (max_len <= kRegsMaxPoints || total_n <= 0) return 0;
-    return static_cast<size_t>(total_n) * fps_scratch_bytes_per_point(max_len);
+    return static_cast<size_t>(total_n) * sizeof(float);
 }
 
 hipError_t pointops_fps_flat(const float* x, const int64_t* ptr, const int64_t* out_ptr,
                              const int64_t* starts, int64_t* out, void* scratch, int64_t batch,
                              int64_t total_n, int64_t max_len, hipStream_t stream) {
+    if (batch < 0 || total_n < 0 || max_len < 0 || max_len > INT32_MAX - 1 || batch > INT32_MAX)
+        return hipErrorInvalidValue;
+    if (batch == 0) return hipSuccess;
+    if (ptr == nullptr || out_ptr == nullptr || starts == nullptr) return hipErrorInvalidValue;
+    return launch_fps(x, ptr, out_ptr, starts, out, static_cast<float*>(scratch), batch, max_len, 0,
+                      0, 0, 0, stream, false);
+}
+
+size_t pointops_fps_flat_sorted_scratch_bytes(int64_t total_n, int64_t max_len) {
+    if (max_len <= kRegsMaxPoints || total_n <= 0) return 0;
+    return static_cast<size_t>(total_n) * fps_scratch_bytes_per_point(max_len);
+}
+
+hipError_t pointops_fps_flat_sorted(const float* x, const int64_t* ptr, const int64_t* out_ptr,
+                                    const int64_t* starts, int64_t* out, void* scratch, int64_t batch,
+                                    int64_t total_n, int64_t max_len, hipStream_t stream) {
     if (batch < 0 || total_n < 0 || max_len < 0 || max_len > INT32_MAX - 1 || batch > INT32_MAX)
         return hipErrorInvalidValue;
     if (batch == 0) return hipSuccess;

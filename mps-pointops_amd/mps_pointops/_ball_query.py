@@ -27,22 +27,43 @@ class BallQueryResult(NamedTuple):
     indices: torch.Tensor
 
 
-def _lengths_or_full(
-    lengths: torch.Tensor | None, *, batch: int, count: int, device: torch.device, name: str
-) -> torch.Tensor | None:
-    """_ball_query_mps.py:73-84 (one host sync when lengths are given).
+def _checked_lengths(specs: list[tuple], device: torch.device) -> list[torch.Tensor | None]:
+    """_ball_query_mps.py:73-84 for (lengths, batch, count, name) in turn (one
+    host sync when lengths are given): a lengths' type errors come before its
+    value errors, and both before the next one's.
 
     ``None`` stays ``None``: the kernel then treats every row as valid, which
     saves two fill launches per call."""
-    if lengths is None:
-        return None
-    if not isinstance(lengths, torch.Tensor):
-        raise TypeError(f"{name} must be a torch.Tensor or None")
-    if lengths.shape != (batch,) or lengths.dtype != torch.int64 or lengths.device != device:
-        raise ValueError(f"{name} must have shape ({batch},), int64 dtype and device {device}")
-    if torch.any((lengths < 0) | (lengths > count)).item():
-        raise ValueError(f"{name} values must lie in [0, {count}]")
-    return lengths.contiguous()
+    valid, failure = [], None
+    for lengths, batch, count, name in specs:
+        if lengths is not None:
+            if not isinstance(lengths, torch.Tensor):
+                failure = TypeError(f"{name} must be a torch.Tensor or None")
+            elif (lengths.shape != (batch,) or lengths.dtype != torch.int64
+                  or lengths.device != device):
+                failure = ValueError(
+                    f"{name} must have shape ({batch},), int64 dtype and device {device}")
+        if failure is not None:
+            break
+        valid.append((lengths, count, name))
+    given = [(lengths, count, name) for lengths, count, name in valid if lengths is not None]
+    if given and device.type == "cuda":
+        bad = _native.outside([(lengths, 0, count) for lengths, count, _ in given])
+    else:
+        bad = [torch.any((t < 0) | (t > count)).item() for t, count, _ in given]
+    for wrong, (_, count, name) in zip(bad, given):
+        if wrong:
+            raise ValueError(f"{name} values must lie in [0, {count}]")
+    if failure is not None:
+        raise failure
+    return [None if lengths is None else lengths.contiguous() for lengths, _, _ in valid]
+
+
+def _lengths_or_full(
+    lengths: torch.Tensor | None, *, batch: int, count: int, device: torch.device, name: str
+) -> torch.Tensor | None:
+    """One tensor of lengths, checked (_checked_lengths)."""
+    return _checked_lengths([(lengths, batch, count, name)], device)[0]
 
 
 def _checked_radius_and_k(radius: float, k: int) -> tuple[float, float]:
@@ -197,12 +218,9 @@ def ball_query(
     if point_count > (1 << 31) - 128:
         raise ValueError("point count exceeds the native kernel's 32-bit index range")
     _native.require_device(queries.device)
-    query_lengths = _lengths_or_full(
-        query_lengths, batch=batch, count=query_count, device=queries.device, name="query_lengths"
-    )
-    point_lengths = _lengths_or_full(
-        point_lengths, batch=batch, count=point_count, device=queries.device, name="point_lengths"
-    )
+    query_lengths, point_lengths = _checked_lengths(
+        [(query_lengths, batch, query_count, "query_lengths"),
+         (point_lengths, batch, point_count, "point_lengths")], queries.device)
     distances, indices = _BallQuery.apply(
         queries.contiguous(), points.contiguous(), query_lengths, point_lengths,
         radius_squared, k,

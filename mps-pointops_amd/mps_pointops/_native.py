@@ -33,6 +33,7 @@ _SIGNATURES: dict[str, list] = {
     "pointops_fps_large": [_vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp],
     "pointops_fps_large_noalloc": [_vp, _vp, _i64, _i64, _i64, _i32, _vp],
     "pointops_fps_flat": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp],
+    "pointops_fps_flat_sorted": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp],
     "pointops_knn3": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp],
     "pointops_knn3_grid": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp],
     "pointops_knn3_windowed": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp],
@@ -63,6 +64,12 @@ _SIGNATURES: dict[str, list] = {
     "pointops_group_points": [_vp, _vp, _i32, _vp, _i64, _i64, _i64, _i64, _vp],
     "pointops_group_points_backward": [_vp, _i64, _vp, _i32, _vp, _vp, _i64, _i64, _i64, _i64, _vp],
     "pointops_group_points_rel": [_vp, _vp, _vp, _vp, _i32, _vp, _i64, _i64, _i64, _i64, _i64, _vp],
+    "pointops_check_range": [_vp, _i32, _i64, _i64, _i64, _vp, _vp],
+    "pointops_check_finite": [_vp, _i32, _vp, _i64, _i64, _i64, _vp, _vp],
+    "pointops_segment_check": [_vp, _i32, _i64, _vp, _vp],
+    "pointops_segment_offsets": [_vp, _i32, _i64, _i64, _vp, _vp],
+    "pointops_edge_count": [_vp, _i64, _i64, _i32, _vp, _vp],
+    "pointops_edge_write": [_vp, _vp, _i64, _i64, _i32, _vp, _vp, _vp],
     "pointops_knn_finish": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _f32, _f32, _vp],
     "pointops_group_rows": [_vp, _vp, _vp, _vp, _i32, _vp, _i64, _i64, _i64, _vp],
     "pointops_group_rows_backward": [_vp, _vp, _i32, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp],
@@ -78,6 +85,7 @@ _SIZE_QUERIES: dict[str, list] = {
     "pointops_fps_query_pipeline_workspace_bytes": [_i64, _i64, _i64, _i64],
     "pointops_fps_large_workspace_bytes": [_i64, _i64],
     "pointops_fps_flat_scratch_bytes": [_i64, _i64],
+    "pointops_fps_flat_sorted_scratch_bytes": [_i64, _i64],
     "pointops_knn3_grid_workspace_bytes": [_i64, _i64, _i64],
     "pointops_knn3_windowed_workspace_bytes": [_i64, _i64, _i64],
     "pointops_knn_screen_workspace_bytes": [_i64, _i64, _i64],
@@ -156,6 +164,11 @@ def stream(device: torch.device) -> int:
 
 
 def call(name: str, *args) -> None:
+    """Enqueue an operator's entry point; RuntimeError on a non-zero status."""
+    _enqueue(name, *args)
+
+
+def _enqueue(name: str, *args) -> None:
     status = getattr(library(), name)(*args)
     if status != 0:
         getter = _hip_error_string()
@@ -165,3 +178,29 @@ def call(name: str, *args) -> None:
 
 def size_query(name: str, *args) -> int:
     return int(getattr(library(), name)(*args))
+
+
+def outside(checks: list[tuple[torch.Tensor, int, int]]) -> list[bool]:
+    """For each (int32/int64 tensor, lo, hi), whether any value lies outside
+    [lo, hi]; all on one ROCm device, read with one synchronisation."""
+    device = checks[0][0].device
+    flags = torch.zeros(len(checks), dtype=torch.int32, device=device)
+    for i, (values, lo, hi) in enumerate(checks):
+        values = values.contiguous()
+        _enqueue("pointops_check_range", values.data_ptr(), 8 * values.element_size(), values.numel(),
+                 lo, hi, flags.data_ptr() + 4 * i, stream(device))
+    return [flag != 0 for flag in flags.tolist()]
+
+
+def nonfinite(clouds: list[tuple[torch.Tensor, torch.Tensor | None]]) -> list[bool]:
+    """For each (float32/float64 (B, P, D) points, lengths or None), whether a
+    row below its cloud's length has a coordinate that is not finite; all on
+    one ROCm device, read with one synchronisation."""
+    device = clouds[0][0].device
+    flags = torch.zeros(len(clouds), dtype=torch.int32, device=device)
+    for i, (points, lengths) in enumerate(clouds):
+        points = points.detach().contiguous()
+        lengths = None if lengths is None else lengths.contiguous()
+        _enqueue("pointops_check_finite", points.data_ptr(), 8 * points.element_size(), ptr(lengths),
+                 *points.shape, flags.data_ptr() + 4 * i, stream(device))
+    return [flag != 0 for flag in flags.tolist()]

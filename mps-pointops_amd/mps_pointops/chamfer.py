@@ -195,11 +195,13 @@ def _check_coordinates(x: Tensor, y: Tensor) -> None:
     _native.require_device(x.device)
 
 
-def _check_finite(cloud: _Cloud, name: str) -> None:
-    """Rows inside a cloud's length must be finite (one host read)."""
-    bad = cloud.valid() & ~torch.isfinite(cloud.points).all(dim=-1)
-    if bool(bad.any().item()):
-        raise ValueError(f"valid {name} coordinates must be finite")
+def _check_finite(x: _Cloud, y: _Cloud, full: bool) -> None:
+    """Rows inside a cloud's length must be finite (one host read; ``full``:
+    every row is)."""
+    bad = _native.nonfinite([(c.points, None if full else c.lengths) for c in (x, y)])
+    for wrong, name in zip(bad, ("x", "y")):
+        if wrong:
+            raise ValueError(f"valid {name} coordinates must be finite")
 
 
 def _check_normals(points: Tensor, normals: Tensor | None, name: str) -> None:
@@ -340,9 +342,8 @@ def chamfer_distance(
     _check_coordinates(x_points, y_points)
     cx = _Cloud(x_points, _lengths_for(x_points, x_lengths, "x_lengths"), x_normals)
     cy = _Cloud(y_points, _lengths_for(y_points, y_lengths, "y_lengths"), y_normals)
-    _check_finite(cx, "x")
-    _check_finite(cy, "y")
     full = x_lengths is None and y_lengths is None  # every row of every cloud is valid
+    _check_finite(cx, cy, full)
     if x_points.shape[-1] != 3 and (x_normals is not None or y_normals is not None):
         raise NotImplementedError("normal loss currently requires D == 3")
     _check_normals(x_points, x_normals, "x_normals")

@@ -8,10 +8,10 @@ contiguous runs described by a sorted batch vector (or, for ``fps``, an
 offset array ``ptr``), and every result uses global row indices.  FPS and
 radius take 3-D coordinates; kNN takes any positive dimension.
 
-All clouds of a call go to one ragged launch (``pointops_fps_flat``,
+All clouds of a call go to one ragged launch (``pointops_fps_flat_sorted``,
 ``pointops_knn_flat``, ``pointops_radius_flat_*``).  A batch vector is
 validated with one device-to-host read (first id, sortedness and last id
-together); its offsets are a bincount prefix sum on the device.
+together, several vectors in one read); its offsets come from one launch.
 """
 
 from __future__ import annotations
@@ -76,11 +76,10 @@ def _optional_batch_size(value) -> int | None:
     return None if value is None else _count_arg(value, "batch_size")
 
 
-def _clouds_in(batch, rows: int, device: torch.device, name: str) -> int:
-    """Number of clouds a sorted batch vector names (its last id + 1; 0 for
-    no vector or no rows).  One device-to-host read covers the checks."""
+def _check_batch(batch, rows: int, device: torch.device, name: str) -> None:
+    """A batch vector's type, shape and place (values: _clouds_in)."""
     if batch is None:
-        return 0
+        return
     if not isinstance(batch, Tensor):
         raise TypeError(f"{name} must be a torch.Tensor or None")
     if batch.ndim != 1 or batch.numel() != rows:
@@ -89,14 +88,50 @@ def _clouds_in(batch, rows: int, device: torch.device, name: str) -> int:
         raise ValueError(f"{name} must be on {device}")
     if batch.dtype not in (torch.int32, torch.int64):
         raise TypeError(f"{name} must have an integer dtype (int32 or int64)")
-    if rows == 0:
-        return 0
-    ids = batch.long()
-    first, descending, last = torch.stack(
-        (ids[0], (ids[1:] < ids[:-1]).any().long(), ids[-1])).tolist()
-    if first < 0 or descending:
-        raise ValueError(f"{name} must be sorted with non-negative batch IDs")
-    return last + 1
+
+
+def _ends_of(batches: list[Tensor]) -> list[list[int]]:
+    """(first id, whether any id is below its predecessor, last id) of each
+    non-empty batch vector, in one device-to-host read."""
+    device = batches[0].device
+    if device.type != "cuda":
+        return [[int(ids[0]), int((ids[1:] < ids[:-1]).any()), int(ids[-1])] for ids in batches]
+    ends = torch.zeros((len(batches), 3), dtype=torch.long, device=device)
+    for i, ids in enumerate(batches):
+        ids = ids.contiguous()
+        _native.call("pointops_segment_check", ids.data_ptr(), 8 * ids.element_size(), len(ids),
+                     ends[i].data_ptr(), _native.stream(device))
+    return ends.tolist()
+
+
+def _clouds_in(specs: list[tuple]) -> list[int]:
+    """Numbers of clouds that sorted batch vectors name (each its last id + 1;
+    0 for no vector or no rows), for (batch, rows, device, name) in turn: a
+    vector's type errors come before its value errors, and both before the
+    next vector's."""
+    valid, failure = [], None
+    for spec in specs:
+        try:
+            _check_batch(*spec)
+        except (TypeError, ValueError) as exc:
+            failure = exc
+            break
+        valid.append(spec)
+    named = [batch for batch, rows, _, _ in valid if batch is not None and rows]
+    distinct = [b for i, b in enumerate(named) if all(b is not other for other in named[:i])]
+    ends = _ends_of(distinct) if distinct else []
+    counts = []
+    for batch, rows, _, name in valid:
+        if batch is None or rows == 0:
+            counts.append(0)
+            continue
+        first, descending, last = next(e for b, e in zip(distinct, ends) if b is batch)
+        if first < 0 or descending:
+            raise ValueError(f"{name} must be sorted with non-negative batch IDs")
+        counts.append(last + 1)
+    if failure is not None:
+        raise failure
+    return counts
 
 
 def _offsets(batch: Tensor | None, rows: int, device: torch.device, clouds: int) -> Tensor:
@@ -104,6 +139,12 @@ def _offsets(batch: Tensor | None, rows: int, device: torch.device, clouds: int)
     vector all rows form one cloud (even when there are none)."""
     if batch is None:
         return torch.tensor([0, rows], dtype=torch.long, device=device)
+    if device.type == "cuda":
+        batch = batch.contiguous()
+        offsets = torch.empty(clouds + 1, dtype=torch.long, device=device)
+        _native.call("pointops_segment_offsets", batch.data_ptr(), 8 * batch.element_size(), rows,
+                     clouds, offsets.data_ptr(), _native.stream(device))
+        return offsets
     offsets = torch.zeros(clouds + 1, dtype=torch.long, device=device)
     if clouds:
         offsets[1:] = torch.bincount(batch.long(), minlength=clouds).cumsum(0)
@@ -124,22 +165,23 @@ class _SearchLayout:
     @classmethod
     def of(cls, x: Tensor, y: Tensor, batch_x, batch_y, batch_size) -> "_SearchLayout":
         requested = _optional_batch_size(batch_size)
-        in_x = _clouds_in(batch_x, len(x), x.device, "batch_x")
-        in_y = _clouds_in(batch_y, len(y), y.device, "batch_y")
+        in_x, in_y = _clouds_in([(batch_x, len(x), x.device, "batch_x"),
+                                 (batch_y, len(y), y.device, "batch_y")])
         clouds = max(1, in_x, in_y, requested or 0)
         if clouds > 1 and (batch_x is None or batch_y is None):
             raise ValueError("batch_x and batch_y are both required for multiple batches")
         if requested is not None and requested < max(in_x, in_y):
             raise ValueError("batch_size is smaller than the largest batch ID")
-        return cls(_offsets(batch_x, len(x), x.device, clouds),
-                   _offsets(batch_y, len(y), y.device, clouds))
+        x_offsets = _offsets(batch_x, len(x), x.device, clouds)
+        same = batch_x is batch_y and len(x) == len(y)
+        return cls(x_offsets, x_offsets if same else _offsets(batch_y, len(y), y.device, clouds))
 
 
 def _fps_offsets(x: Tensor, batch, batch_size, ptr) -> Tensor:
     """Cloud offsets for fps: an explicit ``ptr`` wins over ``batch``."""
     if ptr is None:
         requested = _optional_batch_size(batch_size)
-        named = _clouds_in(batch, len(x), x.device, "batch")
+        (named,) = _clouds_in([(batch, len(x), x.device, "batch")])
         if requested is not None and requested < named:
             raise ValueError("batch_size is smaller than the largest batch ID")
         clouds = max(named, requested or 0)
@@ -242,9 +284,9 @@ def fps(
     points = x.contiguous()
     out = torch.empty(total, dtype=torch.long, device=x.device)
     out_ptr = torch.tensor(out_bounds, dtype=torch.long, device=x.device)
-    scratch_bytes = _native.size_query("pointops_fps_flat_scratch_bytes", len(points), longest)
+    scratch_bytes = _native.size_query("pointops_fps_flat_sorted_scratch_bytes", len(points), longest)
     scratch = torch.empty(scratch_bytes, dtype=torch.uint8, device=x.device) if scratch_bytes else None
-    _native.call("pointops_fps_flat", points.data_ptr(), offsets.data_ptr(), out_ptr.data_ptr(),
+    _native.call("pointops_fps_flat_sorted", points.data_ptr(), offsets.data_ptr(), out_ptr.data_ptr(),
                  starts.contiguous().data_ptr(), out.data_ptr(), _native.ptr(scratch),
                  len(lengths), len(points), longest, _native.stream(x.device))
     return out
@@ -264,11 +306,23 @@ def _search_pair(x, y, *, coordinates: bool) -> None:
         raise TypeError(f"x and y must have the same dtype, got {x.dtype} and {y.dtype}")
 
 
-def _edge_index(table: Tensor) -> Tensor:
+def _edge_index(table: Tensor, skip_self: bool = False, flip: bool = False) -> Tensor:
     """[2, E] (query row, reference row) pairs of a -1 padded (Q, K) table,
-    row-major."""
-    queries, slots = torch.nonzero(table >= 0, as_tuple=True)
-    return torch.stack((queries, table[queries, slots]))
+    row-major; without the pairs of equal rows where ``skip_self``, the
+    reference first where ``flip``."""
+    Q, K = table.shape
+    if Q == 0 or K == 0:
+        return torch.empty((2, 0), dtype=torch.long, device=table.device)
+    stream = _native.stream(table.device)
+    counts = torch.empty(Q, dtype=torch.long, device=table.device)
+    _native.call("pointops_edge_count", table.data_ptr(), Q, K, int(skip_self), counts.data_ptr(),
+                 stream)
+    ends = counts.cumsum(0)
+    edges = torch.empty((2, int(ends[-1].item())), dtype=torch.long, device=table.device)
+    queries, references = (edges[1], edges[0]) if flip else (edges[0], edges[1])
+    _native.call("pointops_edge_write", table.data_ptr(), ends.data_ptr(), Q, K, int(skip_self),
+                 queries.data_ptr(), references.data_ptr(), stream)
+    return edges
 
 
 def knn_indices(x: Tensor, y: Tensor, ptr_x: Tensor, ptr_y: Tensor, k: int) -> Tensor:
@@ -327,6 +381,11 @@ def knn(
     each query within its cloud (flat.py:291-329).  ``min(k, len(x))`` must
     be at most 256; ``cosine=True`` is not implemented; ``num_workers`` has
     no effect."""
+    return _knn_edges(x, y, k, batch_x, batch_y, cosine, num_workers, batch_size)
+
+
+def _knn_edges(x, y, k, batch_x, batch_y, cosine, num_workers, batch_size, skip_self=False,
+               flip=False) -> Tensor:
     _search_pair(x, y, coordinates=False)
     k = _count_arg(k, "k")
     if cosine:
@@ -342,7 +401,7 @@ def knn(
     if width > _KNN_MAX_K:
         raise ValueError(f"effective k must be at most {_KNN_MAX_K} on ROCm, got {width}")
     table = knn_indices(x.contiguous(), y.contiguous(), layout.x_offsets, layout.y_offsets, width)
-    return _edge_index(table)
+    return _edge_index(table, skip_self, flip)
 
 
 def radius(
@@ -360,6 +419,12 @@ def radius(
     query's cloud, in index order, with squared distance below ``r**2``
     (flat.py:332-373); at most ``max_num_neighbors`` per query.
     ``ignore_same_index=True`` is not implemented, as in the reference."""
+    return _radius_edges(x, y, r, batch_x, batch_y, max_num_neighbors, num_workers, batch_size,
+                         ignore_same_index)
+
+
+def _radius_edges(x, y, r, batch_x, batch_y, max_num_neighbors, num_workers, batch_size,
+                  ignore_same_index=False, skip_self=False, flip=False) -> Tensor:
     _search_pair(x, y, coordinates=True)
     limit = _count_arg(max_num_neighbors, "max_num_neighbors")
     _count_arg(num_workers, "num_workers")
@@ -376,7 +441,7 @@ def radius(
     layout = _SearchLayout.of(x, y, batch_x, batch_y, batch_size)
     table = radius_indices(x.contiguous(), y.contiguous(), layout.x_offsets, layout.y_offsets,
                            float(r), min(limit, len(x)))
-    return _edge_index(table)
+    return _edge_index(table, skip_self, flip)
 
 
 # --------------------------------------------------------------- graphs
@@ -385,15 +450,6 @@ def radius(
 def _check_flow(flow: str) -> None:
     if flow not in _FLOWS:
         raise ValueError("flow must be 'source_to_target' or 'target_to_source'")
-
-
-def _as_graph(edges: Tensor, loop: bool, flow: str) -> Tensor:
-    """torch_cluster 1.6.3 orientation of self-search edges: (source,
-    target) rows, reference first for ``source_to_target``; without ``loop``
-    the edges from a point to itself are dropped."""
-    if not loop:
-        edges = edges[:, edges[0] != edges[1]]
-    return edges.flip(0) if flow == "source_to_target" else edges
 
 
 def knn_graph(
@@ -407,12 +463,12 @@ def knn_graph(
     batch_size: int | None = None,
 ) -> Tensor:
     """kNN graph of ``x`` (flat.py:386-404): ``k + 1`` neighbours are searched
-    when self loops are removed."""
+    when self loops are removed.  torch_cluster 1.6.3 orientation: (source,
+    target) rows, reference first for ``source_to_target``."""
     k = _count_arg(k, "k")
     _check_flow(flow)
-    edges = knn(x, x, k if loop else k + 1, batch, batch, cosine=cosine,
-                num_workers=num_workers, batch_size=batch_size)
-    return _as_graph(edges, loop, flow)
+    return _knn_edges(x, x, k if loop else k + 1, batch, batch, cosine, num_workers, batch_size,
+                      skip_self=not loop, flip=flow == "source_to_target")
 
 
 def radius_graph(
@@ -429,9 +485,8 @@ def radius_graph(
     candidates when self loops are removed."""
     limit = _count_arg(max_num_neighbors, "max_num_neighbors")
     _check_flow(flow)
-    edges = radius(x, x, r, batch, batch, limit if loop else limit + 1,
-                   num_workers=num_workers, batch_size=batch_size)
-    return _as_graph(edges, loop, flow)
+    return _radius_edges(x, x, r, batch, batch, limit if loop else limit + 1, num_workers,
+                         batch_size, skip_self=not loop, flip=flow == "source_to_target")
 
 
 __all__ = ["fps", "knn", "radius", "knn_graph", "radius_graph"]

@@ -41,7 +41,13 @@ def _index_arg(idx: Tensor) -> tuple[Tensor, int]:
 
 def _check_range(idx: Tensor, n: int) -> None:
     """torch.gather's index rule (one device-to-host sync)."""
-    if idx.numel() and torch.any((idx < 0) | (idx >= n)).item():
+    if not idx.numel():
+        return
+    if idx.device.type == "cuda" and idx.dtype in (torch.int32, torch.int64):
+        bad = _native.outside([(idx, 0, n - 1)])[0]
+    else:
+        bad = torch.any((idx < 0) | (idx >= n)).item()
+    if bad:
         raise IndexError(f"indices must lie in [0, {n})")
 
 

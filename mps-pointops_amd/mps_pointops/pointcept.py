@@ -177,9 +177,9 @@ def farthest_point_sampling(xyz: Tensor, offset: Tensor, new_offset: Tensor) -> 
     starts = torch.zeros(len(lengths), dtype=torch.long, device=x.device)
     out = torch.empty(target[-1], dtype=torch.long, device=x.device)
     max_len = max(lengths)
-    size = _native.size_query("pointops_fps_flat_scratch_bytes", len(x), max_len)
+    size = _native.size_query("pointops_fps_flat_sorted_scratch_bytes", len(x), max_len)
     scratch = torch.empty(size, dtype=torch.uint8, device=x.device) if size else None
-    _native.call("pointops_fps_flat", x.data_ptr(), ptr.data_ptr(), out_ptr.data_ptr(),
+    _native.call("pointops_fps_flat_sorted", x.data_ptr(), ptr.data_ptr(), out_ptr.data_ptr(),
                  starts.data_ptr(), out.data_ptr(), _native.ptr(scratch), len(lengths), len(x),
                  max_len, _native.stream(x.device))
     return out.to(torch.int32)
@@ -229,7 +229,11 @@ def grouping(idx: Tensor, feat: Tensor, xyz: Tensor, new_xyz: Tensor | None = No
         raise ValueError("idx must be a two-dimensional int32/int64 tensor")
     if idx.device != xyz.device:
         raise ValueError("idx must be on the xyz device")
-    if bool(((idx < -1) | (idx >= len(xyz))).any().item()):
+    if idx.device.type == "cuda" and torch._C._functorch.peek_interpreter_stack() is None:
+        bad = _native.outside([(idx, -1, len(xyz) - 1)])[0]
+    else:
+        bad = bool(((idx < -1) | (idx >= len(xyz))).any().item())
+    if bad:
         raise ValueError("idx contains an out-of-range point index")
     return _grouped(idx, feat, xyz, new_xyz, with_xyz)
 

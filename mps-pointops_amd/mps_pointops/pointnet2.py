@@ -61,6 +61,12 @@ def three_nn(unknown: Tensor, known: Tensor) -> tuple[Tensor, Tensor]:
     return distances, indices
 
 
+def _out_of_range(indices: Tensor, points: int) -> bool:
+    if indices.device.type == "cuda":
+        return _native.outside([(indices, 0, points - 1)])[0]
+    return bool(torch.any((indices < 0) | (indices >= points)).item())
+
+
 def _validate_interpolate(features: Tensor, indices: Tensor, weights: Tensor):
     """pointnet2.py:103-132 (one device-to-host sync for the index bounds)."""
     if not all(isinstance(t, Tensor) for t in (features, indices, weights)):
@@ -87,7 +93,7 @@ def _validate_interpolate(features: Tensor, indices: Tensor, weights: Tensor):
         raise ValueError("three_interpolate supports at most 2**31-1 source points")
     if batch * channels * queries > (1 << 32) - 1:
         raise ValueError("three_interpolate output exceeds the native index range")
-    if indices.numel() and torch.any((indices < 0) | (indices >= points)).item():
+    if indices.numel() and _out_of_range(indices, points):
         raise IndexError(f"indices must lie in [0, {points})")
     return batch, channels, points, queries
 
