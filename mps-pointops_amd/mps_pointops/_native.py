@@ -180,10 +180,27 @@ def size_query(name: str, *args) -> int:
     return int(getattr(library(), name)(*args))
 
 
+def plain(*tensors: torch.Tensor) -> bool:
+    """Whether kernels on raw pointers may stand in for tensor operations on
+    these: no subclasses and no batched gradients (which may hold no memory of
+    their own; a backward's thread does not see the transform), and outside
+    function transforms, forward-mode differentiation, tracing, compilation and
+    dispatch modes, all of which see tensor operations only."""
+    return (all(type(t) in (torch.Tensor, torch.nn.Parameter) and torch._C._has_storage(t)
+                for t in tensors)
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and torch.autograd.forward_ad._current_level < 0
+            and torch._C._len_torch_dispatch_stack() == 0
+            and not torch.jit.is_tracing()
+            and not torch.compiler.is_compiling())
+
+
 def outside(checks: list[tuple[torch.Tensor, int, int]]) -> list[bool]:
     """For each (int32/int64 tensor, lo, hi), whether any value lies outside
     [lo, hi]; all on one ROCm device, read with one synchronisation."""
     device = checks[0][0].device
+    if not plain(*(values for values, _, _ in checks)):
+        return [bool(((v < lo) | (v > hi)).any().item()) for v, lo, hi in checks]
     flags = torch.zeros(len(checks), dtype=torch.int32, device=device)
     for i, (values, lo, hi) in enumerate(checks):
         values = values.contiguous()

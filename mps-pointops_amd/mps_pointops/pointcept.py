@@ -80,6 +80,32 @@ def _zeros_unless(t: Tensor | None, shape, like: Tensor) -> Tensor:
     return torch.zeros(shape, dtype=like.dtype, device=like.device) if t is None else t
 
 
+def _group_rows(feat: Tensor, xyz: Tensor | None, centres: Tensor | None, idx: Tensor) -> Tensor:
+    """What _GroupRows computes, as tensor operations."""
+    grouped = _gather_rows(feat, idx)
+    if xyz is None:
+        return grouped
+    relative = (_gather_rows(xyz, idx) - centres[:, None, :]).where((idx >= 0)[..., None], 0.0)
+    return torch.cat((relative, grouped), dim=-1)
+
+
+def _scatter_rows(grad: Tensor, idx: Tensor, rows: int, with_xyz: bool, want) -> list:
+    """What _ScatterRows computes, as tensor operations (batched gradients:
+    a vectorised Jacobian's backward runs under a function transform); None
+    for each gradient that ``want`` leaves out."""
+    grad = grad.where((idx >= 0)[..., None], 0.0)
+    at = idx.clamp_min(0).reshape(-1)
+    off = 3 if with_xyz else 0
+
+    def added(part: Tensor) -> Tensor:
+        width = part.shape[-1]
+        return part.new_zeros((rows, width)).index_add(0, at, part.reshape(-1, width))
+
+    return [added(grad[..., off:]) if want[0] else None,
+            added(grad[..., :off]) if want[1] else None,
+            -grad[..., :off].sum(dim=1) if want[2] else None]
+
+
 class _GroupRows(torch.autograd.Function):
     """(M, K, C) rows of ``feat`` at ``idx``, after the positions relative to
     ``centres`` where ``xyz`` is given, in one launch.  Linear in all three;
@@ -107,6 +133,8 @@ class _GroupRows(torch.autograd.Function):
         want = ctx.needs_input_grad[:3]
         if grad is None or not any(want):
             return None, None, None, None
+        if not _native.plain(grad):
+            return (*_scatter_rows(grad, idx, ctx.rows, ctx.with_xyz, want), None)
         grads = _ScatterRows.apply(grad, idx, ctx.rows, ctx.with_xyz, want)
         return (*(g if w else None for g, w in zip(grads, want)), None)
 
@@ -143,17 +171,18 @@ class _ScatterRows(torch.autograd.Function):
             centres = _zeros_unless(centres if ctx.want[2] else None, (len(idx), 3), like)
         else:
             xyz = centres = None
+        if not _native.plain(*(t for t in (feat, xyz, centres) if t is not None)):
+            return _group_rows(feat, xyz, centres, idx), None, None, None, None
         return _GroupRows.apply(feat, xyz, centres, idx), None, None, None, None
 
 
 def _native_rows(*tensors: Tensor) -> bool:
-    """Whether the row kernels serve these inputs: float32 on one GPU, outside
-    function transforms and forward-mode differentiation (which go through the
-    tensor operations)."""
+    """Whether the row kernels serve these inputs: float32 on one GPU, where
+    raw pointers may stand for them; anything else goes through the tensor
+    operations."""
     return (all(t.device.type == "cuda" and t.dtype == torch.float32 for t in tensors)
             and len({t.device for t in tensors}) == 1
-            and torch._C._functorch.peek_interpreter_stack() is None
-            and torch.autograd.forward_ad._current_level < 0)
+            and _native.plain(*tensors))
 
 
 def farthest_point_sampling(xyz: Tensor, offset: Tensor, new_offset: Tensor) -> Tensor:
@@ -229,7 +258,7 @@ def grouping(idx: Tensor, feat: Tensor, xyz: Tensor, new_xyz: Tensor | None = No
         raise ValueError("idx must be a two-dimensional int32/int64 tensor")
     if idx.device != xyz.device:
         raise ValueError("idx must be on the xyz device")
-    if idx.device.type == "cuda" and torch._C._functorch.peek_interpreter_stack() is None:
+    if idx.device.type == "cuda":
         bad = _native.outside([(idx, -1, len(xyz) - 1)])[0]
     else:
         bad = bool(((idx < -1) | (idx >= len(xyz))).any().item())
@@ -251,9 +280,7 @@ def _grouped(idx: Tensor, feat: Tensor, xyz: Tensor, new_xyz: Tensor | None,
         raise ValueError("new_xyz must have one row per idx row on the xyz device")
     if len(feat) and _native_rows(feat, xyz, centres):
         return _GroupRows.apply(feat, xyz, centres, idx.contiguous())
-    grouped = _gather_rows(feat, idx)
-    relative = (_gather_rows(xyz, idx) - centres[:, None, :]).where((idx >= 0)[..., None], 0.0)
-    return torch.cat((relative, grouped), dim=-1)
+    return _group_rows(feat, xyz, centres, idx)
 
 
 def knn_query_and_group(feat: Tensor, xyz: Tensor, offset: Tensor | None = None,

@@ -63,7 +63,37 @@ def test_forward_mode_and_vmap_take_the_tensor_operations(cuda_device):
     f = feat.clone().requires_grad_()
     out = pointcept.grouping(idx, f, xyz, new, True)
     each = torch.stack([torch.autograd.grad(out, f, g, retain_graph=True)[0] for g in many])
-    assert each.shape == (5, 3, 4)
+    batched = torch.autograd.grad(out, f, many, is_grads_batched=True)[0]
+    torch.testing.assert_close(batched, each, rtol=1e-5, atol=1e-5)  # sums of at most 4 terms
+
+
+def test_batched_second_gradients_match_one_at_a_time(cuda_device):
+    from mps_pointops import pointcept
+
+    idx = torch.tensor([[0, -1], [1, 1], [2, 0]], device="cuda")
+    inputs = [torch.randn(3, c, device="cuda").requires_grad_() for c in (4, 3)]
+    out = pointcept.grouping(idx, *inputs, None, True)
+    weight = torch.randn_like(out).requires_grad_()
+    first = torch.autograd.grad((out * weight).sum(), inputs, create_graph=True)
+    many = [torch.randn(5, *t.shape, device="cuda") for t in first]
+    batched = torch.autograd.grad(first, weight, many, retain_graph=True, is_grads_batched=True)[0]
+    for i in range(5):
+        one = torch.autograd.grad(first, weight, [m[i] for m in many], retain_graph=True)[0]
+        torch.testing.assert_close(batched[i], one, rtol=1e-6, atol=1e-6)
+
+
+def test_a_trace_and_a_subclass_keep_the_tensor_operations(cuda_device):
+    from mps_pointops import pointcept
+
+    class Marked(torch.Tensor):
+        pass
+
+    idx = torch.tensor([[0, -1], [1, 1], [2, 0]], device="cuda")
+    feat, other = torch.randn(3, 4, device="cuda"), torch.randn(3, 4, device="cuda")
+    xyz = torch.randn(3, 3, device="cuda")
+    traced = torch.jit.trace(lambda f, x: pointcept.grouping(idx, f, x, None, True), (feat, xyz))
+    assert torch.equal(traced(other, xyz), pointcept.grouping(idx, other, xyz, None, True))
+    assert isinstance(pointcept.grouping(idx, feat.as_subclass(Marked), xyz), Marked)
 
 
 @pytest.mark.parametrize("M,K", [(1, 1), (85, 3), (256, 16)])
