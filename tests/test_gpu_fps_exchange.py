@@ -58,3 +58,20 @@ def test_ragged_fps_with_a_large_cloud_matches_oracle(cuda_device, sizes):
         if count:
             want.append(a + O.fps(x[None, a:b], count, 0)[0])
     np.testing.assert_array_equal(got, np.concatenate(want))
+
+
+@pytest.mark.parametrize("kind", ["lattice", "repeated", "one", "octaves", "never", "infinite"])
+@pytest.mark.parametrize("n", [65, 24577, 140_000])
+def test_one_cloud_over_the_chip_with_hard_cuts_matches_oracle(cuda_device, kind, n):
+    """The exchanging kernels of one cloud over many workgroups, whose runs of up
+    to 64 live candidates and longer ones take different code."""
+    import mps_pointops as mp
+
+    xyz = _cloud("octaves" if kind == "infinite" else kind, n)[:1].contiguous()
+    if kind == "infinite":
+        xyz[0, 7] = float("inf")
+        xyz[0, 40, 1] = float("-inf")
+    npoint = min(n, 700)
+    skip = kind == "never"
+    got = mp.furthest_point_sample(xyz.cuda(), npoint, 3, skip, strategy="multigroup")
+    np.testing.assert_array_equal(got.cpu().numpy(), O.fps(xyz, npoint, 3, skip))
