@@ -169,6 +169,16 @@ hipError_t pointops_knn_screen(const float *query, const float *ref, float *dist
 hipError_t pointops_knn_flat(const float *y, const float *x, const int64_t *ptr_y,
                              const int64_t *ptr_x, int64_t *out, int64_t Q, int64_t batch,
                              int64_t D, int64_t K, hipStream_t stream);
+/* Nearest reference per query by the same screen (K = 1; the search of
+ * pointops_chamfer_nearest_f32 with norm 2 for clouds without lengths):
+ * dist2 (B,M) squared distances and idx (B,M), identical to the linear scan,
+ * for finite coordinates; N >= 1.  `workspace`:
+ * pointops_knn_screen_workspace_bytes(B, N, 3) bytes, as above.  Accelerates
+ * chamfer.py:122-158. */
+hipError_t pointops_nearest3_screen(const float *query, const float *ref, float *dist2,
+                                    int64_t *idx, void *workspace, int64_t B, int64_t M, int64_t N,
+                                    hipStream_t stream);
+
 /* The same flat search (identical results) screened as pointops_knn_screen;
  * D <= 128, K <= 64; total_x is x's row count, ptr_x[batch] at most that.
  * `workspace`: pointops_knn_flat_screen_workspace_bytes(total_x, batch, D)

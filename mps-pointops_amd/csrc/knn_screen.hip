@@ -36,7 +36,8 @@
 // row is 256 bytes from L2).  Measured: config 2 98 -> 43 us, 16 x 512 x 1024
 // 41 -> 18 us, D = 64 359 -> 53 us, D = 128 590 -> 75 us (one lane per query,
 // every pair's distance as defined), 3 ragged clouds of 20000, k = 16 1000 ->
-// 190 us (one wave per query).  Eight waves a block, since four left every
+// 190 us (one wave per query); k = 1, squared distances (the Chamfer loss's), both
+// directions of 32 x 8192 x 8192 735 -> 450 us (cell grid).  Eight waves a block, since four left every
 // phase waiting on its own latency (65 against 43 us at config 2); bfloat16 in
 // three products instead of f16 in one took 61 us for D = 64.
 #include <type_traits>
@@ -316,6 +317,7 @@ struct ScreenArgs {
     ScreenLayout L;
     int64_t batch, M, N, QS;  // dense: queries of a cloud lie QS rows apart
     int D, K;
+    bool squared;  // dense: distances squared, not their roots
 };
 
 // KS k-steps (D <= 16 KS); D3: one fragment holds everything.  Eight waves,
@@ -584,9 +586,14 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
         // the least; then the count says on which side, interpolating.
         float guess = least + (sum / some - least) * -__logf(1.f - fminf(static_cast<float>(K) / some, 0.99f));
         float reach_lo = 0.f, reach_hi = some;
-        if (some < static_cast<float>(K)) hi = 3e38f;  // everything finite is listed
         const int most = K + 2 + K / 8;
         bool done = some <= static_cast<float>(most);
+        if (some < static_cast<float>(K)) {
+            hi = 3e38f;  // everything finite is listed
+        } else if (K == 1) {
+            hi = least;  // one group reaches the least minimum
+            done = true;
+        }
         for (int it = 0; it < 12 && ballot(!done) != 0; ++it) {
             if (!(guess > lo && guess < hi) || it > 6) guess = 0.5f * (lo + hi);
             float reach = 0.f;
@@ -775,7 +782,8 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
                 if constexpr (FLAT) {
                     a.idx[slot] = ref0 + at;
                 } else {
-                    a.dist[slot] = sqrtf(i2f(static_cast<int>(key)));
+                    const float d = i2f(static_cast<int>(key));
+                    a.dist[slot] = a.squared ? d : sqrtf(d);
                     a.idx[slot] = at;
                 }
             }
@@ -800,7 +808,7 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
             if constexpr (FLAT) {
                 a.idx[slot] = li[0] < 0 ? int64_t(-1) : ref0 + li[0];
             } else {
-                a.dist[slot] = sqrtf(ld[0]);
+                a.dist[slot] = a.squared ? ld[0] : sqrtf(ld[0]);
                 a.idx[slot] = D3 ? static_cast<int64_t>(static_cast<uint32_t>(li[0]))
                                  : (li[0] < 0 ? int64_t(-1) : int64_t(li[0]));
             }
@@ -940,6 +948,29 @@ hipError_t pointops_knn_screen(const float* query, const float* ref, float* dist
     a.QS = M;
     a.D = static_cast<int>(D);
     a.K = static_cast<int>(K);
+    return launch_screen<false>(a, workspace, B * N, blocks, stream);
+}
+
+hipError_t pointops_nearest3_screen(const float* query, const float* ref, float* dist2, int64_t* idx,
+                                    void* workspace, int64_t B, int64_t M, int64_t N,
+                                    hipStream_t stream) {
+    if (B < 0 || M < 0 || N < 1) return hipErrorInvalidValue;
+    if (B == 0 || M == 0) return hipSuccess;
+    const int64_t blocks = screen_blocks(M, B);
+    if (workspace == nullptr || N > INT32_MAX - kWave || !screen_fits(blocks, B * N, B))
+        return hipErrorInvalidValue;
+    ScreenArgs a{};
+    a.query = query;
+    a.ref = ref;
+    a.dist = dist2;
+    a.idx = idx;
+    a.batch = B;
+    a.M = M;
+    a.N = N;
+    a.QS = M;
+    a.D = 3;
+    a.K = 1;
+    a.squared = true;
     return launch_screen<false>(a, workspace, B * N, blocks, stream);
 }
 

@@ -47,6 +47,45 @@ def _grid_eligible(query: Tensor, ref: Tensor, norm: int, full: bool) -> bool:
             and batch * ((query_count + 63) // 64) < limit)
 
 
+# The matrix-core screen's range of references, in us of the two directions
+# together (a tenth of one side far from the other) against the grid and the
+# scan: 2 x 1024 x 1024 27 / 165 / 86, 16 x 4096 x 4096 93 / 314 / 332, 32 x 8192
+# x 8192 450 / 735 / 1100, 8 x 16384 x 16384 387 / 638 / 1350, 1 x 32768 x 32768
+# 214 / 491 / 2600, 4 x 65536 x 65536 2566 / 1355 / 8700.  (The grid's time
+# depends on the data: 32 x 8192 x 8192 162 us where every query has a close
+# reference, 573 us the other way; the screen takes 225 us either way.)
+_SCREEN_MIN_REFS = 512
+_SCREEN_MAX_REFS = 1 << 15
+
+
+def _screen_eligible(query: Tensor, ref: Tensor, norm: int, full: bool) -> bool:
+    batch, query_count, dimension = query.shape
+    ref_count = ref.shape[1]
+    limit = (1 << 31) - 64  # the entry point's launch and index range
+    return (full and norm == 2 and dimension == 3 and query.dtype == torch.float32
+            and _SCREEN_MIN_REFS <= ref_count <= _SCREEN_MAX_REFS
+            and batch * ((query_count + 63) // 64) < limit
+            and batch * (ref_count // 32 + 1) < 1 << 30)
+
+
+def _nearest_screen(query: Tensor, ref: Tensor) -> tuple[Tensor, Tensor]:
+    """pointops_nearest3_screen: all pairs as matrix products whose error is
+    bounded, the few references they leave computed as the scan kernel does.
+    Results equal the scan kernel's everywhere."""
+    batch, query_count, _ = query.shape
+    ref_count = ref.shape[1]
+    query = query.contiguous()
+    ref = ref.contiguous()
+    distances = torch.empty((batch, query_count), device=query.device, dtype=query.dtype)
+    indices = torch.empty((batch, query_count), device=query.device, dtype=torch.int64)
+    size = _native.size_query("pointops_knn_screen_workspace_bytes", batch, ref_count, 3)
+    workspace = torch.empty(size, dtype=torch.uint8, device=query.device)
+    _native.call("pointops_nearest3_screen", query.data_ptr(), ref.data_ptr(), distances.data_ptr(),
+                 indices.data_ptr(), workspace.data_ptr(), batch, query_count, ref_count,
+                 _native.stream(query.device))
+    return distances, indices
+
+
 def _nearest_grid(query: Tensor, ref: Tensor) -> tuple[Tensor, Tensor]:
     """pointops_nearest3_grid: the grid search, and a linear scan inside the
     same call for queries whose nearest reference is several cells away.
@@ -90,6 +129,8 @@ def _nearest_device(query: Tensor, ref: Tensor, query_lengths: Tensor, ref_lengt
     """Distance (squared L2 or L1) and first-minimum index per query row;
     rows beyond the query lengths, and rows of an empty reference cloud, are
     (0, -1) (chamfer.py:122-158).  ``full``: no lengths were given."""
+    if _screen_eligible(query, ref, norm, full):
+        return _nearest_screen(query, ref)
     if _grid_eligible(query, ref, norm, full):
         return _nearest_grid(query, ref)
     return _nearest_scan(query, ref, query_lengths, ref_lengths, norm)

@@ -114,3 +114,31 @@ def test_flat_screen_matches_scan(cuda_device, kind, D, sizes_x, sizes_y, k):
                  px.data_ptr(), got.data_ptr(), ws.data_ptr(), len(y), len(x), len(sizes_x), D, k,
                  st)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("kind", ["uniform", "lattice", "copies", "far", "overflow"])
+@pytest.mark.parametrize("B,M,N", [(3, 1, 512), (2, 63, 513), (1, 65, 1023), (2, 300, 4097), (1, 1000, 32768)])
+def test_nearest_screen_matches_scan(cuda_device, kind, B, M, N):
+    """The Chamfer loss's nearest reference and squared distance, bit for bit:
+    ties, more copies of one point than a list holds, clouds far from the
+    origin, distances that overflow."""
+    from mps_pointops import chamfer
+
+    g = torch.Generator().manual_seed(B * M + N)
+    q, r = torch.rand(B, M, 3, generator=g), torch.rand(B, N, 3, generator=g)
+    if kind == "lattice":
+        q, r = (q * 6).round(), (r * 6).round()
+    elif kind == "copies":
+        r[:, : N // 2] = q[:, :1]
+    elif kind == "far":
+        q, r = q + 1e4, r + 1e4
+    elif kind == "overflow":
+        q[:, ::2] *= 3e19
+        r[:, 1::3] *= -3e19
+    q, r = q.cuda(), r.cuda()
+    assert chamfer._screen_eligible(q, r, 2, True)
+    lengths = [torch.full((B,), n, dtype=torch.int64, device=q.device) for n in (M, N)]
+    d, i = chamfer._nearest_device(q, r, *lengths, 2, full=True)
+    want_d, want_i = chamfer._nearest_scan(q, r, *lengths, 2)
+    assert torch.equal(i, want_i)
+    assert torch.equal(d.view(torch.int32), want_d.view(torch.int32))
