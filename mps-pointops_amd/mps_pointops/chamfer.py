@@ -53,8 +53,13 @@ def _grid_eligible(query: Tensor, ref: Tensor, norm: int, full: bool) -> bool:
 # x 8192 450 / 735 / 1100, 8 x 16384 x 16384 387 / 638 / 1350, 1 x 32768 x 32768
 # 214 / 491 / 2600, 4 x 65536 x 65536 2566 / 1355 / 8700.  (The grid's time
 # depends on the data: 32 x 8192 x 8192 162 us where every query has a close
-# reference, 573 us the other way; the screen takes 225 us either way.)
+# reference, 573 us the other way; the screen takes 225 us either way.)  Its 64
+# queries cost about 20 ns before any reference, so many queries need more
+# references for it to pay: 32 x 1024 queries x 512 references 18 against the
+# scan's 23, 8 x 8192 x 1024 31 against 44, but 32 x 8192 x 512 90 against 40 and
+# x 768 92 against 57 (x 4096 155 against 270).
 _SCREEN_MIN_REFS = 512
+_SCREEN_MIN_REFS_MANY = 2048
 _SCREEN_MAX_REFS = 1 << 15
 
 
@@ -62,9 +67,10 @@ def _screen_eligible(query: Tensor, ref: Tensor, norm: int, full: bool) -> bool:
     batch, query_count, dimension = query.shape
     ref_count = ref.shape[1]
     limit = (1 << 31) - 64  # the entry point's launch and index range
+    blocks = batch * ((query_count + 63) // 64)
     return (full and norm == 2 and dimension == 3 and query.dtype == torch.float32
-            and _SCREEN_MIN_REFS <= ref_count <= _SCREEN_MAX_REFS
-            and batch * ((query_count + 63) // 64) < limit
+            and min(max(_SCREEN_MIN_REFS, blocks), _SCREEN_MIN_REFS_MANY) <= ref_count
+            and ref_count <= _SCREEN_MAX_REFS and blocks < limit
             and batch * (ref_count // 32 + 1) < 1 << 30)
 
 
