@@ -644,8 +644,14 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
                 for (int i = 1; i < 16; ++i) least = fminf(least, acc[u][i]);
                 uint32_t h = 0;
                 if (ballot(least <= lim[u]) != 0 && real) {
+                    // Bit i from the sign of limit - s (set: beyond it): a
+                    // comparison and a select per bit wait for vcc each time (front
+                    // end 367 -> 360 us, 3 ragged clouds of 20000 with K = 16 and
+                    // their grouping 631 -> 613 us).
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) h |= acc[u][i] <= lim[u] ? 1u << i : 0u;
+                    for (int i = 15; i >= 0; --i)
+                        h = __builtin_amdgcn_alignbit(h, static_cast<uint32_t>(f2i(lim[u] - acc[u][i])), 31);
+                    h = ~h & 0xFFFFu;
                 }
                 hit[u][j / 2] |= h << (16 * (j & 1));
             }
