@@ -151,8 +151,8 @@ hipError_t pointops_knn_feat(const float *query, const float *ref, float *dist, 
                              hipStream_t stream);
 
 /* The dense search (identical results: pointops_knn3 for D = 3, else
- * pointops_knn_feat) screened on the matrix cores: products of operands split
- * into bfloat16 parts, with a bound on their error, rule out all but about K
+ * pointops_knn_feat) screened on the matrix cores: products of bfloat16
+ * parts (D = 3) or of scaled float16, with a bound on their error, rule out all but about K
  * references of each query, whose distances are then computed and ranked as
  * the other entry points do.  D <= 128, K <= 64.  `workspace`:
  * pointops_knn_screen_workspace_bytes(B, N, D) bytes, 16-byte aligned, no
@@ -162,13 +162,6 @@ hipError_t pointops_knn_screen(const float *query, const float *ref, float *dist
                                void *workspace, int64_t B, int64_t M, int64_t N, int64_t D,
                                int64_t K, hipStream_t stream);
 
-/* Flat (ragged) kNN, global x indices padded with -1, (Q,K).  Replaces
- * _flat_search_mps.py:96-107 (kernels/flat_search.metal:44-154 for D = 3,
- * kernels/feature_knn.metal:166-199 otherwise).  y (Q,D) queries, x (Nx,D)
- * references, ptr_y/ptr_x (batch+1,) segment offsets. */
-hipError_t pointops_knn_flat(const float *y, const float *x, const int64_t *ptr_y,
-                             const int64_t *ptr_x, int64_t *out, int64_t Q, int64_t batch,
-                             int64_t D, int64_t K, hipStream_t stream);
 /* Nearest reference per query by the same screen (K = 1; the search of
  * pointops_chamfer_nearest_f32 with norm 2 for clouds without lengths):
  * dist2 (B,M) squared distances and idx (B,M), identical to the linear scan,
@@ -179,6 +172,13 @@ hipError_t pointops_nearest3_screen(const float *query, const float *ref, float 
                                     int64_t *idx, void *workspace, int64_t B, int64_t M, int64_t N,
                                     hipStream_t stream);
 
+/* Flat (ragged) kNN, global x indices padded with -1, (Q,K).  Replaces
+ * _flat_search_mps.py:96-107 (kernels/flat_search.metal:44-154 for D = 3,
+ * kernels/feature_knn.metal:166-199 otherwise).  y (Q,D) queries, x (Nx,D)
+ * references, ptr_y/ptr_x (batch+1,) segment offsets. */
+hipError_t pointops_knn_flat(const float *y, const float *x, const int64_t *ptr_y,
+                             const int64_t *ptr_x, int64_t *out, int64_t Q, int64_t batch,
+                             int64_t D, int64_t K, hipStream_t stream);
 /* The same flat search (identical results) screened as pointops_knn_screen;
  * D <= 128, K <= 64; total_x is x's row count, ptr_x[batch] at most that.
  * `workspace`: pointops_knn_flat_screen_workspace_bytes(total_x, batch, D)

@@ -2,7 +2,7 @@
 //
 // The searches define every rounding of a distance (knn.hip), which a matrix
 // product cannot reproduce, but it can tell which references cannot be among
-// the K nearest.  Each block serves 64 queries of one cloud; its four waves
+// the K nearest.  Each block serves 64 queries of one cloud; its eight waves
 // split the cloud's tiles of 32 references and twice compute, for all pairs,
 //
 //     s = |r|^2 - 2 q.r     (the squared distance less |q|^2)
