@@ -267,19 +267,27 @@ def grouping(idx: Tensor, feat: Tensor, xyz: Tensor, new_xyz: Tensor | None = No
     return _grouped(idx, feat, xyz, new_xyz, with_xyz)
 
 
+def _kept(idx: Tensor, *inputs: Tensor) -> Tensor:
+    """Contiguous indices for _GroupRows: a copy where a backward will read
+    them again, since the caller may write to its own before that."""
+    if torch.is_grad_enabled() and any(t.requires_grad for t in inputs):
+        return idx.clone(memory_format=torch.contiguous_format)
+    return idx.contiguous()
+
+
 def _grouped(idx: Tensor, feat: Tensor, xyz: Tensor, new_xyz: Tensor | None,
              with_xyz: bool) -> Tensor:
     """grouping for indices that are known to be in range."""
     if not with_xyz:
         if len(feat) and _native_rows(feat):
-            return _GroupRows.apply(feat, None, None, idx.contiguous())
+            return _GroupRows.apply(feat, None, None, _kept(idx, feat))
         return _gather_rows(feat, idx)
     centres = xyz if new_xyz is None else new_xyz
     _points(centres, "new_xyz")
     if centres.device != xyz.device or len(centres) != len(idx):
         raise ValueError("new_xyz must have one row per idx row on the xyz device")
     if len(feat) and _native_rows(feat, xyz, centres):
-        return _GroupRows.apply(feat, xyz, centres, idx.contiguous())
+        return _GroupRows.apply(feat, xyz, centres, _kept(idx, feat, xyz, centres))
     return _group_rows(feat, xyz, centres, idx)
 
 

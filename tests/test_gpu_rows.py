@@ -96,6 +96,30 @@ def test_a_trace_and_a_subclass_keep_the_tensor_operations(cuda_device):
     assert isinstance(pointcept.grouping(idx, feat.as_subclass(Marked), xyz), Marked)
 
 
+@pytest.mark.parametrize("with_xyz", [False, True])
+@pytest.mark.parametrize("own_idx", [False, True])
+def test_indices_may_be_written_to_after_the_call(cuda_device, with_xyz, own_idx):
+    """The gradient belongs to the indices of the call, whether the caller
+    passed them or got them back."""
+    from mps_pointops import pointcept
+
+    g = torch.Generator().manual_seed(5)
+    xyz = torch.randn(40, 3, generator=g).cuda()
+    offset = torch.tensor([3, 40], dtype=torch.int32, device="cuda")  # 3 < K: -1 among them
+    idx, _ = pointcept.knn_query(5, xyz, offset)
+    weight = torch.randn(40, 5, 9 if with_xyz else 6, generator=g).cuda()
+    grads = []
+    for write in (False, True):
+        feat = torch.ones(40, 6, device="cuda").requires_grad_()
+        out, at = pointcept.knn_query_and_group(feat, xyz, offset, nsample=5, with_xyz=with_xyz,
+                                                idx=idx.clone() if own_idx else None)
+        assert torch.equal(at, idx)
+        if write:
+            at[at < 0] = 0
+        grads.append(torch.autograd.grad(out, feat, weight)[0])
+    torch.testing.assert_close(grads[1], grads[0], rtol=1e-5, atol=1e-5)  # sums of at most 40 terms
+
+
 @pytest.mark.parametrize("M,K", [(1, 1), (85, 3), (256, 16)])
 def test_knn_finish_matches_tensor_operations(cuda_device, M, K):
     from mps_pointops import _native
