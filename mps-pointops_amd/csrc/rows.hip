@@ -64,8 +64,9 @@ __global__ __launch_bounds__(kRowsThreads) void group_rows_kernel(
 }
 
 // One wave per query: its K W gradients are contiguous, each added to its
-// neighbour's feature or position by a hardware float atomic (the order of
-// whose additions is not fixed, like index_add's); the query's own position
+// neighbour's feature or position by a hardware float atomic, the order of
+// whose additions is not fixed (where the caller has asked for deterministic
+// algorithms it uses tensor operations instead); the query's own position
 // takes the negated sum of its relative offsets' gradients.
 template <typename I>
 __global__ __launch_bounds__(kRowsThreads) void group_rows_grad_kernel(

@@ -90,9 +90,10 @@ def _group_rows(feat: Tensor, xyz: Tensor | None, centres: Tensor | None, idx: T
 
 
 def _scatter_rows(grad: Tensor, idx: Tensor, rows: int, with_xyz: bool, want) -> list:
-    """What _ScatterRows computes, as tensor operations (batched gradients:
-    a vectorised Jacobian's backward runs under a function transform); None
-    for each gradient that ``want`` leaves out."""
+    """What _ScatterRows computes, as tensor operations: for batched gradients
+    (a vectorised Jacobian's backward runs under a function transform) and for
+    deterministic algorithms, whose index_add has a fixed order that float
+    atomics have not.  None for each gradient that ``want`` leaves out."""
     grad = grad.where((idx >= 0)[..., None], 0.0)
     at = idx.clamp_min(0).reshape(-1)
     off = 3 if with_xyz else 0
@@ -133,7 +134,7 @@ class _GroupRows(torch.autograd.Function):
         want = ctx.needs_input_grad[:3]
         if grad is None or not any(want):
             return None, None, None, None
-        if not _native.plain(grad):
+        if not _native.plain(grad) or torch.are_deterministic_algorithms_enabled():
             return (*_scatter_rows(grad, idx, ctx.rows, ctx.with_xyz, want), None)
         grads = _ScatterRows.apply(grad, idx, ctx.rows, ctx.with_xyz, want)
         return (*(g if w else None for g, w in zip(grads, want)), None)

@@ -120,6 +120,28 @@ def test_indices_may_be_written_to_after_the_call(cuda_device, with_xyz, own_idx
     torch.testing.assert_close(grads[1], grads[0], rtol=1e-5, atol=1e-5)  # sums of at most 40 terms
 
 
+@pytest.mark.parametrize("with_xyz", [False, True])
+def test_deterministic_algorithms_repeat_the_gradient(cuda_device, with_xyz):
+    """Bit for bit, with thousands of terms on each of a few rows."""
+    from mps_pointops import pointcept
+
+    g = torch.Generator().manual_seed(6)
+    idx = torch.randint(-1, 4, (2000, 32), generator=g).cuda()
+    feat, xyz = torch.randn(4, 16, generator=g).cuda(), torch.randn(4, 3, generator=g).cuda()
+    new = torch.randn(2000, 3, generator=g).cuda().requires_grad_() if with_xyz else None
+    inputs = [feat.requires_grad_()] + ([xyz.requires_grad_(), new] if with_xyz else [])
+    weight = torch.randn(2000, 32, 19 if with_xyz else 16, generator=g).cuda()
+    out = pointcept.grouping(idx, feat, xyz, new, with_xyz)
+    torch.use_deterministic_algorithms(True)
+    try:
+        first, *others = (torch.autograd.grad(out, inputs, weight, retain_graph=True) for _ in range(8))
+    finally:
+        torch.use_deterministic_algorithms(False)
+    for other in others:
+        for a, b in zip(first, other):
+            assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("M,K", [(1, 1), (85, 3), (256, 16)])
 def test_knn_finish_matches_tensor_operations(cuda_device, M, K):
     from mps_pointops import _native
