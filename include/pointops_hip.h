@@ -180,7 +180,8 @@ hipError_t pointops_knn_flat(const float *y, const float *x, const int64_t *ptr_
                              const int64_t *ptr_x, int64_t *out, int64_t Q, int64_t batch,
                              int64_t D, int64_t K, hipStream_t stream);
 /* The same flat search (identical results) screened as pointops_knn_screen;
- * D <= 128, K <= 64; total_x is x's row count, ptr_x[batch] at most that.
+ * D <= 128, K <= 64; total_x < 2^31 - 64 is x's row count, ptr_x[batch] at
+ * most that.
  * `workspace`: pointops_knn_flat_screen_workspace_bytes(total_x, batch, D)
  * bytes, 16-byte aligned, no initialisation needed. */
 size_t pointops_knn_flat_screen_workspace_bytes(int64_t total_x, int64_t batch, int64_t D);

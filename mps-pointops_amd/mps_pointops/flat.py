@@ -26,6 +26,7 @@ from torch import Tensor
 
 from . import _native
 from ._ball_query import _checked_radius_and_k
+from .ops import SCREEN_MAX_ROWS
 
 _KNN_MAX_K = 256          # widest neighbour list of the native kNN (ops.py:30)
 # Searches of at most this many dimensions and neighbours are screened on the
@@ -42,7 +43,7 @@ _SCREEN_MIN_PAIRS = 1 << 20
 
 def _screened(rows_x: int, rows_y: int, clouds: int, D: int, k: int) -> bool:
     mean = rows_x / max(clouds, 1)
-    return (D <= _SCREEN_MAX_D and k <= _SCREEN_MAX_K and mean >= (64 if D == 3 else 128)
+    return (D <= _SCREEN_MAX_D and k <= _SCREEN_MAX_K and rows_x <= SCREEN_MAX_ROWS and mean >= (64 if D == 3 else 128)
             and rows_y * mean >= _SCREEN_MIN_PAIRS)
 
 

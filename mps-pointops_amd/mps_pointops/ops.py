@@ -46,6 +46,10 @@ _KNN_WINDOW_MAX_M = 16384
 _KNN_SCREEN_MAX_D = 128
 _KNN_SCREEN_MAX_K = 64
 _KNN_SCREEN_MIN_PAIRS = 1 << 20
+# Reference rows in all (also of the ragged searches): beyond these the
+# screen's workspace (up to 256 bytes a row) and its 32-bit numbers of rows and
+# tiles would refuse what the scanning entry points take.
+SCREEN_MAX_ROWS = 1 << 27
 
 
 def _screened(B: int, M: int, N: int, D: int, k: int) -> bool:
@@ -56,7 +60,7 @@ def _screened(B: int, M: int, N: int, D: int, k: int) -> bool:
     39 against 35 us, 8 x 256 x 256 (D = 68, k = 20) 38 against 28, 8 x 600 x
     600 (D = 40, k = 20) 44 against 53, 4 x 1000 x 1000 (D = 100, k = 40) 79
     against 129."""
-    if D > _KNN_SCREEN_MAX_D or k > _KNN_SCREEN_MAX_K:
+    if D > _KNN_SCREEN_MAX_D or k > _KNN_SCREEN_MAX_K or B * N > SCREEN_MAX_ROWS:
         return False
     if D == 3:
         return N >= _KNN_WINDOW_MIN_N
