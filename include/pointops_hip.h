@@ -41,8 +41,10 @@ int pointops_device_supported(int device);
  * (`_library("fps").furthest_point_sample`, kernels/fps.metal:19-107).
  * xyz (B,N,3) f32 -> out (B,npoint) int64; ties go to the smaller index; once
  * every point is taken the rest repeat the first maximum (index 0).
- * `scratch` must hold pointops_fps_dense_scratch_bytes(B, N) bytes (0 means
- * it may be NULL: the running distances then live on chip). */
+ * `scratch` must hold pointops_fps_dense_scratch_bytes(B, N) bytes: the sorted
+ * points of clouds of 8193 to 24576 (where it is 16-byte aligned; else, and for
+ * larger clouds, the running distances, several times slower).  0 means it may
+ * be NULL: both then live on chip. */
 size_t pointops_fps_dense_scratch_bytes(int64_t B, int64_t N);
 hipError_t pointops_fps_dense(const float *xyz, int64_t *out, void *scratch, int64_t B,
                               int64_t N, int64_t npoint, int64_t start_idx,
@@ -89,8 +91,8 @@ hipError_t pointops_fps_flat(const float *x, const int64_t *ptr, const int64_t *
                              hipStream_t stream);
 
 /* The same search with room for each cloud's sorted points in `scratch`
- * (pointops_fps_flat_sorted_scratch_bytes(total_n, max_len) bytes, 16-byte
- * aligned): several times faster for clouds of 8193 to 24576 points. */
+ * (pointops_fps_flat_sorted_scratch_bytes(total_n, max_len) bytes): where it is
+ * 16-byte aligned, several times faster for clouds of 8193 to 24576 points. */
 size_t pointops_fps_flat_sorted_scratch_bytes(int64_t total_n, int64_t max_len);
 hipError_t pointops_fps_flat_sorted(const float *x, const int64_t *ptr, const int64_t *out_ptr,
                                     const int64_t *starts, int64_t *out, void *scratch,

@@ -37,6 +37,7 @@
 //                           CUs' registers, the cloud streamed from HBM.
 #include <hip/hip_cooperative_groups.h>
 
+#include <atomic>
 #include <cstdlib>
 #include <mutex>
 #include <type_traits>
@@ -1578,6 +1579,7 @@ __global__ __launch_bounds__(kLeadThreads) void fps_lead_kernel(
 // step, took 17.8 ms (4.35 us a step).
 constexpr int kWideMaxTiles = 48;  // tiles per follower: 6 bytes x 24576 points of LDS
 constexpr int64_t kWideMaxPoints = int64_t(kWideMaxTiles) * kLeadFollowers * kWave;
+constexpr int kWidePointBytes = sizeof(float) + sizeof(uint16_t);  // of dynamic LDS
 constexpr int kWideBatch = 4;      // tiles loaded together
 // Clouds of at most this many samples are left to fps_global_kernel, which
 // needs no sort: 8 x 16384 points, 32 samples 140 us against 175 (64 samples
@@ -2631,6 +2633,23 @@ size_t fps_scratch_bytes_per_point(int64_t max_len) {
     return max_len <= kWideMaxPoints ? sizeof(float4) : sizeof(float);
 }
 
+// Allows fps_wide_kernel its largest dynamic LDS, once per device: the limit
+// belongs to the process, so a call that set its own size could lower it
+// between another thread's set and launch.
+hipError_t fps_wide_allow_lds() {
+    static std::atomic<uint64_t> allowed{0};  // a bit per device
+    int dev = 0;
+    const hipError_t err = hipGetDevice(&dev);
+    if (err != hipSuccess) return err;
+    const uint64_t bit = dev < 64 ? uint64_t(1) << dev : 0;
+    if ((allowed.load(std::memory_order_acquire) & bit) != 0) return hipSuccess;
+    const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(&fps_wide_kernel),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize,
+                                               static_cast<int>(kWideMaxPoints * kWidePointBytes));
+    if (set == hipSuccess) allowed.fetch_or(bit, std::memory_order_release);
+    return set;
+}
+
 hipError_t launch_fps(const float* xyz, const int64_t* ptr, const int64_t* out_ptr,
                       const int64_t* starts, int64_t* out, float* scratch, int64_t blocks,
                       int64_t max_len, int64_t N, int64_t npoint, int64_t start, int skip,
@@ -2650,8 +2669,9 @@ hipError_t launch_fps(const float* xyz, const int64_t* ptr, const int64_t* out_p
     // kWideFew samples and the global kernel the others; a dense launch is all
     // one or all the other, a ragged one may hold both, so it runs both (in
     // turn on the stream: the second may reuse the first's scratch).
-    // (`sorted`: the scratch has room for the wide kernel's points.)
-    const bool wide = sorted && max_len <= kWideMaxPoints;
+    // (`sorted`: the scratch has room for the wide kernel's points, which it
+    // reads 16 bytes at a time.)
+    const bool wide = sorted && max_len <= kWideMaxPoints && reinterpret_cast<uintptr_t>(scratch) % 16 == 0;
     if (!wide || ptr != nullptr || npoint <= kWideFew) {
         hipLaunchKernelGGL((fps_global_kernel<kGlobalThreads>), dim3(static_cast<uint32_t>(blocks)),
                            dim3(kGlobalThreads), 0, stream, xyz, ptr, out_ptr, starts, out, scratch,
@@ -2661,12 +2681,10 @@ hipError_t launch_fps(const float* xyz, const int64_t* ptr, const int64_t* out_p
     }
     constexpr int kRow = kLeadFollowers * kWave;
     const int cap = static_cast<int>((max_len + kRow - 1) / kRow) * kRow;
-    const int lds = cap * static_cast<int>(sizeof(float) + sizeof(uint16_t));
-    const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(&fps_wide_kernel),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    const hipError_t err = fps_wide_allow_lds();
     if (err != hipSuccess) return err;
     hipLaunchKernelGGL(fps_wide_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kLeadThreads),
-                       static_cast<size_t>(lds), stream, xyz, ptr, out_ptr, starts, out,
+                       static_cast<size_t>(cap) * kWidePointBytes, stream, xyz, ptr, out_ptr, starts, out,
                        reinterpret_cast<float4*>(scratch), cap, N, npoint, start, skip, kWideFew);
     return hipGetLastError();
 }

@@ -75,3 +75,38 @@ def test_one_cloud_over_the_chip_with_hard_cuts_matches_oracle(cuda_device, kind
     skip = kind == "never"
     got = mp.furthest_point_sample(xyz.cuda(), npoint, 3, skip, strategy="multigroup")
     np.testing.assert_array_equal(got.cpu().numpy(), O.fps(xyz, npoint, 3, skip))
+
+
+def test_threads_sampling_clouds_of_different_sizes(cuda_device):
+    """The kernel's dynamic LDS differs per call, its limit belongs to the
+    process: calls of several threads leave each other's alone."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    import mps_pointops as mp
+
+    clouds = [torch.rand(1, n, 3, generator=torch.Generator().manual_seed(n)).cuda()
+              for n in (8193, 24576, 12000, 20000)]
+    want = [mp.furthest_point_sample(x, 64) for x in clouds]
+
+    def sample(i):
+        return i % 4, mp.furthest_point_sample(clouds[i % 4], 64)
+
+    with ThreadPoolExecutor(4) as pool:
+        for i, got in pool.map(sample, range(80)):
+            assert torch.equal(got, want[i])
+
+
+def test_unaligned_scratch_is_served(cuda_device):
+    """Scratch at any 4-byte boundary, as the running distances need: the
+    kernel that reads 16 bytes at a time is left out."""
+    from mps_pointops import _native
+
+    n = 9000
+    xyz = torch.rand(1, n, 3, generator=torch.Generator().manual_seed(1))
+    x, out = xyz.cuda(), torch.empty(1, 100, dtype=torch.long, device="cuda")
+    size = _native.size_query("pointops_fps_dense_scratch_bytes", 1, n)
+    scratch = torch.empty(size + 16, dtype=torch.uint8, device="cuda")
+    for offset in (0, 4):
+        _native.call("pointops_fps_dense", x.data_ptr(), out.data_ptr(), scratch.data_ptr() + offset,
+                     1, n, 100, 0, 0, _native.stream(x.device))
+        np.testing.assert_array_equal(out.cpu().numpy(), O.fps(xyz, 100, 0))
