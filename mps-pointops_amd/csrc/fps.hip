@@ -1034,36 +1034,55 @@ __device__ __forceinline__ int lead_block(int& cmd, int& wv, int& rem, uint32_t&
 // quarter octave below m and KC - 1 or KC keys wanted, 283 us so (fewer keys
 // shorten the runs: KC - 3 288 us; more probes lengthen the exchange: exactly
 // KC 306 us).
+//
+// Where many keys are the same (lattices, repeated points) no threshold may
+// leave that many, and a bisection to the last bit held the exchange up: after
+// kCutHalvings probes any cut serves (a run then ends sooner), and without one
+// the next probe is m itself, which settles whether there is any (integer
+// lattices in 32 x 4096: 3660 -> 2360 us, half of the points at the origin
+// 536 -> 372 us).
 struct KeyCut {
     uint64_t first, second;  // lanes whose d1 / d2 is at or above the cut
 };
+constexpr int kCutHalvings = 5;
 template <int KC>
 __device__ __forceinline__ KeyCut cut_top_keys(int d1, int d2, int m, uint32_t& guess) {
     KeyCut best{0, 0};
     if (m < 0) return best;  // only points that are never sampled
-    int lo = -1, hi = m + 1;  // more than KC keys at lo (-1: not known yet), at most KC at hi
-    uint32_t below = guess;   // largest key less the next outward probe
-    for (;;) {
-        int t;
-        if (lo < 0) {
-            t = static_cast<uint32_t>(m) > below ? m - static_cast<int>(below) : 0;
-            below <<= 1;
-        } else {
-            if (hi - lo <= 1) return best;
-            t = lo + (hi - lo) / 2;
-        }
+    int lo, hi = m + 1;  // more than KC keys at lo, at most KC (`best`) at hi
+    int t;
+    auto few = [&]() {  // how many keys reach t, -1 for more than KC
         const uint64_t a = ballot(d1 >= t);
         const uint64_t b = ballot(d2 >= t);
         const int count = __popcll(a) + __popcll(b);
         if (count > KC) {
             lo = t;
-        } else {
-            hi = t;
-            best = {a, b};
-            if (count >= KC - 2 || t == 0) {
-                guess = max(static_cast<uint32_t>(m - t), 1u << 12);
-                return best;
-            }
+            return -1;
+        }
+        hi = t;
+        best = {a, b};
+        return count;
+    };
+    for (uint32_t below = guess;; below <<= 1) {
+        t = static_cast<uint32_t>(m) > below ? m - static_cast<int>(below) : 0;
+        const int count = few();
+        if (__builtin_expect(count < 0, 0)) break;
+        if (count >= KC - 2 || t == 0) {
+            guess = max(static_cast<uint32_t>(m - t), 1u << 12);
+            return best;
+        }
+    }
+    for (int halvings = kCutHalvings;; --halvings) {
+        t = lo + static_cast<int>(static_cast<uint32_t>(hi - lo) / 2);
+        if (t == lo) return best;
+        if (__builtin_expect(halvings == 0, 0)) {  // see above
+            if (best.first != 0) return best;
+            t = m;
+            halvings = kCutHalvings;
+        }
+        if (few() >= KC - 2) {
+            guess = max(static_cast<uint32_t>(m - t), 1u << 12);
+            return best;
         }
     }
 }
@@ -1607,6 +1626,7 @@ __global__ __launch_bounds__(kLeadThreads) void fps_wide_kernel(
     __shared__ float4 cand_pos[2][kWave];
     __shared__ int cand_key[2][kWave];
     __shared__ int bounds[NF];
+    __shared__ int ties[NF];  // smallest index left out at the bound itself (0: not known)
     // Per 4 steps the packed lanes and the chosen key of the first of them;
     // the leader's other lanes write the padding behind the rows, so that
     // one store without an exec mask hits distinct addresses.
@@ -1758,7 +1778,7 @@ __global__ __launch_bounds__(kLeadThreads) void fps_wide_kernel(
     // The leader's ring store: lanes 0 and 1 the row, the others the padding.
     const int ring_at = lane < 2 ? lane : kLeadRing / 4 * 2 + lane - 2;
     const int ring_row = lane < 2 ? 2 : 0;
-    uint32_t cut_guess = 1u << 21;
+    uint32_t cut_guess = 1u << 21, tie_guess = 1u << 12;
     int64_t step = 1;
     int parity = 0;
     for (;;) {
@@ -1791,7 +1811,7 @@ __global__ __launch_bounds__(kLeadThreads) void fps_wide_kernel(
             };
             const bool has1 = (cut.first >> lane) & 1u;
             const bool has2 = (cut.second >> lane) & 1u;
-            int count, bound;
+            int count, bound, tied = 0;
             // A lane that holds the largest distance three times may keep
             // back its smallest index: then as without a cut.
             if (cut.first != 0 && ballot(d3 == top) == 0) {
@@ -1807,25 +1827,42 @@ __global__ __launch_bounds__(kLeadThreads) void fps_wide_kernel(
                 }
                 bound = wave_max_i32_l63(has2 ? d3 : has1 ? d2 : d1);
             } else {
-                // No cut (more than KC points share the largest distance, or
-                // none can be sampled): the follower's best point alone, the
-                // smallest index among the largest distances, and that
-                // distance as the bound: no later step of the run can take a
-                // key at it.
-                int j = INT_MAX;
+                // No cut (many points share the largest distance, or none can
+                // be sampled): those of the smallest indices among them, by
+                // a cut of the indices, that distance as the bound, and the
+                // smallest index left out, up to which the run may go on at
+                // that distance.
+                constexpr int kNone = 1 << 16;  // above every index
+                int i1 = kNone, i2 = kNone, i3 = kNone;
+#pragma unroll 8
                 for (int t = 0; t < tiles; ++t) {
                     const int q = pos0 + t * kWave + lane;
-                    j = f2i(md[q]) == top ? min(j, static_cast<int>(index_of[q])) : j;
+                    const int j = f2i(md[q]) == top ? static_cast<int>(index_of[q]) : kNone;
+                    i3 = min(i3, max(i2, j));
+                    i2 = min(i2, max(i1, j));
+                    i1 = min(i1, j);
                 }
-                j = wave_min(j);
-                const int f = min(j, n - 1);  // a follower without points: any point
-                if (lane == 0) put(0, top, make_float4(p[3 * f], p[3 * f + 1], p[3 * f + 2], 0.f), j);
-                count = 1;
+                const int least = wave_min(i1);
+                const KeyCut low = cut_top_keys<KC>(kNone - i1, kNone - i2, kNone - least, tie_guess);
+                const bool low1 = (low.first >> lane) & 1u;
+                const bool low2 = (low.second >> lane) & 1u;
+                auto point = [&](int j) {  // (a follower without points: any point)
+                    const float* r = p + 3 * min(j, n - 1);
+                    return make_float4(r[0], r[1], r[2], 0.f);
+                };
+                const int n1 = __popcll(low.first);
+                count = n1 + __popcll(low.second);
+                if (low1) put(lanes_below(low.first), top, point(i1), i1);
+                if (low2) put(n1 + lanes_below(low.second), top, point(i2), i2);
                 bound = top;
+                tied = wave_min(low2 ? i3 : low1 ? i2 : i1);
             }
             if (lane >= count && lane < KC)  // unfilled slots never win a step
                 put(lane, INT_MIN, make_float4(0.f, 0.f, 0.f, 0.f), INT_MAX);
-            if (lane == 0) bounds[wave] = bound;
+            if (lane == 0) {
+                bounds[wave] = bound;
+                ties[wave] = tied;
+            }
         }
         __syncthreads();  // candidates and bounds published; the last run applied
         if (done[parity]) break;  // uniform: written by the leader before this barrier
@@ -1858,6 +1895,35 @@ __global__ __launch_bounds__(kLeadThreads) void fps_wide_kernel(
                 __hip_atomic_store(&marks[lane == 0 ? 0 : lane + (lane == 1)], base + taken,
                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 block_key = wv;
+            }
+            // At the largest bound itself the run goes on, a step at a time,
+            // while the chosen candidate's index is below every one left out
+            // at that distance (lattices: thousands of points at one distance,
+            // and runs of one step otherwise).
+            if (wv == maxb) {
+                int tied = INT_MAX;
+#pragma unroll
+                for (int w = 0; w < NF; ++w) tied = bounds[w] == maxb ? min(tied, ties[w]) : tied;
+                const int steps = uniform(static_cast<int>(rest < kLeadRing ? rest : kLeadRing));
+                int in_block = ((taken - 1) & 3) + 1;  // steps in `packed`
+                while (taken < steps && wv == maxb && wave_min(cmd == wv ? cidx : INT_MAX) < uniform(tied)) {
+                    if (in_block == 4) {  // its row and the count, as above
+                        ring[ring_at + ((taken >> 2) - 1) * ring_row] = lane == 0 ? packed : static_cast<uint32_t>(block_key);
+                        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+                        __hip_atomic_store(&marks[lane == 0 ? 0 : lane + (lane == 1)], base + taken,
+                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        packed = 0;
+                        in_block = 0;
+                        block_key = wv;
+                    }
+                    int one = 1;
+                    uint32_t chosen = 0;
+                    lead_block(cmd, wv, one, chosen, sh, mine.x, mine.y, mine.z, -cidx, maxb);
+                    packed |= chosen << (8 * in_block);
+                    ++in_block;
+                    ++taken;
+                    wv = wave_max_i32_l63(cmd);
+                }
             }
             // The last block's row (full or partial), then the count and the
             // run's end in one store.

@@ -77,6 +77,45 @@ def test_one_cloud_over_the_chip_with_hard_cuts_matches_oracle(cuda_device, kind
     np.testing.assert_array_equal(got.cpu().numpy(), O.fps(xyz, npoint, 3, skip))
 
 
+@pytest.mark.parametrize("n,side", [(8193, 4), (9000, 10), (16384, 13), (24576, 29)])
+def test_lattices_beyond_8192_points(cuda_device, n, side):
+    """Runs that go on through points at one distance: the indices, and a time
+    below that of the kernel that takes one step at a time whatever the data (it
+    was up to twice that when each such step cost an exchange)."""
+    import mps_pointops as mp
+    from mps_pointops import _native
+
+    g = torch.Generator().manual_seed(n)
+    xyz = torch.randint(0, side, (2, n, 3), generator=g).float()
+    x, npoint = xyz.cuda(), 1000
+    got = mp.furthest_point_sample(x, npoint, 3)
+    np.testing.assert_array_equal(got.cpu().numpy(), O.fps(xyz, npoint, 3))
+    ptr, out_ptr = (torch.tensor([0, m, 2 * m], device="cuda") for m in (n, npoint))
+    starts = torch.full((2,), 3, device="cuda")
+    out = torch.empty(2 * npoint, dtype=torch.long, device="cuda")
+    scratch = torch.empty(2 * n, device="cuda")
+
+    def stepwise():
+        _native.call("pointops_fps_flat", x.data_ptr(), ptr.data_ptr(), out_ptr.data_ptr(),
+                     starts.data_ptr(), out.data_ptr(), scratch.data_ptr(), 2, 2 * n, n,
+                     _native.stream(x.device))
+
+    times = []
+    for call in (stepwise, lambda: mp.furthest_point_sample(x, npoint, 3)):
+        begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        call()
+        each = []
+        for _ in range(5):
+            begin.record()
+            call()
+            end.record()
+            end.synchronize()
+            each.append(begin.elapsed_time(end))
+        times.append(min(each))
+    assert torch.equal(out.view(2, -1) - torch.tensor([[0], [n]], device="cuda"), got)
+    assert times[1] < times[0]
+
+
 def test_threads_sampling_clouds_of_different_sizes(cuda_device):
     """The kernel's dynamic LDS differs per call, its limit belongs to the
     process: calls of several threads leave each other's alone."""
