@@ -10,23 +10,31 @@
 // on the matrix cores.  For D = 3 the operands are split into two bf16 parts
 // and all the products and a three-part norm are the 16 slots of one
 // v_mfma_f32_32x32x16_bf16; other widths take the coordinates, relative to a
-// centre and scaled, in f16.  |s + |q|^2 - d| <= E, with d the exact kernels'
-// rounded squared distance and E = err (|q| + max |r|)^2 (see screen_error).
+// centre and scaled, in f16.  With d the exact kernels' rounded squared
+// distance, |s + |q|^2 - d| <= 2 E |q|^2 + 2 E |r|^2 (see screen_error).  Each
+// reference carries its own part of that, so that one far from the others
+// loosens nothing but its own bound: s +- 2 E |r|^2 is the norm taken 1 +- 2 E
+// times, which is a slot of the product for D = 3.
 //
-// Pass 1 keeps, per query, the minima of 128 groups of references: one
-// v_min3 for two pairs.  K groups hold K distinct references, so the K-th
-// smallest minimum T bounds the K-th smallest d by T + |q|^2 + E, and every
-// neighbour has s <= T + 2E.  Pass 2 repeats the products and lists the
-// references at or below that (about K + K^2 / 256 of them, plus those within
-// 2E).  The listed references' distances are then computed as the searches
+// Pass 1 keeps, per query, the minima of s + 2 E |r|^2 over 128 groups of
+// references: one v_min3 for two pairs.  K groups hold K distinct references,
+// so the K-th smallest minimum T bounds the K-th smallest d by T + |q|^2 + 2 E
+// |q|^2, and every neighbour has s - 2 E |r|^2 <= T + 4 E |q|^2.  Pass 2 repeats
+// the products and lists the references at or below that (about K + K^2 / 256
+// of them, plus those within the error).  The listed references' distances are then computed as the searches
 // define them, and ranked by (distance, index): the results are the other
 // kernels' bit for bit.  Consecutive references fall into different groups,
 // so an order that puts neighbours next to each other does not spoil T.
 //
+// References that are not finite or too far for the operands' ranges are left
+// out: they lie beyond every reach that a served query may have.  (One such
+// reference, or one point at 20 beside 32 unit cubes of 4096, left nearly every
+// query of its cloud over when the bound took the cloud's largest norm: 390 to
+// 430 us at config 2's shape, now 41 to 62.)
+//
 // A query that the screen cannot serve (more than kScreenCap references
-// listed, as among many copies of one point; a coordinate that is not finite
-// or beyond 2^50 in its cloud) is searched by one wave over all references,
-// inside the same launch.
+// listed, as among many copies of one point; not finite or beyond 2^48 itself)
+// is searched by one wave over all references, inside the same launch.
 //
 // What bounds it: not the products (134 M pairs at config 2 are 5500 cycles a
 // block) but the phases around them, in cycles of a block at 32 x 1024 queries
@@ -58,7 +66,12 @@ constexpr int kScreenGroups = 128;  // minima per query
 constexpr int kScreenCap = 128;     // listed references per query
 constexpr int kScreenMaxK = 64;
 constexpr int kGroupStride = 72;    // floats between groups: 8 groups x 8 queries hit 64 banks
-constexpr float kScreenMaxSq = 1.2676506e30f;  // 2^100: squares of sums stay finite
+constexpr float kScreenMaxSq = 1.2676506e30f;      // 2^100: squares of sums stay finite
+constexpr float kScreenMaxQuerySq = 7.9228163e28f;  // 2^96, and
+constexpr float kScreenMaxReach = 3.1691265e29f;    // 2^98: see kernel
+constexpr float kScreenMaxRow = 65000.f;            // scaled: f16, and
+constexpr float kScreenMaxQuery = 32000.f;          // twice that for -2 q
+constexpr float kScreenMaxReachF16 = 1e9f;          // below (65000 - 32000)^2
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -67,7 +80,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 struct ScreenLayout {
     uint4* frag;    // per tile and k-step: 64 lanes x 8 bf16 or f16
     float* norm;    // D != 3: |r|^2 per tile row (+inf behind the last reference)
-    float* far_sq;  // per tile: largest |r|^2 (+inf: not to be screened)
+    float* far_sq;  // per tile: largest |r|^2, with the sign set where a row is left out
 };
 
 // Tiles are numbered by segment: segment b's begin at lo / 32 + b, where lo is
@@ -91,8 +104,8 @@ size_t screen_layout(int64_t rows, int64_t batch, int64_t D, ScreenLayout* L, ch
     return frag + norm + static_cast<size_t>(tiles) * sizeof(float);
 }
 
-// The relative error of the screen, against (|q| + max |r|)^2, which is at
-// least |q - r|^2 and four times |q| |r|.
+// The relative error E of the screen: |s + |q|^2 - d| <= E (|q| + |r|)^2, which
+// is at least |q - r|^2 and four times |q| |r|, and at most 2 |q|^2 + 2 |r|^2.
 // D = 3: a two-part operand is within 2^-16 of the float (relative), so the
 // doubled products of a pair are within 4 x 2^-16 |q| |r|, a quarter of which
 // counts: 2^-16; 16 terms summed in float32, 2^-23 each (allowing for
@@ -100,17 +113,22 @@ size_t screen_layout(int64_t rows, int64_t batch, int64_t D, ScreenLayout* L, ch
 // Others: an f16 operand is within 2^-11, so the doubled products are within
 // 4 x 2^-11 |q| |r|: 2^-11; D terms at 2^-23 and 2 (D + 6) 2^-24 for the norms
 // and the exact chain.  (Coordinates below f16's normal range lose at most
-// 2^-25 of the scaled unit each: screen_slack.)
+// 2^-25 of the scaled unit each, at most `lost` (|q| + |r|) in all; for a row,
+// lost |r| <= 1e-5 |r|^2 + lost^2 / 4e-5, whose first part is counted here.)
 __host__ __device__ inline float screen_error(int D) {
-    return D == 3 ? 2.3e-5f : 4.8828125e-4f * 1.02f + static_cast<float>(D + 6) * 3.6e-7f;
+    return D == 3 ? 2.3e-5f : 4.8828125e-4f * 1.02f + static_cast<float>(D + 6) * 3.6e-7f + 5e-6f;
 }
+// bf16 bits of 2 E for D = 3, 0.5 % up (of which rounding |r|^2 takes 0.2 %).
+constexpr uint32_t kScreenError3 = 0x3842u;
 // Absolute slack, in the scale of s: operands and products below the normal
-// ranges, and exact distances (of unscaled coordinates) below float32's, each
-// of whose roundings may be off by 2^-149.
-__host__ __device__ inline float screen_slack(int D, float span, float scale) {
+// ranges (far: the largest |r|), and exact distances (of unscaled coordinates)
+// below float32's, each of whose roundings may be off by 2^-149.
+__host__ __device__ inline float screen_slack(int D, float q, float far, float scale) {
     if (D == 3) return 1e-30f;
     const float tiny = scale * 5.3e-23f;  // 2^-74
-    return 1e-30f + span * static_cast<float>(D) * 1.2e-7f + static_cast<float>(2 * D) * (tiny * tiny);
+    const float lost = static_cast<float>(D) * 1.2e-7f;
+    return 1e-30f + lost * q + fminf(lost * far, lost * lost * 2.5e4f) +
+           static_cast<float>(2 * D) * (tiny * tiny);
 }
 
 // bf16 parts of a float, rounded to nearest: v = hi + lo to 2^-18.
@@ -139,20 +157,52 @@ __device__ __forceinline__ uint4 f16_frag(const float (&f)[8]) {
     return __builtin_bit_cast(uint4, v);
 }
 
+// The value of the lane whose number differs in the bits X, within a group of 8.
+template <int X>
+__device__ __forceinline__ int xor8(int v) {
+    constexpr int kQuadXor3 = 0x1B;
+    if constexpr (X == 1) return dpp<kDppQuadXor1>(v);
+    else if constexpr (X == 2) return dpp<kDppQuadXor2>(v);
+    else if constexpr (X == 3) return dpp<kQuadXor3>(v);
+    else if constexpr (X == 7) return dpp<kDppRowHalfMirror>(v);
+    else return xor8<7 - X>(dpp<kDppRowHalfMirror>(v));
+}
+template <int X>
+__device__ __forceinline__ int after8(uint32_t key, int i) {
+    const uint32_t other = static_cast<uint32_t>(xor8<X>(static_cast<int>(key)));
+    return other < key || (other == key && (i ^ X) < i) ? 1 : 0;
+}
+// Rank of a lane's key among its group of 8 lanes, equal keys by lane.
+__device__ __forceinline__ int rank8(uint32_t key, int i) {
+    return after8<1>(key, i) + after8<2>(key, i) + after8<3>(key, i) + after8<4>(key, i) +
+           after8<5>(key, i) + after8<6>(key, i) + after8<7>(key, i);
+}
+
+// Of the two middle values of eight the one nearer to 0 (0 if neither is
+// finite): with up to half of the eight somewhere else -- padding, strays --
+// it lies among the others unless those are nearer to the origin.
+__device__ __forceinline__ float nearer(float lower, float upper) {
+    const float c = fabsf(upper) < fabsf(lower) ? upper : lower;
+    return isfinite(c) ? c : 0.f;
+}
+
 // Centre of a 3-D segment for the screen (its coordinates are taken relative
-// to it, which keeps E small for clouds far from the origin): the mean of 8
-// points spread over it.  Any point serves; 0 if a coordinate is not finite.
-__device__ __forceinline__ void screen_centre(const float* __restrict__ ref, int64_t n, float (&c)[3]) {
-    float s[3] = {0.f, 0.f, 0.f};
+// to it, which keeps E small for clouds far from the origin): per axis a middle
+// one of 8 points spread over it.  Any point serves.  One wave, a lane per
+// value; every wave of a launch computes the same for a segment.
+__device__ __forceinline__ void screen_centre(const float* __restrict__ ref, int64_t n, int lane, float (&c)[3]) {
+    const int i = lane & 7;
+    const float v = ref[3 * ((n * i) >> 3) + min(lane >> 3, 2)];
+    const uint32_t bits = static_cast<uint32_t>(f2i(v));
+    const uint32_t key = v != v ? 0xFFFFFFFFu : bits ^ ((bits >> 31) != 0 ? 0xFFFFFFFFu : 0x80000000u);
+    const int rank = rank8(key, i);
+    const uint64_t lower = ballot(rank == 3), upper = ballot(rank == 4);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const float* p = ref + 3 * ((n * i) >> 3);
-        s[0] += p[0];
-        s[1] += p[1];
-        s[2] += p[2];
+    for (int a = 0; a < 3; ++a) {
+        const uint64_t group = uint64_t(0xFF) << (8 * a);
+        c[a] = nearer(i2f(readlane(f2i(v), static_cast<int>(__builtin_ctzll(lower & group)))),
+                      i2f(readlane(f2i(v), static_cast<int>(__builtin_ctzll(upper & group)))));
     }
-#pragma unroll
-    for (int a = 0; a < 3; ++a) c[a] = isfinite(s[a]) ? s[a] * 0.125f : 0.f;
 }
 
 // Eight dimensions from d0 of a row (0 behind the last).
@@ -171,32 +221,60 @@ __device__ __forceinline__ void load8(const float* __restrict__ r, int d0, int D
     }
 }
 
-// Centre and scale of a feature segment, from 8 rows spread over it: their
-// mean (any point serves; 0 where it is not finite) to centre[], 0 behind D, and the
-// power of two that takes the largest difference between their coordinates to
-// [4, 8).  f16 reaches 8000 times further, and a row beyond that is not
-// screened.  One wave, lane l for dimensions l and l + 64; every wave of a
-// launch computes the same values for a segment.
+// The middle one nearer to 0 of eight values (NaN counts as +inf).
+__device__ __forceinline__ float middle_of(const float (&v)[8]) {
+    float w[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) w[i] = v[i] == v[i] ? v[i] : INFINITY;
+    auto order = [&](int i, int j) {
+        const float a = w[i], b = w[j];
+        w[i] = fminf(a, b);
+        w[j] = fmaxf(a, b);
+    };
+    // Batcher's odd-even merge sort.
+    order(0, 1); order(2, 3); order(4, 5); order(6, 7);
+    order(0, 2); order(1, 3); order(4, 6); order(5, 7);
+    order(1, 2); order(5, 6);
+    order(0, 4); order(1, 5); order(2, 6); order(3, 7);
+    order(2, 4); order(3, 5);
+    order(1, 2); order(3, 4); order(5, 6);
+    return nearer(w[3], w[4]);
+}
+
+// Centre and scale of a feature segment, from 8 rows spread over it: per
+// dimension a middle value to centre[] (any serves), 0 behind D, and the power
+// of two that takes the middle one of the rows' largest differences from it
+// (of those that are not 0: repeated rows and padding) to [4, 8).  f16 reaches
+// 8000 times further, and a row beyond that is not screened.  One wave, lane l
+// for dimensions l and l + 64; every wave of a launch computes the same values
+// for a segment.
 constexpr int kScreenMaxD = 128;
 __device__ __forceinline__ float screen_frame(const float* __restrict__ ref, int64_t n, int D, int lane,
                                               float* centre) {
-    float most = 0.f;
+    float most[8] = {};
     for (int t = lane; t < D; t += kWave) {
         float v[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[i] = ref[((n * i) >> 3) * D + t];
-        float sum = v[0];
+        const float c = middle_of(v);
+        centre[t] = c;
 #pragma unroll
-        for (int i = 1; i < 8; ++i) {
-            sum = sum + v[i];
-            most = fmaxf(most, fabsf(v[i] - v[0]));
-        }
-        centre[t] = isfinite(sum) ? sum * 0.125f : 0.f;
+        for (int i = 0; i < 8; ++i) most[i] = fmaxf(most[i], fabsf(v[i] - c));  // (ignores NaN)
     }
     for (int t = D + lane; t < kScreenMaxD; t += kWave) centre[t] = 0.f;
-    most = wave_max(most);  // (NaN is ignored here and found in its own row)
-    if (!(most > 1e-25f && most < 1e25f)) return 1.f;
-    const int e = ((f2i(most) >> 23) & 0xFF) - 127;  // most in [2^e, 2^(e+1))
+    float mine = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float m = wave_max(most[i]);
+        mine = (lane & 7) == i ? m : mine;
+    }
+    const bool some = mine > 1e-25f && mine < 1e25f;
+    const int rank = rank8(some ? static_cast<uint32_t>(f2i(mine)) : 0xFFFFFFFFu, lane & 7);
+    const int count = __popcll(ballot(some) & 0xFF);
+    if (count == 0) return 1.f;
+    const uint64_t at = ballot(rank == (count - 1) / 2) & 0xFF;
+    const int bits = readlane(f2i(mine), static_cast<int>(__builtin_ctzll(at)));
+    const int e = ((bits >> 23) & 0xFF) - 127;  // in [2^e, 2^(e+1))
     return i2f((2 - e + 127) << 23);
 }
 
@@ -226,10 +304,10 @@ __device__ __forceinline__ ScreenSegment screen_segment(const int64_t* __restric
 }
 
 // Half (lane / 32) of a 3-D reference's slots, its coordinates relative to the
-// centre: h, h, l, l of the coordinates, then the norm; a row behind the last
-// reference is 0 with an infinite norm.  `sq`: its squared norm.
-__device__ __forceinline__ uint4 ref_frag3(float x, float y, float z, bool valid, int half, float& sq) {
-    sq = x * x + y * y + z * z;
+// centre: h, h, l, l of the coordinates, the norm, and the norm once more for
+// its part of the error bound; a row that is not `screened` is 0 with an
+// infinite norm.  `sq`: its squared norm.
+__device__ __forceinline__ uint4 ref_frag3(float x, float y, float z, float sq, bool screened, int half) {
     uint32_t h[3], l[3], nh, nm, nl;
     bf16_split(x, h[0], l[0]);
     bf16_split(y, h[1], l[1]);
@@ -237,20 +315,18 @@ __device__ __forceinline__ uint4 ref_frag3(float x, float y, float z, bool valid
     nh = bf16_bits(sq);
     bf16_split(sq - bf16_value(nh), nm, nl);
     uint32_t v[8] = {h[0], h[1], h[2], h[0], h[1], h[2], l[0], l[1]};
-    const uint32_t w[8] = {l[2], l[0], l[1], l[2], nh, nm, nl, 0};
+    const uint32_t w[8] = {l[2], l[0], l[1], l[2], nh, nm, nl, nh};
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         v[i] = half ? w[i] : v[i];
-        v[i] = valid ? v[i] : (half && i == 4 ? 0x7F80u : 0u);
+        v[i] = screened ? v[i] : (half && i == 4 ? 0x7F80u : 0u);
     }
     return pack8(v);
 }
 
-// A valid row's part in its tile's or cloud's largest squared norm: +inf where
-// it is not to be screened (NaN compares false).
-__device__ __forceinline__ float far_of(float sq, bool valid) {
-    return valid ? (sq < kScreenMaxSq ? sq : INFINITY) : 0.f;
-}
+// Whether a row or query is screened: finite, and close enough for the squares
+// of sums to stay finite (NaN compares false).
+__device__ __forceinline__ bool near_enough(float sq) { return sq < kScreenMaxSq; }
 
 // One wave per tile: the references' fragments, norms and largest norm.
 // Lane l holds row l % 32 and dimensions 8 (l / 32) .. + 7 of each k-step.
@@ -276,10 +352,14 @@ __global__ __launch_bounds__(kPrepThreads) void screen_prep_kernel(
     const bool valid = s.at + row < s.n;
     const float* r = ref + (s.lo + (valid ? s.at + row : 0)) * D;
     float sq = 0.f;
+    bool screened;
     if constexpr (D3) {
         float c[3];
-        screen_centre(ref + 3 * s.lo, s.n, c);
-        L.frag[t * kWave + lane] = ref_frag3(r[0] - c[0], r[1] - c[1], r[2] - c[2], valid, half, sq);
+        screen_centre(ref + 3 * s.lo, s.n, lane, c);
+        const float x = r[0] - c[0], y = r[1] - c[1], z = r[2] - c[2];
+        sq = x * x + y * y + z * z;
+        screened = valid && near_enough(sq);
+        L.frag[t * kWave + lane] = ref_frag3(x, y, z, sq, screened, half);
     } else {
         // Coordinates relative to the segment's centre, scaled.
         const bool vec = D % 4 == 0 && reinterpret_cast<uintptr_t>(ref) % 16 == 0;
@@ -296,15 +376,19 @@ __global__ __launch_bounds__(kPrepThreads) void screen_prep_kernel(
             for (int i = 0; i < 8; ++i) {
                 f[i] = valid ? (f[i] - o[i]) * scale : 0.f;  // (0 behind D)
                 sq = sq + f[i] * f[i];
-                if (!(fabsf(f[i]) < 65000.f)) sq = INFINITY;  // beyond f16, or NaN
+                if (!(fabsf(f[i]) < kScreenMaxRow)) sq = INFINITY;  // beyond f16, or NaN
             }
             L.frag[(t * steps + k) * kWave + lane] = f16_frag(f);
         }
         sq = sq + __shfl_xor(sq, 32, kWave);
-        if (half == 0) L.norm[t * kTileRefs + row] = valid ? sq : INFINITY;
+        screened = valid && near_enough(sq);
+        if (!screened)  // no products with what f16 made of it
+            for (int k = 0; k < steps; ++k) L.frag[(t * steps + k) * kWave + lane] = make_uint4(0, 0, 0, 0);
+        if (half == 0) L.norm[t * kTileRefs + row] = screened ? sq : INFINITY;
     }
-    const float most = wave_max(far_of(sq, valid));
-    if (lane == 0) L.far_sq[t] = most;
+    const float most = wave_max(screened ? sq : 0.f);
+    const bool all = ballot(valid && !screened) == 0;
+    if (lane == 0) L.far_sq[t] = all ? most : -most;
 }
 
 struct ScreenArgs {
@@ -378,7 +462,7 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
     uint4 bq[kU][KS];
     float c[3] = {0.f, 0.f, 0.f};
     if constexpr (D3) {
-        if (n > 0) screen_centre(a.ref + 3 * ref0, n, c);
+        if (n > 0) screen_centre(a.ref + 3 * ref0, n, lane, c);
     }
     const bool vec = D % 4 == 0 && reinterpret_cast<uintptr_t>(a.query) % 16 == 0;
     const bool vec_rows = vec && reinterpret_cast<uintptr_t>(a.ref) % 16 == 0;
@@ -400,9 +484,10 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
             bf16_split(-2.f * x, h[0], l[0]);
             bf16_split(-2.f * y, h[1], l[1]);
             bf16_split(-2.f * z, h[2], l[2]);
-            // Slots: h, l, h, l against the references' h, h, l, l; 1 against the norm's parts.
+            // Slots: h, l, h, l against the references' h, h, l, l; 1 against
+            // the norm's parts, and 2 E against the norm once more.
             uint32_t v[8] = {h[0], h[1], h[2], l[0], l[1], l[2], h[0], h[1]};
-            const uint32_t w[8] = {h[2], l[0], l[1], l[2], 0x3F80u, 0x3F80u, 0x3F80u, 0};
+            const uint32_t w[8] = {h[2], l[0], l[1], l[2], 0x3F80u, 0x3F80u, 0x3F80u, kScreenError3};
 #pragma unroll
             for (int i = 0; i < 8; ++i) v[i] = half ? w[i] : v[i];
             bq[u][0] = pack8(v);
@@ -417,7 +502,7 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
                 for (int i = 0; i < 8; ++i) {
                     f[i] = (f[i] - o[i]) * scale;  // (0 behind D)
                     sq = sq + f[i] * f[i];
-                    if (!(fabsf(f[i]) < 32000.f)) sq = INFINITY;  // -2 f beyond f16, or NaN
+                    if (!(fabsf(f[i]) < kScreenMaxQuery)) sq = INFINITY;  // -2 f beyond f16, or NaN
                     f[i] = -2.f * f[i];
                 }
                 bq[u][k] = f16_frag(f);
@@ -427,16 +512,25 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
         if (wave == 0 && half == 0) norm_q[qi] = sq;
     }
     if (tid < kScreenQueries) count[tid] = 0;
-    float my_far = 0.f;  // without PREP: of the rows this lane has seen
+    // The wave's part of the largest |r|^2 (not needed for D3) and of whether
+    // a row is left out (the sign).
+    bool left_out = false;
     if constexpr (PREP) {
         float far_sq = 0.f;
-        for (int i = tid; i < tiles; i += kScreenThreads) far_sq = fmaxf(far_sq, a.L.far_sq[tile0 + i]);
+        for (int i = tid; i < tiles; i += kScreenThreads) {
+            const float v = a.L.far_sq[tile0 + i];
+            far_sq = fmaxf(far_sq, fabsf(v));
+            left_out = left_out || f2i(v) < 0;
+        }
         far_sq = wave_max(far_sq);
+        if (ballot(left_out) != 0) far_sq = -far_sq;
         if (lane == 0) far_red[wave] = far_sq;
     }
 
-    // The screen of one tile against the wave's queries: acc[u][i] is
-    // s of reference 8 (i / 4) + 4 half + i % 4 and query 32 (u0 + u) + col.
+    // The screen of one tile against the wave's queries: acc[u][i] is s, with
+    // the reference's part of the bound added (pass 1) or taken off (pass 2), of
+    // reference 8 (i / 4) + 4 half + i % 4 and query 32 (u0 + u) + col.
+    float norm_part = 1.f + 2.f * screen_error(D);  // (D3: a slot of the query's fragment)
     auto load = [&](int t, uint4 (&f)[KS], float4 (&nr)[D3 ? 1 : 4]) {
         if constexpr (!PREP) {  // the coordinates, for as_fragment
             const float* r = a.ref + 3 * (ref0 + min<int64_t>(t * kTileRefs + col, n - 1));
@@ -455,9 +549,11 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
     auto as_fragment = [&](int t, uint4& f) {
         if constexpr (!PREP) {
             const bool valid = t * kTileRefs + col < n;
-            float sq;
-            f = ref_frag3(i2f(f.x) - c[0], i2f(f.y) - c[1], i2f(f.z) - c[2], valid, half, sq);
-            my_far = fmaxf(my_far, far_of(sq, valid));
+            const float x = i2f(f.x) - c[0], y = i2f(f.y) - c[1], z = i2f(f.z) - c[2];
+            const float sq = x * x + y * y + z * z;
+            const bool screened = valid && near_enough(sq);
+            left_out = left_out || (valid && !screened);
+            f = ref_frag3(x, y, z, sq, screened, half);
         }
     };
     auto screen = [&](const uint4 (&f)[KS], const float4 (&nr)[D3 ? 1 : 4], f32x16 (&acc)[kU]) {
@@ -471,10 +567,10 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
             for (int u = 0; u < kU; ++u)
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
-                    acc[u][4 * g] = nr[g].x;
-                    acc[u][4 * g + 1] = nr[g].y;
-                    acc[u][4 * g + 2] = nr[g].z;
-                    acc[u][4 * g + 3] = nr[g].w;
+                    acc[u][4 * g] = nr[g].x * norm_part;
+                    acc[u][4 * g + 1] = nr[g].y * norm_part;
+                    acc[u][4 * g + 2] = nr[g].z * norm_part;
+                    acc[u][4 * g + 3] = nr[g].w * norm_part;
                 }
 #pragma unroll
             for (int k = 0; k < KS; ++k)
@@ -545,13 +641,17 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
             }
     }
     if constexpr (!PREP) {
-        my_far = wave_max(my_far);
-        if (lane == 0) far_red[wave] = my_far;
+        const bool any = ballot(left_out) != 0;
+        if (lane == 0) far_red[wave] = any ? -0.f : 0.f;
     }
     __syncthreads();  // minima, norms, largest norms, cleared counts
-    float far_sq = far_red[0];
+    float far_sq = 0.f;
+    left_out = false;
 #pragma unroll
-    for (int w = 1; w < kScreenWaves; ++w) far_sq = fmaxf(far_sq, far_red[w]);
+    for (int w = 0; w < kScreenWaves; ++w) {
+        far_sq = fmaxf(far_sq, fabsf(far_red[w]));
+        left_out = left_out || f2i(far_red[w]) < 0;
+    }
 
     // ---- the limit of each query: eight lanes per query, 16 groups each,
     // searched for the K-th smallest minimum.  Any threshold that K groups
@@ -613,18 +713,27 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
             }
         }
         if (part == 0) {
-            const float span = sqrtf(nq_sq) + sqrtf(far_sq);
-            const float e = screen_error(D) * (span * span) + screen_slack(D, span, scale);
-            // (In the coordinates' own scale, so that no distance overflows.)
+            const float e = 2.f * screen_error(D) * nq_sq + screen_slack(D, sqrtf(nq_sq), sqrtf(far_sq), scale);
+            const float reach = hi + e;  // K references are within it
+            // Rows left out lie beyond every reach that is allowed here: (2^50 -
+            // 2^48)^2 from such a query, or (65000 - 32000)^2 in one dimension.
+            // (Norms in the coordinates' own scale, so that no distance overflows.)
             const float back = 1.f / scale;
-            const bool served = qi < nq && nq_sq * back * back < kScreenMaxSq &&
-                                far_sq * back * back < kScreenMaxSq;
+            const bool served = qi < nq && nq_sq * back * back < kScreenMaxQuerySq &&
+                                (D3 || far_sq * back * back < kScreenMaxSq) &&
+                                (!left_out || (some >= static_cast<float>(K) &&
+                                               reach < (D3 ? kScreenMaxReach : kScreenMaxReachF16)));
             // (Finite, so that the rows behind the last, at +inf, are not listed.)
-            limit[qi] = served ? fminf(hi + 2.f * e - nq_sq, 3e38f) : -INFINITY;
+            limit[qi] = served ? fminf(reach + e - nq_sq, 3e38f) : -INFINITY;
             if (qi < nq && !served) count[qi] = kScreenCap + 1;
         }
     }
     __syncthreads();  // limits
+    norm_part = 1.f - 2.f * screen_error(D);
+    if constexpr (D3) {
+#pragma unroll
+        for (int u = 0; u < kU; ++u) bq[u][0].w ^= half ? 0x80000000u : 0u;  // - 2 E
+    }
 
     // ---- pass 2: the references within each query's limit
     {

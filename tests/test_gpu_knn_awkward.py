@@ -1,0 +1,81 @@
+"""Searches screened on the matrix cores over inputs that once made the screen
+useless: results against the scanning entry points, and times against the same
+search of ordinary input.  The times are minima of several calls and their limits
+lie well above what is measured (an order of magnitude below what they caught)."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# (B, M, N, D, k): config 2's search, a small one (no workspace), features
+SHAPES = [(32, 1024, 4096, 3, 16), (16, 512, 1024, 3, 16), (8, 1024, 2048, 64, 20)]
+
+
+def _best(call) -> float:
+    begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    for _ in range(3):
+        call()
+    times = []
+    for _ in range(5):
+        begin.record()
+        for _ in range(10):
+            call()
+        end.record()
+        end.synchronize()
+        times.append(begin.elapsed_time(end))
+    return min(times)
+
+
+def _cloud(shape):
+    B, M, N, D, k = shape
+    g = torch.Generator().manual_seed(N + D)
+    r = torch.rand(B, N, D, generator=g) if D == 3 else torch.randn(B, N, D, generator=g)
+    return r.cuda(), torch.randperm(N, generator=g)[:M].cuda(), k
+
+
+def _scan(q, r, k):
+    """The same search by the entry points' scan: more than 64 neighbours."""
+    from mps_pointops import _native
+
+    B, M, D = q.shape
+    wide = 65
+    dist = torch.empty(B, M, wide, device="cuda")
+    idx = torch.empty(B, M, wide, dtype=torch.long, device="cuda")
+    args = (q.data_ptr(), r.data_ptr(), dist.data_ptr(), idx.data_ptr(), B, M, r.shape[1])
+    if D == 3:
+        _native.call("pointops_knn3", *args, wide, _native.stream(q.device))
+    else:
+        _native.call("pointops_knn_feat", *args, D, wide, _native.stream(q.device))
+    return dist[..., :k], idx[..., :k]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("value", [20.0, 1e3, 1e6, 1e30, float("inf"), float("nan")])
+@pytest.mark.parametrize("at", [7, 0])
+def test_one_stray_reference_costs_itself(cuda_device, shape, value, at):
+    import mps_pointops as mp
+
+    r, pick, k = _cloud(shape)
+    pick = torch.where(pick == at, at + 1, pick)  # (the stray asks nothing)
+    q = r[:, pick].contiguous()
+    plain = _best(lambda: mp.knn(q, r, k))
+    r[:, at] = value
+    got = mp.knn(q, r, k)
+    want = _scan(q, r, k)
+    assert torch.equal(got[1], want[1])
+    assert torch.equal(got[0], want[0])
+    assert _best(lambda: mp.knn(q, r, k)) < 1.5 * plain
+
+
+@pytest.mark.parametrize("value", [50.0, float("nan")])
+def test_strays_of_ragged_clouds_cost_themselves(cuda_device, value):
+    from mps_pointops import flat
+
+    sizes = [20000, 15000, 25000]
+    x = torch.rand(sum(sizes), 3, generator=torch.Generator().manual_seed(1)).cuda()
+    ptr = torch.tensor([0, *sizes]).cumsum(0).cuda()
+    y = x.clone()
+    plain = _best(lambda: flat.knn_indices(x, y, ptr, ptr, 16))
+    x[::5000] = value
+    assert _best(lambda: flat.knn_indices(x, y, ptr, ptr, 16)) < 1.5 * plain
