@@ -30,11 +30,16 @@
 // out: they lie beyond every reach that a served query may have.  (One such
 // reference, or one point at 20 beside 32 unit cubes of 4096, left nearly every
 // query of its cloud over when the bound took the cloud's largest norm: 390 to
-// 430 us at config 2's shape, now 41 to 62.)
+// 430 us at config 2's shape, now 41 to 57.)
 //
-// A query that the screen cannot serve (more than kScreenCap references
-// listed, as among many copies of one point; not finite or beyond 2^48 itself)
-// is searched by one wave over all references, inside the same launch.
+// A query with more than kScreenCap references listed (copies of one point,
+// clusters tighter than E) or that the screen cannot serve (not finite or beyond
+// 2^48 itself) is left over: pass 2's hits once more, as bits, ranked by exact
+// distance 64 at a time in index order, inside the same launch.  One wave each
+// over every reference, eight queries in turn, took five times as long: half of
+// both clouds copies of one point 478 -> 80 us at config 2's shape, D = 64 features
+// in 16 clusters of 0.05 1019 -> 205 us (the scans that came before the screen: 77 and 355
+// us); half of them zeros, which tie as everyone's nearest, 1245 -> 394 (297).
 //
 // What bounds it: not the products (134 M pairs at config 2 are 5500 cycles a
 // block) but the phases around them, in cycles of a block at 32 x 1024 queries
@@ -178,6 +183,14 @@ __device__ __forceinline__ int rank8(uint32_t key, int i) {
            after8<5>(key, i) + after8<6>(key, i) + after8<7>(key, i);
 }
 
+// Row i of the eight that a segment of n rows is looked at by: spread over it,
+// in no common step (clouds may carry something every so many rows).
+__device__ __forceinline__ int64_t sample8(int64_t n, int i) {
+    constexpr uint64_t lo = 27329ull << 48 | 18553ull << 32 | 9719ull << 16 | 2039ull;   // of 65536
+    constexpr uint64_t hi = 60757ull << 48 | 51971ull << 32 | 43973ull << 16 | 35323ull;
+    return (n * static_cast<int64_t>(((i < 4 ? lo : hi) >> (16 * (i & 3))) & 0xFFFFu)) >> 16;
+}
+
 // Of the two middle values of eight the one nearer to 0 (0 if neither is
 // finite): with up to half of the eight somewhere else -- padding, strays --
 // it lies among the others unless those are nearer to the origin.
@@ -192,7 +205,7 @@ __device__ __forceinline__ float nearer(float lower, float upper) {
 // value; every wave of a launch computes the same for a segment.
 __device__ __forceinline__ void screen_centre(const float* __restrict__ ref, int64_t n, int lane, float (&c)[3]) {
     const int i = lane & 7;
-    const float v = ref[3 * ((n * i) >> 3) + min(lane >> 3, 2)];
+    const float v = ref[3 * sample8(n, i) + min(lane >> 3, 2)];
     const uint32_t bits = static_cast<uint32_t>(f2i(v));
     const uint32_t key = v != v ? 0xFFFFFFFFu : bits ^ ((bits >> 31) != 0 ? 0xFFFFFFFFu : 0x80000000u);
     const int rank = rank8(key, i);
@@ -255,7 +268,7 @@ __device__ __forceinline__ float screen_frame(const float* __restrict__ ref, int
     for (int t = lane; t < D; t += kWave) {
         float v[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = ref[((n * i) >> 3) * D + t];
+        for (int i = 0; i < 8; ++i) v[i] = ref[sample8(n, i) * D + t];
         const float c = middle_of(v);
         centre[t] = c;
 #pragma unroll
@@ -404,6 +417,81 @@ struct ScreenArgs {
     bool squared;  // dense: distances squared, not their roots
 };
 
+// ---- the queries the screen leaves over
+// Their references at or below the limit are found again as bits, kMaskTiles
+// tiles at a time in index order, and ranked 64 at a time (LeftList).
+constexpr int kMaskTiles = 126;
+constexpr int kMaskStride = kMaskTiles + 1;  // words per query: odd, no bank conflicts
+static_assert(kScreenQueries * kMaskStride <= kScreenQueries * kScreenCap, "masks fit the lists");
+constexpr int kLeftMany = 8;    // more candidates at once are sorted and merged
+constexpr int kLeftShares = 8;  // up to eight queries are searched by all waves, each a share
+
+__device__ __forceinline__ uint64_t shfl64(uint64_t v, int from) {
+    const uint32_t lo = __shfl(static_cast<int>(v), from, kWave), hi = __shfl(static_cast<int>(v >> 32), from, kWave);
+    return static_cast<uint64_t>(hi) << 32 | lo;
+}
+// One stage of a bitonic network on a word per lane: the lanes that differ in
+// bit j exchange, ascending where `up`.
+__device__ __forceinline__ uint64_t bitonic(uint64_t v, int j, bool up, int lane) {
+    const uint64_t other = shfl64(v, lane ^ j);
+    const bool least = ((lane & j) == 0) == up;
+    return (other < v) == least ? other : v;
+}
+
+// The nearest references of one query, (distance bits, index) words in order
+// over the lanes.  References are offered in index order, and only a distance
+// below `below` is ranked: at first the bound that pass 1 gave, then, with
+// K in the list, the K-th nearest so far (a later reference at that distance
+// is behind it).  A list of zeros ends its query, which is how copies of one
+// point are served.
+struct LeftList {
+    float d[1];
+    int i[1];
+    uint32_t below;
+
+    __device__ __forceinline__ void settle(int K) {
+        float last;
+        int at;
+        list_tail<1>(d, i, K, last, at);
+        if (at != -1) below = min(below, static_cast<uint32_t>(f2i(last)));
+    }
+    // Takes the nearest 64 of the list and of another, in order.
+    __device__ __forceinline__ void merge(uint64_t other, int lane) {
+        const uint64_t mine = static_cast<uint64_t>(static_cast<uint32_t>(f2i(d[0]))) << 32 | static_cast<uint32_t>(i[0]);
+        other = shfl64(other, kWave - 1 - lane);
+        uint64_t word = other < mine ? other : mine;
+#pragma unroll
+        for (int j = kWave / 2; j > 0; j >>= 1) word = bitonic(word, j, true, lane);
+        d[0] = i2f(static_cast<int>(word >> 32));
+        i[0] = static_cast<int>(word);
+    }
+    // This lane's reference, if `in`: its index and distance.
+    __device__ __forceinline__ void offer(bool in, int index, float dist, int K, int lane) {
+        const int key = f2i(dist);  // (NaN is above every bound)
+        uint64_t pending = ballot(in && static_cast<uint32_t>(key) < below);
+        if (pending == 0) return;
+        if (__popcll(pending) > kLeftMany) {
+            uint64_t word = static_cast<uint64_t>(static_cast<uint32_t>(key)) << 32 | static_cast<uint32_t>(index);
+            word = ((pending >> lane) & 1u) ? word : ~uint64_t(0);
+#pragma unroll
+            for (int k = 2; k <= kWave; k <<= 1)
+#pragma unroll
+                for (int j = k >> 1; j > 0; j >>= 1) word = bitonic(word, j, (lane & k) == 0, lane);
+            merge(word, lane);
+            settle(K);
+            return;
+        }
+        do {
+            const int src = __builtin_ctzll(pending);
+            pending &= pending - 1;
+            const int k = readlane(key, src);
+            if (static_cast<uint32_t>(k) >= below) continue;  // an earlier one lowered it
+            list_insert<1>(d, i, K, lane, i2f(k), readlane(index, src));
+            settle(K);
+        } while (pending != 0);
+    }
+};
+
 // KS k-steps (D <= 16 KS); D3: one fragment holds everything.  Eight waves,
 // each with an eighth of the tiles against all 64 queries (two columns of 32).
 // PREP: the fragments come from screen_prep_kernel; otherwise (D3 only) each
@@ -420,8 +508,10 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
     __shared__ __align__(16) uint32_t own_keys[D3 ? 4 : kScreenQueries * kScreenCap];
     __shared__ int count[kScreenQueries];
     __shared__ float limit[kScreenQueries];
+    __shared__ float within[kScreenQueries];  // no less than the K-th smallest distance
     __shared__ float norm_q[kScreenQueries];
     __shared__ float far_red[kScreenWaves];
+    __shared__ int left_q[kScreenQueries];
     __shared__ __align__(16) float centres[kScreenWaves][D3 ? 4 : kScreenMaxD];  // a copy per wave: no barrier
     // The exact phase: the listed references' keys (where the minima were, for
     // D3), and each wave's rows of 16 dimensions (where the minima were).
@@ -579,23 +669,24 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
                     acc[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16(f[k]), as_f16(bq[u][k]), acc[u], 0, 0, 0);
         }
     };
-    // The wave's tiles, kBatch at a time (the next ones requested before the
-    // current ones are used): use(j, t, acc) for t = t0 + kScreenWaves j, then
-    // flush(t0), for every batch.  Tiles behind the last are replaced by the
-    // wave's first; use() sees t.
-    auto walk = [&](auto use, auto flush) {
-        if (wave >= tiles) return;
+    // The wave's tiles of begin .. end - 1, kBatch at a time (the next ones
+    // requested before the current ones are used): use(j, t, acc) for t = t0 +
+    // kScreenWaves j, then flush(t0), for every batch.  Tiles behind the last
+    // are replaced by the wave's first; use() sees t.
+    auto walk = [&](int begin, int end, auto use, auto flush) {
+        const int t_first = begin + wave;
+        if (t_first >= end) return;
         uint4 f[kBatch][KS];
         float4 nr[kBatch][D3 ? 1 : 4];
         auto fetch = [&](int t0) {
 #pragma unroll
             for (int j = 0; j < kBatch; ++j) {
                 const int t = t0 + j * kScreenWaves;
-                load(t < tiles ? t : wave, f[j], nr[j]);
+                load(t < end ? t : t_first, f[j], nr[j]);
             }
         };
-        fetch(wave);
-        for (int t0 = wave; t0 < tiles; t0 += kBatch * kScreenWaves) {
+        fetch(t_first);
+        for (int t0 = t_first; t0 < end; t0 += kBatch * kScreenWaves) {
             uint4 cf[kBatch][KS];
             float4 cn[kBatch][D3 ? 1 : 4];
 #pragma unroll
@@ -610,12 +701,23 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
             for (int j = 0; j < kBatch; ++j) {
                 f32x16 acc[kU];
                 const int t = t0 + j * kScreenWaves;
-                as_fragment(t < tiles ? t : wave, cf[j][0]);
+                as_fragment(t < end ? t : t_first, cf[j][0]);
                 screen(cf[j], cn[j], acc);
                 use(j, t, acc);
             }
             flush(t0);
         }
+    };
+
+    // Bit i from the sign of limit - s (set: beyond it): a comparison and a
+    // select per bit wait for vcc each time (front end 367 -> 360 us, 3 ragged
+    // clouds of 20000 with K = 16 and their grouping 631 -> 613 us).
+    auto hits_of = [](float lim, const f32x16& acc) {
+        uint32_t h = 0;
+#pragma unroll
+        for (int i = 15; i >= 0; --i)
+            h = __builtin_amdgcn_alignbit(h, static_cast<uint32_t>(f2i(lim - acc[i])), 31);
+        return ~h & 0xFFFFu;
     };
 
     // ---- pass 1: group minima
@@ -625,7 +727,7 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
         for (int u = 0; u < kU; ++u)
 #pragma unroll
             for (int i = 0; i < 16; ++i) m[u][i] = INFINITY;
-        walk([&](int, int, const f32x16 (&acc)[kU]) {  // (a tile again changes no minimum)
+        walk(0, tiles, [&](int, int, const f32x16 (&acc)[kU]) {  // (a tile again changes no minimum)
 #pragma unroll
             for (int u = 0; u < kU; ++u)
 #pragma unroll
@@ -725,6 +827,7 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
                                                reach < (D3 ? kScreenMaxReach : kScreenMaxReachF16)));
             // (Finite, so that the rows behind the last, at +inf, are not listed.)
             limit[qi] = served ? fminf(reach + e - nq_sq, 3e38f) : -INFINITY;
+            within[qi] = served && some >= static_cast<float>(K) ? reach * 1.000001f * back * back : INFINITY;
             if (qi < nq && !served) count[qi] = kScreenCap + 1;
         }
     }
@@ -744,7 +847,7 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
         // lane and column with hits.
         constexpr int kWords = (kBatch + 1) / 2;
         uint32_t hit[kU][kWords] = {};
-        walk([&](int j, int t, const f32x16 (&acc)[kU]) {
+        walk(0, tiles, [&](int j, int t, const f32x16 (&acc)[kU]) {
             const bool real = t < tiles;
 #pragma unroll
             for (int u = 0; u < kU; ++u) {
@@ -752,16 +855,7 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
 #pragma unroll
                 for (int i = 1; i < 16; ++i) least = fminf(least, acc[u][i]);
                 uint32_t h = 0;
-                if (ballot(least <= lim[u]) != 0 && real) {
-                    // Bit i from the sign of limit - s (set: beyond it): a
-                    // comparison and a select per bit wait for vcc each time (front
-                    // end 367 -> 360 us, 3 ragged clouds of 20000 with K = 16 and
-                    // their grouping 631 -> 613 us).
-#pragma unroll
-                    for (int i = 15; i >= 0; --i)
-                        h = __builtin_amdgcn_alignbit(h, static_cast<uint32_t>(f2i(lim[u] - acc[u][i])), 31);
-                    h = ~h & 0xFFFFu;
-                }
+                if (ballot(least <= lim[u]) != 0 && real) h = hits_of(lim[u], acc[u]);
                 hit[u][j / 2] |= h << (16 * (j & 1));
             }
         }, [&](int t0) {
@@ -773,6 +867,11 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
                 for (int w = 0; w < kWords; ++w) n_hit += __popc(hit[u][w]);
                 at[u] = 0;
                 if (n_hit != 0) at[u] = atomicAdd(&count[32 * u + col], n_hit);
+                if (at[u] + n_hit > kScreenCap) {  // left over: no more of its hits
+                    lim[u] = -INFINITY;
+#pragma unroll
+                    for (int w = 0; w < kWords; ++w) hit[u][w] = 0;
+                }
             }
 #pragma unroll
             for (int u = 0; u < kU; ++u) {
@@ -784,13 +883,70 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
                         hit[u][w] &= hit[u][w] - 1;
                         // (Rows behind the last are at +inf, above every limit.)
                         const int t = t0 + (2 * w + (i >> 4)) * kScreenWaves;
-                        if (at[u] < kScreenCap) list[at[u]] = t * kTileRefs + 8 * ((i >> 2) & 3) + 4 * half + (i & 3);
+                        list[at[u]] = t * kTileRefs + 8 * ((i >> 2) & 3) + 4 * half + (i & 3);
                         ++at[u];
                     }
             }
         });
     }
     __syncthreads();  // lists
+
+    // This lane's reference row r against its query row q, as the searches
+    // define it (all lanes take part).
+    auto distance = [&](int64_t r, const float* q) -> float {
+        if constexpr (D3) {
+            const float* rr = a.ref + 3 * r;
+            return sqdist3(rr[0], rr[1], rr[2], q[0], q[1], q[2]);
+        } else if (vec_rows) {
+            // The 64 rows, 16 dimensions at a time, through LDS: four lanes
+            // read a row's 64 bytes together (a lane reading its own row
+            // would fetch each of its cache lines once per 16 bytes).
+            constexpr int kRow = 20;  // floats between rows: no bank conflicts
+            float4* const rows = reinterpret_cast<float4*>(groups + wave * kWave * kRow);
+            static_assert(kScreenWaves * kWave * kRow <= kScreenGroups * kGroupStride + 1024, "rows fit");
+            float d = 0.f;  // 0 + d0^2 = d0^2
+            const int part = lane & 3;
+            float4 next[4], qn[4];
+            const float* src[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                qn[k] = 4 * k < D ? *reinterpret_cast<const float4*>(q + 4 * k) : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int64_t other = __shfl(r, 16 * k + (lane >> 2), kWave);
+                src[k] = a.ref + other * D + 4 * part;
+                next[k] = 4 * part < D ? *reinterpret_cast<const float4*>(src[k]) : make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+            for (int d0 = 0; d0 < D; d0 += 16) {
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int k = 0; k < 4; ++k) rows[(16 * k + (lane >> 2)) * (kRow / 4) + part] = next[k];
+                __builtin_amdgcn_wave_barrier();
+                float4 x4[4], qc[4];  // (behind D: not used)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) x4[k] = rows[lane * (kRow / 4) + k];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    qc[k] = qn[k];
+                    if (d0 + 16 + 4 * part < D) next[k] = *reinterpret_cast<const float4*>(src[k] + d0 + 16);
+                    if (d0 + 16 + 4 * k < D) qn[k] = *reinterpret_cast<const float4*>(q + d0 + 16 + 4 * k);
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    if (d0 + 4 * k >= D) break;
+                    const float4 x = x4[k], y = qc[k];
+                    const float x0 = x.x - y.x, x1 = x.y - y.y, x2 = x.z - y.z, x3 = x.w - y.w;
+                    d = d + x0 * x0;
+                    d = d + x1 * x1;
+                    d = d + x2 * x2;
+                    d = d + x3 * x3;
+                }
+            }
+            return d;
+        } else {
+            return sqdist_nd(a.ref + r * D, q, D);
+        }
+    };
 
     // ---- exact distances: the wave's eight queries' lists end to end, a lane
     // per listed reference
@@ -816,57 +972,7 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
         const int slot = (q0 + i) * kScreenCap + (valid ? e - base : 0);
         const int64_t r = ref0 + (valid ? listed[slot] : 0);
         const float* q = a.query + (row0 + q0 + i) * D;
-        float d;
-        if constexpr (D3) {
-            const float* rr = a.ref + 3 * r;
-            d = sqdist3(rr[0], rr[1], rr[2], q[0], q[1], q[2]);
-        } else if (vec_rows) {
-            // The 64 rows, 16 dimensions at a time, through LDS: four lanes
-            // read a row's 64 bytes together (a lane reading its own row
-            // would fetch each of its cache lines once per 16 bytes).
-            constexpr int kRow = 20;  // floats between rows: no bank conflicts
-            float4* const rows = reinterpret_cast<float4*>(groups + wave * kWave * kRow);
-            static_assert(kScreenWaves * kWave * kRow <= kScreenGroups * kGroupStride + 1024, "rows fit");
-            d = 0.f;  // 0 + d0^2 = d0^2
-            const int part = lane & 3;
-            float4 next[4], qn[4];
-            const float* src[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                qn[k] = 4 * k < D ? *reinterpret_cast<const float4*>(q + 4 * k) : make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int64_t other = __shfl(r, 16 * k + (lane >> 2), kWave);
-                src[k] = a.ref + other * D + 4 * part;
-                next[k] = 4 * part < D ? *reinterpret_cast<const float4*>(src[k]) : make_float4(0.f, 0.f, 0.f, 0.f);
-            }
-            for (int d0 = 0; d0 < D; d0 += 16) {
-                __builtin_amdgcn_wave_barrier();
-#pragma unroll
-                for (int k = 0; k < 4; ++k) rows[(16 * k + (lane >> 2)) * (kRow / 4) + part] = next[k];
-                __builtin_amdgcn_wave_barrier();
-                float4 qc[4];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    qc[k] = qn[k];
-                    if (d0 + 16 + 4 * part < D) next[k] = *reinterpret_cast<const float4*>(src[k] + d0 + 16);
-                    if (d0 + 16 + 4 * k < D) qn[k] = *reinterpret_cast<const float4*>(q + d0 + 16 + 4 * k);
-                }
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    if (d0 + 4 * k >= D) break;
-                    const float4 x = rows[lane * (kRow / 4) + k];
-                    const float4 y = qc[k];
-                    const float x0 = x.x - y.x, x1 = x.y - y.y, x2 = x.z - y.z, x3 = x.w - y.w;
-                    d = d + x0 * x0;
-                    d = d + x1 * x1;
-                    d = d + x2 * x2;
-                    d = d + x3 * x3;
-                }
-            }
-        } else {
-            d = sqdist_nd(a.ref + r * D, q, D);
-        }
+        const float d = distance(r, q);
         if (valid) keys[slot] = static_cast<uint32_t>(f2i(d));
     }
     __builtin_amdgcn_wave_barrier();
@@ -907,26 +1013,118 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
             for (int s = K + col; s < a.K; s += 32) a.idx[(out0 + qi) * a.K + s] = -1;
     }
 
-    // ---- the queries left over: one wave each, over every reference
-    for (int qi = wave; qi < nq; qi += kScreenWaves) {
-        if (uniform(count[qi]) <= kScreenCap) continue;
-        const float* q = a.query + (row0 + qi) * D;
-        float ld[1] = {INFINITY};
-        int li[1] = {-1};
-        bool ok = true;
-        if constexpr (!D3 || FLAT)  // dense 3-D queries match at infinite distances
-            for (int t = 0; t < D; ++t) ok = ok && isfinite(q[t]);
-        if (ok)
-            scan_refs<1, D3, !D3 || FLAT>(q, a.ref + ref0 * D, static_cast<int>(n), D, a.K, lane, ld, li);
-        if (lane < a.K) {
-            const int64_t slot = (out0 + qi) * a.K + lane;
-            if constexpr (FLAT) {
-                a.idx[slot] = li[0] < 0 ? int64_t(-1) : ref0 + li[0];
-            } else {
-                a.dist[slot] = a.squared ? ld[0] : sqrtf(ld[0]);
-                a.idx[slot] = D3 ? static_cast<int64_t>(static_cast<uint32_t>(li[0]))
-                                 : (li[0] < 0 ? int64_t(-1) : int64_t(li[0]));
+    // ---- the queries left over
+    const bool mine_left = lane < nq && count[lane] > kScreenCap;
+    const uint64_t left = ballot(mine_left);  // the same in every wave
+    if (left == 0) return;
+    const int lefts = __popcll(left);
+    const int shares = lefts <= kScreenQueries / kLeftShares ? kLeftShares : 1;
+    if (wave == 0 && mine_left) left_q[lanes_below(left)] = lane;
+    __syncthreads();  // left_q; every wave has ranked: the lists and keys are free
+    // List `item` (a query and share; item % 8 is its wave): 64 keys, 64 indices.
+    auto keys_of = [&](int item) { return keys + item * kScreenCap + lane; };
+    for (int item = wave; item < lefts * shares; item += kScreenWaves) {
+        keys_of(item)[0] = 0x7F800000u;
+        keys_of(item)[kWave] = 0xFFFFFFFFu;
+    }
+    if (tiles == 0) __syncthreads();  // (else the last of the loop's)
+    for (int t0 = 0; t0 < tiles; t0 += kMaskTiles) {
+        const int t1 = min(t0 + kMaskTiles, tiles);
+        // The hits of these tiles, a word a query and tile; a query without a
+        // limit takes every reference.
+        uint16_t* const masks = reinterpret_cast<uint16_t*>(listed);
+        float lim[kU];
+        bool wanted[kU], every[kU];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            lim[u] = limit[32 * u + col];
+            wanted[u] = (left >> (32 * u + col)) & 1u;
+            every[u] = lim[u] == -INFINITY;
+        }
+        walk(t0, t1, [&](int, int t, const f32x16 (&acc)[kU]) {
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+                const uint32_t h = hits_of(lim[u], acc[u]);
+                if (wanted[u] && t < t1)
+                    masks[((32 * u + col) * kMaskStride + t - t0) * 2 + half] = static_cast<uint16_t>(every[u] ? 0xFFFFu : h);
             }
+        }, [](int) {});
+        __syncthreads();  // masks
+        for (int item = wave; item < lefts * shares; item += kScreenWaves) {
+            const int qi = uniform(left_q[item / shares]), share = item % shares;
+            const float* q = a.query + (row0 + qi) * D;
+            // Nothing is at a distance from a query that is not finite (dense
+            // 3-D searches match at infinite distances).
+            bool never = false;
+            for (int t = lane; t < D; t += kWave) never = never || (D3 && !FLAT ? q[t] != q[t] : !isfinite(q[t]));
+            if (ballot(never) != 0) continue;
+            LeftList list;
+            list.d[0] = i2f(static_cast<int>(keys_of(item)[0]));
+            list.i[0] = static_cast<int>(keys_of(item)[kWave]);
+            list.below = static_cast<uint32_t>(uniform(min(f2i(within[qi]), D3 && !FLAT ? 0x7F800000 : 0x7F7FFFFF))) + 1u;
+            list.settle(a.K);
+            // Lane l looks at tiles 2 l and 2 l + 1; then the pairs with hits
+            // one by one, lane l at reference l, their hits queued over the
+            // lanes until 64 are there.
+            const uint32_t* words = listed + qi * kMaskStride;
+            const int pairs = (t1 - t0 + 1) / 2;
+            auto word_of = [&](int t) { return t < t1 - t0 ? words[t] : 0u; };
+            uint64_t todo = ballot(lane < pairs && lane % shares == share &&
+                                   (word_of(2 * lane) | word_of(2 * lane + 1)) != 0);
+            int queued = 0, queue = 0;
+            auto rank = [&]() {
+                const bool in = lane < queued;
+                const int at = in ? queue : 0;
+                list.offer(in, at, distance(ref0 + at, q), a.K, lane);
+                queued = 0;
+            };
+            while (todo != 0 && list.below != 0) {
+                const int pair = static_cast<int>(__builtin_ctzll(todo));
+                todo &= todo - 1;
+                const int j = (t0 + 2 * pair) * kTileRefs + lane;
+                const uint32_t word = word_of(2 * pair + half);
+                const int bit = 16 * ((lane >> 2) & 1) + 4 * ((lane >> 3) & 3) + (lane & 3);
+                const bool hit = ((word >> bit) & 1u) != 0 && j < n;
+                const uint64_t hits = ballot(hit);
+                const int more = __popcll(hits);
+                // Every lane sends its index to a lane of its own: the hits in
+                // order from lane `queued` on, around the end.
+                const int to = (queued + (hit ? lanes_below(hits) : more + lanes_below(~hits))) & (kWave - 1);
+                const int sent = __builtin_amdgcn_ds_permute(to << 2, j);
+                const int place = (lane - queued) & (kWave - 1);
+                const bool fits = place < more && place + queued < kWave;
+                queue = fits ? sent : queue;
+                const int total = queued + more;
+                queued = min(total, kWave);
+                if (total >= kWave) {
+                    rank();
+                    queue = sent;  // the others, from lane 0 on
+                    queued = total - kWave;
+                }
+            }
+            if (queued != 0 && list.below != 0) rank();
+            keys_of(item)[0] = static_cast<uint32_t>(f2i(list.d[0]));
+            keys_of(item)[kWave] = static_cast<uint32_t>(list.i[0]);
+        }
+        __syncthreads();  // masks read, lists written
+    }
+    for (int r = wave; r < lefts; r += kScreenWaves) {
+        const int qi = uniform(left_q[r]);
+        LeftList list;
+        list.d[0] = i2f(static_cast<int>(keys_of(r * shares)[0]));
+        list.i[0] = static_cast<int>(keys_of(r * shares)[kWave]);
+        for (int s = 1; s < shares; ++s)
+            list.merge(static_cast<uint64_t>(keys_of(r * shares + s)[0]) << 32 | keys_of(r * shares + s)[kWave], lane);
+        if (lane >= a.K) continue;
+        const float d = list.d[0];
+        const int at = list.i[0];
+        const int64_t slot = (out0 + qi) * a.K + lane;
+        if constexpr (FLAT) {
+            a.idx[slot] = at < 0 ? int64_t(-1) : ref0 + at;
+        } else {
+            a.dist[slot] = a.squared ? d : sqrtf(d);
+            a.idx[slot] = D3 ? static_cast<int64_t>(static_cast<uint32_t>(at))
+                             : (at < 0 ? int64_t(-1) : int64_t(at));
         }
     }
 }

@@ -79,3 +79,65 @@ def test_strays_of_ragged_clouds_cost_themselves(cuda_device, value):
     plain = _best(lambda: flat.knn_indices(x, y, ptr, ptr, 16))
     x[::5000] = value
     assert _best(lambda: flat.knn_indices(x, y, ptr, ptr, 16)) < 1.5 * plain
+
+
+def _copies(r, g):
+    r[:, r.shape[1] // 2:] = 0.0
+    return r
+
+
+def _clusters(r, g):
+    B, N, D = r.shape
+    centre = torch.randn(B, 16, D, generator=g).cuda()
+    which = torch.randint(0, 16, (B, N, 1), generator=g).cuda().expand(-1, -1, D)
+    return centre.gather(1, which) + 0.05 * r
+
+
+def _lattice(r, g):
+    return (r * 4).round()
+
+
+@pytest.mark.parametrize("shape", SHAPES + [(1, 700, 20000, 3, 64), (2, 70, 9000, 3, 1), (1, 100, 5000, 40, 33)])
+@pytest.mark.parametrize("kind", [_copies, _clusters, _lattice])
+@pytest.mark.parametrize("few", [False, True])
+def test_queries_left_over(cuda_device, shape, kind, few):
+    """More references within the limit than a list holds, for all or a few of
+    a block's queries (which the waves then share), over one and several ranges
+    of tiles."""
+    from mps_pointops import ops
+
+    r, pick, k = _cloud(shape)
+    g = torch.Generator().manual_seed(7)
+    r = kind(r, g).contiguous()
+    q = r[:, pick].contiguous()
+    if few:  # only every 50th query lies among them
+        keep = torch.arange(q.shape[1], device="cuda") % 50 == 0
+        q = torch.where(keep[:, None], q, q + 3.0 + torch.rand(q.shape, generator=g).cuda())
+    from mps_pointops import _native
+
+    want = _scan(q, r, k)
+    dist, idx = torch.empty_like(want[0]).contiguous(), torch.empty_like(want[1]).contiguous()
+    B, M, D = q.shape
+    N = r.shape[1]
+    ws = torch.empty(_native.size_query("pointops_knn_screen_workspace_bytes", B, N, D),
+                     dtype=torch.uint8, device="cuda")
+    _native.call("pointops_knn_screen", q.data_ptr(), r.data_ptr(), dist.data_ptr(), idx.data_ptr(),
+                 ws.data_ptr(), B, M, N, D, k, _native.stream(q.device))
+    assert torch.equal(idx, want[1])
+    assert torch.equal(dist, want[0])
+    got = ops.knn(q, r, k)  # whichever entry point serves it
+    assert torch.equal(got[1], want[1])
+    assert torch.equal(got[0], want[0])
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("kind", [_copies, _clusters])
+def test_queries_left_over_take_no_longer_than_a_scan(cuda_device, shape, kind):
+    """Against the scan of the same pairs (more than 64 neighbours), which needs
+    several times as long as the search of ordinary input."""
+    import mps_pointops as mp
+
+    r, pick, k = _cloud(shape)
+    r = kind(r, torch.Generator().manual_seed(7)).contiguous()
+    q = r[:, pick].contiguous()
+    assert _best(lambda: mp.knn(q, r, k)) < _best(lambda: _scan(q, r, k))
