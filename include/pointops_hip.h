@@ -126,8 +126,8 @@ hipError_t pointops_knn3_grid(const float *query, const float *ref, float *dist,
  * dist2 (B,M) the squared distance fl32((dx^2 + dy^2) + dz^2), idx (B,M)
  * the smallest index attaining it, identical to the linear scan, for
  * finite coordinates.  Queries whose nearest reference lies more than a few
- * cells away are finished inside the call by a linear scan over their
- * cloud.  `workspace`: pointops_knn3_grid_workspace_bytes(B, M, N); N >= 1,
+ * cells away are finished inside the call by the matrix-core screen
+ * (pointops_nearest3_screen).  `workspace`: pointops_knn3_grid_workspace_bytes(B, M, N); N >= 1,
  * B <= 65535.
  * Accelerates chamfer.py:122-158 for large clouds. */
 hipError_t pointops_nearest3_grid(const float *query, const float *ref, float *dist2,

@@ -30,7 +30,7 @@
 namespace pointops {
 
 hipError_t knn3_screen_rows(const float* query, const float* ref, float* dist, int64_t* idx,
-                            void* workspace, int64_t B, int64_t M, int64_t QS, int64_t N, int64_t K,
+                            void* workspace, int64_t B, int64_t M, int64_t N, int64_t K,
                             hipStream_t stream);
 
 namespace {
@@ -371,7 +371,7 @@ hipError_t launch_dense(const float* query, const float* ref, float* dist, int64
     // us, 16 x 256 x 384, k = 32 26 against 53 us.  Its screen loosens with
     // the cloud's extent against its spacing, so large clouds are scanned.
     if (DIM3 && N >= (K <= 8 ? 512 : 256) && N <= kScreenMaxRefs && K <= 64 && lane_grid_ok)
-        return knn3_screen_rows(query, ref, dist, idx, nullptr, B, M, M, N, K, stream);
+        return knn3_screen_rows(query, ref, dist, idx, nullptr, B, M, N, K, stream);
     if (DIM3 && K <= 32 && lane_grid_ok) {
         if (K <= 8) return launch_lane<8>(query, ref, dist, idx, B, M, N, K, stream);
         if (K <= 16) return launch_lane<16>(query, ref, dist, idx, B, M, N, K, stream);

@@ -34,6 +34,11 @@
 #include "pointops_hip.h"
 
 namespace pointops {
+
+hipError_t nearest3_screen_listed(const float* query, const float* ref, const int* count, const int* list,
+                                  float* dist2, int64_t* idx, void* workspace, int64_t B, int64_t M,
+                                  int64_t N, hipStream_t stream);
+
 namespace {
 
 constexpr int kGridPrepThreads = 256;
@@ -43,9 +48,19 @@ constexpr int kGridMaxDim = 1024;
 constexpr int kGridSearchWaves = 4;
 constexpr int kGridCap = 16;  // buffered candidates per lane
 constexpr int kGridMaxGrow = 8;  // box faces a quad may add before its query is listed (measured best of 4-24)
-// Nearest mode: box faces a lane may add before its query is left to the
-// fill pass (measured best of 4-24).
+// Nearest mode leaves a query to the screen (knn_screen.hip) after this many box
+// faces; up to kGridQuitRefs references, where the screen's share is cheap,
+// already after kGridQuitGrow faces, kGridQuitScan scanned references (cells
+// crowded because a stray point stretches the grid, or at a dense spot) or an
+// empty first box.  One direction of 32 x 8192, a tenth of the queries far: 445
+// us after 6 faces, 327 after 4, 264 after 2, 241 after 1, but then 8 x 16384
+// uniform points take 137 instead of 106 us, as do 10^5 after 2 (241 instead
+// of 85); crowded by a stray 541 without a limit, 385 with 512, where 10^5
+// points on a sphere need more (284 instead of 118).
 constexpr int kGridNearestGrow = 6;
+constexpr int64_t kGridQuitRefs = 1 << 15;
+constexpr int kGridQuitGrow = 2;
+constexpr int kGridQuitScan = 512;
 constexpr int kGridQueriesPerWave = kWave / 4;  // one quad of lanes per query
 constexpr uint32_t kGridMatchLimit = 0x7F800001u;  // keys below: finite or +inf
 // Listed queries (those the search leaves to a linear pass) are compacted in
@@ -708,7 +723,7 @@ __device__ __forceinline__ float box_bound(const GridParams& P, float h, const f
 template <int S>
 __global__ __launch_bounds__(kGridSearchWaves * kWave) void knn3_grid_kernel(
     const float* __restrict__ query, GridLayout L, float* __restrict__ out_dist,
-    int64_t* __restrict__ out_idx, int64_t B, int64_t M, int64_t N, int K, int nearest) {
+    int64_t* __restrict__ out_idx, int64_t B, int64_t M, int64_t N, int K, int nearest, int max_grow, int max_scan) {
     constexpr int KMAX = 4 * S;
     __shared__ uint2 bufs[kGridSearchWaves][kGridCap][kWave];
     const int lane = lane_id();
@@ -763,7 +778,7 @@ __global__ __launch_bounds__(kGridSearchWaves * kWave) void knn3_grid_kernel(
     };
 
     const bool qfinite = finite3(q[0], q[1], q[2]);
-    // Queries left to the linear pass: the whole wave when the batch has
+    // Queries left to the linear pass (nearest mode: the screen): the whole wave when the batch has
     // non-finite references or the wave a non-finite query, else the quads
     // whose walk needs more faces than the mode allows.
     const bool full = P.nonfinite > 0 || ballot(active && !qfinite) != 0;
@@ -794,6 +809,7 @@ __global__ __launch_bounds__(kGridSearchWaves * kWave) void knn3_grid_kernel(
             ne = ok ? off[c1 + 1] : 0;
         };
         bool done = !active, want = false;
+        int scanned = 0;
         if (!done) fetch();
         for (;;) {
             drain(want);
@@ -816,7 +832,7 @@ __global__ __launch_bounds__(kGridSearchWaves * kWave) void knn3_grid_kernel(
                     done = true;
                 } else if (qc != 0) {
                     want = true;  // merge first, then check again
-                } else if (grow == (nearest ? kGridNearestGrow : kGridMaxGrow)) {
+                } else if (grow == max_grow || (max_scan != 0 && tau == ~0ull)) {
                     listed = true;
                     done = true;
                 } else {
@@ -849,6 +865,10 @@ __global__ __launch_bounds__(kGridSearchWaves * kWave) void knn3_grid_kernel(
             for (int u = 0; u < 8; ++u) rv[u] = srt[min(base + 4 * u, last)];
             admit8s(rv, has ? e - base : 0);
             if (has) p += 32;
+            if (max_scan != 0 && has && (scanned += 32) > max_scan) {
+                listed = done = true;
+                p = e;
+            }
         }
     }
     // Every query's mark at its sorted position (in q_rank, dead since the
@@ -1046,85 +1066,9 @@ __global__ __launch_bounds__(kGateThreads) void ball_grid_choice_kernel(GridLayo
     *choice = grid ? 1 : 0;
 }
 
-// Nearest mode's second pass over each cloud's list of the queries the grid
-// search left (their nearest reference is several cells away): one
-// workgroup per 64 listed queries, lane = query, 8 waves splitting the
-// references (batches of 8 read with wide scalar loads, the next batch
-// requested before the current one is scanned), the best (squared distance,
-// smallest index) per wave combined in LDS.  Workgroups past the list's end
-// return at once.
-constexpr int kFillThreads = 512;
-
 __global__ void grid_zero_kernel(int* __restrict__ p, int64_t n) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i < n) p[i] = 0;
-}
-
-__global__ __launch_bounds__(kFillThreads) void nearest_fill_kernel(
-    const float* __restrict__ query, const float* __restrict__ ref,
-    const int* __restrict__ miss_count, const int* __restrict__ miss_list,
-    float* __restrict__ dist2, int64_t* __restrict__ idx, int64_t M, int64_t N) {
-    constexpr int NWF = kFillThreads / kWave;
-    __shared__ int keys[NWF][kWave];
-    __shared__ int ids[NWF][kWave];
-    const int lane = lane_id();
-    const int wave = uniform(threadIdx.x / kWave);
-    const int64_t groups = (M + kWave - 1) / kWave;
-    const int64_t b = blockIdx.x / groups;
-    const int64_t first = (blockIdx.x - b * groups) * kWave;
-    const int64_t count = miss_count[b];
-    if (first >= count) return;  // uniform over the workgroup, before any barrier
-    const bool active = first + lane < count;
-    const int64_t row = b * M + miss_list[b * M + (active ? first + lane : first)];
-    const float qx = query[3 * row], qy = query[3 * row + 1], qz = query[3 * row + 2];
-    const float* rp = ref + 3 * b * N;
-    const int64_t per = (N + NWF - 1) / NWF;
-    const int64_t lo = min(N, wave * per), hi = min(N, lo + per);
-    int best = 0x7FFFFFFF, bi = 0;
-    const int64_t hi8 = lo + ((hi - lo) & ~int64_t(7));
-    float cur[24], nxt[24];
-    if (lo < hi8) {
-#pragma unroll
-        for (int t = 0; t < 24; ++t) cur[t] = rp[3 * lo + t];
-    }
-    for (int64_t j = lo; j < hi8; j += 8) {  // ascending: the first minimum is kept
-        if (j + 8 < hi8) {
-#pragma unroll
-            for (int t = 0; t < 24; ++t) nxt[t] = rp[3 * (j + 8) + t];
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int key = f2i(sqdist3(cur[3 * u], cur[3 * u + 1], cur[3 * u + 2], qx, qy, qz));
-            if (key < best) {
-                best = key;
-                bi = static_cast<int>(j + u);
-            }
-        }
-#pragma unroll
-        for (int t = 0; t < 24; ++t) cur[t] = nxt[t];
-    }
-    for (int64_t j = hi8; j < hi; ++j) {
-        const int key = f2i(sqdist3(rp[3 * j], rp[3 * j + 1], rp[3 * j + 2], qx, qy, qz));
-        if (key < best) {
-            best = key;
-            bi = static_cast<int>(j);
-        }
-    }
-    keys[wave][lane] = best;
-    ids[wave][lane] = bi;
-    __syncthreads();
-    if (wave != 0 || !active) return;
-    int k = keys[0][lane], i = ids[0][lane];
-#pragma unroll
-    for (int w = 1; w < NWF; ++w) {
-        const int kk = keys[w][lane], ii = ids[w][lane];
-        if (kk < k || (kk == k && ii < i)) {
-            k = kk;
-            i = ii;
-        }
-    }
-    dist2[row] = i2f(k);
-    idx[row] = i;
 }
 
 // After the search, per cloud with listed queries: blocks [0, ltiles)
@@ -1527,6 +1471,12 @@ void grid_list(const GridLayout& L, int64_t B, int64_t M, int64_t N, bool boxes,
                        dim3(kGridPrepThreads), 0, stream, L, N, M);
 }
 
+// Where nearest mode's screen of the listed queries has its workspace, behind
+// the grid's.
+size_t nearest_screen_offset(int64_t B, int64_t M, int64_t N) {
+    return (grid_layout_bytes(B, M, N, nullptr, nullptr) + 15) / 16 * 16;
+}
+
 // Search launch shape: 16 queries per wave, kGridSearchWaves waves per
 // workgroup, a multiple of 8 workgroups for the XCD-local deal.
 bool grid_search_grid(int64_t B, int64_t M, dim3& grid) {
@@ -1543,7 +1493,7 @@ extern "C" {
 
 size_t pointops_knn3_grid_workspace_bytes(int64_t B, int64_t M, int64_t N) {
     if (B <= 0 || M <= 0 || N <= 0) return 0;
-    return grid_layout_bytes(B, M, N, nullptr, nullptr);
+    return nearest_screen_offset(B, M, N) + pointops_knn_screen_workspace_bytes(B, N, 3);
 }
 
 hipError_t pointops_knn3_grid(const float* query, const float* ref, float* dist, int64_t* idx,
@@ -1563,13 +1513,13 @@ hipError_t pointops_knn3_grid(const float* query, const float* ref, float* dist,
     const dim3 block(kGridSearchWaves * kWave);
     const int k = static_cast<int>(K);
     if (K <= 4)
-        hipLaunchKernelGGL((knn3_grid_kernel<1>), grid, block, 0, stream, query, L, dist, idx, B, M, N, k, 0);
+        hipLaunchKernelGGL((knn3_grid_kernel<1>), grid, block, 0, stream, query, L, dist, idx, B, M, N, k, 0, kGridMaxGrow, 0);
     else if (K <= 8)
-        hipLaunchKernelGGL((knn3_grid_kernel<2>), grid, block, 0, stream, query, L, dist, idx, B, M, N, k, 0);
+        hipLaunchKernelGGL((knn3_grid_kernel<2>), grid, block, 0, stream, query, L, dist, idx, B, M, N, k, 0, kGridMaxGrow, 0);
     else if (K <= 16)
-        hipLaunchKernelGGL((knn3_grid_kernel<4>), grid, block, 0, stream, query, L, dist, idx, B, M, N, k, 0);
+        hipLaunchKernelGGL((knn3_grid_kernel<4>), grid, block, 0, stream, query, L, dist, idx, B, M, N, k, 0, kGridMaxGrow, 0);
     else
-        hipLaunchKernelGGL((knn3_grid_kernel<8>), grid, block, 0, stream, query, L, dist, idx, B, M, N, k, 0);
+        hipLaunchKernelGGL((knn3_grid_kernel<8>), grid, block, 0, stream, query, L, dist, idx, B, M, N, k, 0, kGridMaxGrow, 0);
     grid_list(L, B, M, N, true, stream);
     const dim3 listed(static_cast<uint32_t>(B * ((M + kWave - 1) / kWave)));
     const dim3 lblock(kListedWaves * kWave);
@@ -1596,18 +1546,20 @@ hipError_t pointops_nearest3_grid(const float* query, const float* ref, float* d
     grid_layout_bytes(B, M, N, &L, static_cast<char*>(workspace));
     grid_build(query, ref, L, B, M, N, 1, 0.f, 1, stream);
     grid_list_zero(L, B, stream);
+    const bool quit = N <= kGridQuitRefs;
     hipLaunchKernelGGL((knn3_grid_kernel<1>), grid, dim3(kGridSearchWaves * kWave), 0, stream, query,
-                       L, dist2, idx, B, M, N, 1, 1);
+                       L, dist2, idx, B, M, N, 1, 1, quit ? kGridQuitGrow : kGridNearestGrow, quit ? kGridQuitScan : 0);
     grid_list(L, B, M, N, false, stream);
-    const int64_t fill_blocks = B * ((M + kWave - 1) / kWave);
-    hipLaunchKernelGGL(nearest_fill_kernel, dim3(static_cast<uint32_t>(fill_blocks)),
-                       dim3(kFillThreads), 0, stream, query, ref, L.list_total, L.list, dist2, idx,
-                       M, N);
-    return hipGetLastError();
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) return err;
+    return nearest3_screen_listed(query, ref, L.list_total, L.list, dist2, idx,
+                                  static_cast<char*>(workspace) + nearest_screen_offset(B, M, N), B, M, N,
+                                  stream);
 }
 
 size_t pointops_ball_query_grid_workspace_bytes(int64_t B, int64_t Q, int64_t P) {
-    return pointops_knn3_grid_workspace_bytes(B, Q, P);
+    if (B <= 0 || Q <= 0 || P <= 0) return 0;
+    return grid_layout_bytes(B, Q, P, nullptr, nullptr);
 }
 
 }  // extern "C"
@@ -1663,7 +1615,8 @@ hipError_t pointops_ball_query_grid_f32(const float* queries, const float* point
 }
 
 size_t pointops_ball_query_auto_workspace_bytes(int64_t B, int64_t Q, int64_t P) {
-    return pointops_knn3_grid_workspace_bytes(B, Q, P);
+    if (B <= 0 || Q <= 0 || P <= 0) return 0;
+    return grid_layout_bytes(B, Q, P, nullptr, nullptr);
 }
 
 hipError_t pointops_ball_query_auto_f32(const float* queries, const float* points, int64_t* idx,

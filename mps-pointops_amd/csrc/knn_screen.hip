@@ -345,8 +345,8 @@ __device__ __forceinline__ bool near_enough(float sq) { return sq < kScreenMaxSq
 // Lane l holds row l % 32 and dimensions 8 (l / 32) .. + 7 of each k-step.
 template <bool D3, bool FLAT>
 __global__ __launch_bounds__(kPrepThreads) void screen_prep_kernel(
-    const float* __restrict__ ref, const int64_t* __restrict__ ptr, ScreenLayout L, int64_t batch,
-    int64_t N, int64_t tiles, int D, int steps) {
+    const float* __restrict__ ref, const int64_t* __restrict__ ptr, const int* __restrict__ wanted,
+    ScreenLayout L, int64_t batch, int64_t N, int64_t tiles, int D, int steps) {
     const int lane = lane_id();
     const int64_t t = static_cast<int64_t>(blockIdx.x) * (kPrepThreads / kWave) + uniform(threadIdx.x / kWave);
     if (t >= tiles) return;
@@ -356,6 +356,7 @@ __global__ __launch_bounds__(kPrepThreads) void screen_prep_kernel(
     } else {  // every cloud has the same number of tiles here
         const int64_t per = (N + kTileRefs - 1) / kTileRefs;
         s.b = t / per;
+        if (wanted != nullptr && wanted[s.b] == 0) return;  // no query of the cloud is searched
         s.lo = s.b * N;
         s.n = N;
         s.at = (t - s.b * per) * kTileRefs;
@@ -412,7 +413,9 @@ struct ScreenArgs {
     float* dist;           // dense outputs
     int64_t* idx;          // dense or flat indices
     ScreenLayout L;
-    int64_t batch, M, N, QS;  // dense: queries of a cloud lie QS rows apart
+    int64_t batch, M, N;
+    const int* list;        // LIST: per cloud, rows of its queries to search (M apart)
+    const int* list_count;
     int D, K;
     bool squared;  // dense: distances squared, not their roots
 };
@@ -496,8 +499,8 @@ struct LeftList {
 // each with an eighth of the tiles against all 64 queries (two columns of 32).
 // PREP: the fragments come from screen_prep_kernel; otherwise (D3 only) each
 // wave makes them from the coordinates as it goes, twice, which for small
-// clouds costs less than a launch.
-template <int KS, bool D3, bool FLAT, bool PREP>
+// clouds costs less than a launch.  LIST: only the listed queries of each cloud.
+template <int KS, bool D3, bool FLAT, bool PREP, bool LIST>
 __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(const ScreenArgs a) {
     constexpr int kBatch = D3 ? 4 : KS <= 4 ? 2 : 1;  // tiles in flight
     constexpr int kU = 2;               // columns of 32 queries
@@ -524,13 +527,13 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
     const int col = lane & 31, half = lane >> 5;
     const int D = a.D;
     // This block's queries and their cloud's references.
-    int64_t row0, ref0, n, tile0, out0, b;
+    int64_t row0, ref0, n, tile0, b;
     int nq;
     if constexpr (FLAT) {
         const ScreenSegment s = screen_segment(a.ptr_y, a.batch, blockIdx.x, kScreenQueries);
         if (s.at >= s.n) return;  // a number no segment uses (uniform)
         b = s.b;
-        row0 = out0 = s.lo + s.at;
+        row0 = s.lo + s.at;
         nq = static_cast<int>(min<int64_t>(kScreenQueries, s.n - s.at));
         ref0 = a.ptr_x[b];
         n = a.ptr_x[b + 1] - ref0;
@@ -539,12 +542,16 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
         const CloudBlock cb = cloud_block(static_cast<uint32_t>((a.M + kScreenQueries - 1) / kScreenQueries));
         b = cb.b;
         const int64_t m0 = static_cast<int64_t>(cb.x) * kScreenQueries;
-        row0 = out0 = b * a.QS + m0;
-        nq = static_cast<int>(min<int64_t>(kScreenQueries, a.M - m0));
+        row0 = b * a.M + m0;
+        const int64_t rows = LIST ? a.list_count[b] : a.M;
+        if (LIST && m0 >= rows) return;  // (uniform)
+        nq = static_cast<int>(min<int64_t>(kScreenQueries, rows - m0));
         ref0 = b * a.N;
         n = a.N;
         tile0 = b * ((n + kTileRefs - 1) / kTileRefs);
     }
+    // Row of query qi, of the queries and of the outputs.
+    auto row_of = [&](int qi) -> int64_t { return LIST ? b * a.M + a.list[row0 + qi] : row0 + qi; };
     const int tiles = static_cast<int>((n + kTileRefs - 1) / kTileRefs);
     const int K = static_cast<int>(min<int64_t>(a.K, n));
 
@@ -565,7 +572,7 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
         const int qi = 32 * u + col;
-        const float* q = a.query + (row0 + (qi < nq ? qi : 0)) * D;
+        const float* q = a.query + row_of(qi < nq ? qi : 0) * D;
         float sq = 0.f;
         if constexpr (D3) {
             const float x = q[0] - c[0], y = q[1] - c[1], z = q[2] - c[2];
@@ -971,7 +978,7 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
         }
         const int slot = (q0 + i) * kScreenCap + (valid ? e - base : 0);
         const int64_t r = ref0 + (valid ? listed[slot] : 0);
-        const float* q = a.query + (row0 + q0 + i) * D;
+        const float* q = a.query + row_of(q0 + i) * D;
         const float d = distance(r, q);
         if (valid) keys[slot] = static_cast<uint32_t>(f2i(d));
     }
@@ -999,7 +1006,7 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
                         before_mine(k.z, l.z, o + 2) + before_mine(k.w, l.w, o + 3);
             }
             if (rank < K) {
-                const int64_t slot = (out0 + qi) * a.K + rank;
+                const int64_t slot = row_of(qi) * a.K + rank;
                 if constexpr (FLAT) {
                     a.idx[slot] = ref0 + at;
                 } else {
@@ -1010,7 +1017,7 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
             }
         }
         if constexpr (FLAT)  // a segment of fewer than K references
-            for (int s = K + col; s < a.K; s += 32) a.idx[(out0 + qi) * a.K + s] = -1;
+            for (int s = K + col; s < a.K; s += 32) a.idx[row_of(qi) * a.K + s] = -1;
     }
 
     // ---- the queries left over
@@ -1052,7 +1059,7 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
         __syncthreads();  // masks
         for (int item = wave; item < lefts * shares; item += kScreenWaves) {
             const int qi = uniform(left_q[item / shares]), share = item % shares;
-            const float* q = a.query + (row0 + qi) * D;
+            const float* q = a.query + row_of(qi) * D;
             // Nothing is at a distance from a query that is not finite (dense
             // 3-D searches match at infinite distances).
             bool never = false;
@@ -1118,7 +1125,7 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
         if (lane >= a.K) continue;
         const float d = list.d[0];
         const int at = list.i[0];
-        const int64_t slot = (out0 + qi) * a.K + lane;
+        const int64_t slot = row_of(qi) * a.K + lane;
         if constexpr (FLAT) {
             a.idx[slot] = at < 0 ? int64_t(-1) : ref0 + at;
         } else {
@@ -1129,9 +1136,9 @@ __global__ __launch_bounds__(kScreenThreads, D3 ? 4 : 2) void knn_screen_kernel(
     }
 }
 
-template <int KS, bool D3, bool FLAT, bool PREP = true>
+template <int KS, bool D3, bool FLAT, bool PREP = true, bool LIST = false>
 hipError_t launch_search(const ScreenArgs& a, int64_t blocks, hipStream_t stream) {
-    hipLaunchKernelGGL((knn_screen_kernel<KS, D3, FLAT, PREP>), dim3(static_cast<uint32_t>(blocks)),
+    hipLaunchKernelGGL((knn_screen_kernel<KS, D3, FLAT, PREP, LIST>), dim3(static_cast<uint32_t>(blocks)),
                        dim3(kScreenThreads), 0, stream, a);
     return hipGetLastError();
 }
@@ -1154,10 +1161,10 @@ hipError_t launch_prep(const ScreenArgs& a, int64_t ref_rows, hipStream_t stream
     const dim3 grid(static_cast<uint32_t>((tiles + kPrepWaves - 1) / kPrepWaves));
     if (a.D == 3)
         hipLaunchKernelGGL((screen_prep_kernel<true, FLAT>), grid, dim3(kPrepThreads), 0, stream, a.ref,
-                           a.ptr_x, a.L, a.batch, a.N, tiles, a.D, 1);
+                           a.ptr_x, a.list_count, a.L, a.batch, a.N, tiles, a.D, 1);
     else
         hipLaunchKernelGGL((screen_prep_kernel<false, FLAT>), grid, dim3(kPrepThreads), 0, stream, a.ref,
-                           a.ptr_x, a.L, a.batch, a.N, tiles, a.D, screen_kernel_steps(a.D));
+                           a.ptr_x, a.list_count, a.L, a.batch, a.N, tiles, a.D, screen_kernel_steps(a.D));
     return hipGetLastError();
 }
 
@@ -1193,9 +1200,8 @@ namespace pointops {
 
 // The dense 3-D search in two launches: knn3_screen_prepare (the references'
 // fragments into `workspace`, pointops_knn_screen_workspace_bytes(B, N, 3)
-// bytes) and knn3_screen_rows (the queries -- M rows per cloud whose rows,
-// queries and both outputs, lie QS rows apart -- over a workspace filled for
-// the same references, B and N, or without one).
+// bytes) and knn3_screen_rows (the queries, over a workspace filled for the same
+// references, B and N, or without one).
 hipError_t knn3_screen_prepare(const float* ref, void* workspace, int64_t B, int64_t N, hipStream_t stream) {
     if (B < 1 || N < 1 || workspace == nullptr || N > INT32_MAX - kWave || !screen_fits(B, B * N, B))
         return hipErrorInvalidValue;
@@ -1209,9 +1215,9 @@ hipError_t knn3_screen_prepare(const float* ref, void* workspace, int64_t B, int
 }
 
 hipError_t knn3_screen_rows(const float* query, const float* ref, float* dist, int64_t* idx,
-                            void* workspace, int64_t B, int64_t M, int64_t QS, int64_t N, int64_t K,
+                            void* workspace, int64_t B, int64_t M, int64_t N, int64_t K,
                             hipStream_t stream) {
-    if (B < 1 || M < 1 || QS < M || K < 1 || K > kScreenMaxK || K > N || N > INT32_MAX - kWave ||
+    if (B < 1 || M < 1 || K < 1 || K > kScreenMaxK || K > N || N > INT32_MAX - kWave ||
         !screen_fits(screen_blocks(M, B), B * N, B))
         return hipErrorInvalidValue;
     ScreenArgs a{};
@@ -1222,12 +1228,39 @@ hipError_t knn3_screen_rows(const float* query, const float* ref, float* dist, i
     a.batch = B;
     a.M = M;
     a.N = N;
-    a.QS = QS;
     a.D = 3;
     a.K = static_cast<int>(K);
     if (workspace == nullptr) return launch_search<1, true, false, false>(a, screen_blocks(M, B), stream);
     screen_workspace(B * N, B, 3, &a.L, workspace);
     return launch_blocks<false>(a, screen_blocks(M, B), stream);
+}
+
+// The nearest reference (squared distance, smallest index) of the first
+// count[b] queries of each cloud's list, M ints a cloud, whose other rows are
+// not written; clouds without any cost two empty launches.
+hipError_t nearest3_screen_listed(const float* query, const float* ref, const int* count, const int* list,
+                                  float* dist2, int64_t* idx, void* workspace, int64_t B, int64_t M,
+                                  int64_t N, hipStream_t stream) {
+    if (B < 1 || M < 1 || N < 1 || N > INT32_MAX - kWave || workspace == nullptr ||
+        !screen_fits(screen_blocks(M, B), B * N, B))
+        return hipErrorInvalidValue;
+    ScreenArgs a{};
+    a.query = query;
+    a.ref = ref;
+    a.dist = dist2;
+    a.idx = idx;
+    a.batch = B;
+    a.M = M;
+    a.N = N;
+    a.list = list;
+    a.list_count = count;
+    a.D = 3;
+    a.K = 1;
+    a.squared = true;
+    screen_workspace(B * N, B, 3, &a.L, workspace);
+    const hipError_t err = launch_prep<false>(a, B * N, stream);
+    if (err != hipSuccess) return err;
+    return launch_search<1, true, false, true, true>(a, screen_blocks(M, B), stream);
 }
 
 }  // namespace pointops
@@ -1258,7 +1291,6 @@ hipError_t pointops_knn_screen(const float* query, const float* ref, float* dist
     a.batch = B;
     a.M = M;
     a.N = N;
-    a.QS = M;
     a.D = static_cast<int>(D);
     a.K = static_cast<int>(K);
     return launch_screen<false>(a, workspace, B * N, blocks, stream);
@@ -1280,7 +1312,6 @@ hipError_t pointops_nearest3_screen(const float* query, const float* ref, float*
     a.batch = B;
     a.M = M;
     a.N = N;
-    a.QS = M;
     a.D = 3;
     a.K = 1;
     a.squared = true;

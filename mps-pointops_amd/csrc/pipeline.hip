@@ -50,7 +50,7 @@ hipError_t fps_dense_progress(const float* xyz, int64_t* out, int64_t B, int64_t
 hipError_t knn3_screen_prepare(const float* ref, void* workspace, int64_t B, int64_t N,
                                hipStream_t stream);
 hipError_t knn3_screen_rows(const float* query, const float* ref, float* dist, int64_t* idx,
-                            void* workspace, int64_t B, int64_t M, int64_t QS, int64_t N, int64_t K,
+                            void* workspace, int64_t B, int64_t M, int64_t N, int64_t K,
                             hipStream_t stream);
 
 namespace {
@@ -239,8 +239,7 @@ hipError_t pointops_fps_query_pipeline_f32(
         }
     }
     if (knn_k > 0) {  // after the last gate: every centre is in place
-        err = knn3_screen_rows(centres, xyz, knn_dist, knn_idx, knn_ws, B, npoint, npoint, N, knn_k,
-                               query_stream);
+        err = knn3_screen_rows(centres, xyz, knn_dist, knn_idx, knn_ws, B, npoint, N, knn_k, query_stream);
         if (err != hipSuccess) return err;
     }
     // Work queued on fps_stream after this call sees every output.

@@ -47,17 +47,12 @@ def _grid_eligible(query: Tensor, ref: Tensor, norm: int, full: bool) -> bool:
             and batch * ((query_count + 63) // 64) < limit)
 
 
-# The matrix-core screen's range of references, in us of the two directions
-# together (a tenth of one side far from the other) against the grid and the
-# scan: 2 x 1024 x 1024 27 / 165 / 86, 16 x 4096 x 4096 93 / 314 / 332, 32 x 8192
-# x 8192 450 / 735 / 1100, 8 x 16384 x 16384 387 / 638 / 1350, 1 x 32768 x 32768
-# 214 / 491 / 2600, 4 x 65536 x 65536 2566 / 1355 / 8700.  (The grid's time
-# depends on the data: 32 x 8192 x 8192 162 us where every query has a close
-# reference, 573 us the other way; the screen takes 225 us either way.)  Its 64
-# queries cost about 20 ns before any reference, so many queries need more
-# references for it to pay: 32 x 1024 queries x 512 references 18 against the
-# scan's 23, 8 x 8192 x 1024 31 against 44, but 32 x 8192 x 512 90 against 40 and
-# x 768 92 against 57 (x 4096 155 against 270).
+# The matrix-core screen's range of references.  Its time does not depend on the
+# data, in us for one direction against the scan: 2 x 1024 x 1024 16 / 43, 16 x 4096
+# x 4096 44 / 165, 8 x 8192 x 8192 62.  Its 64 queries cost about 20 ns before any
+# reference, so many queries need more references for it to pay: 32 x 1024 queries x
+# 512 references 18 against the scan's 23, 8 x 8192 x 1024 31 against 44, but 32 x
+# 8192 x 512 90 against 40 and x 768 92 against 57 (x 4096 155 against 270).
 _SCREEN_MIN_REFS = 512
 _SCREEN_MIN_REFS_MANY = 2048
 _SCREEN_MAX_REFS = 1 << 15
@@ -72,6 +67,19 @@ def _screen_eligible(query: Tensor, ref: Tensor, norm: int, full: bool) -> bool:
             and min(max(_SCREEN_MIN_REFS, blocks), _SCREEN_MIN_REFS_MANY) <= ref_count
             and ref_count <= _SCREEN_MAX_REFS and blocks < limit
             and batch * (ref_count // 32 + 1) < 1 << 30)
+
+
+def _grid_pays(batch: int, query_count: int, ref_count: int) -> bool:
+    """Whether the grid search is the faster one for clouds that lie close to
+    each other, whose few far queries it leaves to the screen: about 10 + 85 ns
+    a million pairs for the screen against 45 us + 0.32 ns a query + 0.13 ns a
+    reference.  Measured, grid (clouds close / a tenth of the queries far) and
+    screen: 32 x 8192 x 8192 169 / 260 and 220 us, 8 x 16384 x 16384 121 / 200 and 190,
+    4 x 32768 x 32768 119 / 248 and 347, 1 x 32768 x 32768 64 / 154 and 98; the
+    other way 16 x 8192 x 8192 103 / 180 and 114, 12 x 8192 x 8192 91 / 155 and 90,
+    32 x 4096 x 8192 113 / 194 and 119."""
+    pairs = batch * query_count * ref_count
+    return 10 + 8.5e-8 * pairs > 45 + batch * (3.2e-4 * query_count + 1.3e-4 * ref_count)
 
 
 def _nearest_screen(query: Tensor, ref: Tensor) -> tuple[Tensor, Tensor]:
@@ -93,8 +101,8 @@ def _nearest_screen(query: Tensor, ref: Tensor) -> tuple[Tensor, Tensor]:
 
 
 def _nearest_grid(query: Tensor, ref: Tensor) -> tuple[Tensor, Tensor]:
-    """pointops_nearest3_grid: the grid search, and a linear scan inside the
-    same call for queries whose nearest reference is several cells away.
+    """pointops_nearest3_grid: the grid search, and the screen inside the same
+    call for queries whose nearest reference is several cells away.
     Results equal the scan kernel's everywhere."""
     batch, query_count, _ = query.shape
     ref_count = ref.shape[1]
@@ -135,10 +143,12 @@ def _nearest_device(query: Tensor, ref: Tensor, query_lengths: Tensor, ref_lengt
     """Distance (squared L2 or L1) and first-minimum index per query row;
     rows beyond the query lengths, and rows of an empty reference cloud, are
     (0, -1) (chamfer.py:122-158).  ``full``: no lengths were given."""
-    if _screen_eligible(query, ref, norm, full):
-        return _nearest_screen(query, ref)
-    if _grid_eligible(query, ref, norm, full):
+    screened = _screen_eligible(query, ref, norm, full)
+    if _grid_eligible(query, ref, norm, full) and not (
+            screened and not _grid_pays(query.shape[0], query.shape[1], ref.shape[1])):
         return _nearest_grid(query, ref)
+    if screened:
+        return _nearest_screen(query, ref)
     return _nearest_scan(query, ref, query_lengths, ref_lengths, norm)
 
 
