@@ -21,11 +21,10 @@ __device__ __forceinline__ float sqdist_nd(const float* __restrict__ r, const fl
     return s;
 }
 
-// The same chain with rows read 16 bytes at a time where `vec` (D % 4 == 0 and
-// both rows 16-byte aligned): a lane's row is then D / 4 requests.
+// The same chain with rows read 16 bytes at a time (D % 4 == 0 and both rows
+// 16-byte aligned): a lane's row is then D / 4 requests.
 __device__ __forceinline__ float sqdist_rows(const float* __restrict__ r, const float* __restrict__ q,
-                                             int D, bool vec) {
-    if (!vec) return sqdist_nd(r, q, D);
+                                             int D) {
     float s = 0.f;  // 0 + d0^2 = d0^2
 #pragma unroll 8
     for (int t = 0; t < D; t += 4) {
@@ -120,9 +119,10 @@ __device__ __forceinline__ void list_tail(const float (&ld)[SLOTS], const int (&
     ti = i;
 }
 
-// One wave: scan n references and keep the K best keys.
-template <int SLOTS, bool DIM3, bool FINITE_ONLY>
-__device__ __forceinline__ void scan_refs(const float* __restrict__ qp, const float* __restrict__ rp,
+// One wave: scan n references and keep the K best keys (VEC: rows as
+// sqdist_rows reads them).
+template <int SLOTS, bool DIM3, bool FINITE_ONLY, bool VEC>
+__device__ __forceinline__ void scan_refs_by(const float* __restrict__ qp, const float* __restrict__ rp,
                                           int n, int D, int K, int lane, float (&ld)[SLOTS],
                                           int (&li)[SLOTS]) {
     float td = INFINITY;
@@ -135,8 +135,6 @@ __device__ __forceinline__ void scan_refs(const float* __restrict__ qp, const fl
         qy = qp[1];
         qz = qp[2];
     }
-    const bool vec = !DIM3 && D % 4 == 0 &&
-                     (reinterpret_cast<uintptr_t>(rp) | reinterpret_cast<uintptr_t>(qp)) % 16 == 0;
     const uint32_t stride = visit_stride(chunks);
     uint32_t chunk = 0;
     for (uint32_t c = 0; c < chunks; ++c) {
@@ -150,7 +148,8 @@ __device__ __forceinline__ void scan_refs(const float* __restrict__ qp, const fl
                 const float* r = rp + 3 * static_cast<int64_t>(j);
                 d = sqdist3(r[0], r[1], r[2], qx, qy, qz);
             } else {
-                d = sqdist_rows(rp + static_cast<int64_t>(j) * D, qp, D, vec);
+                const float* r = rp + static_cast<int64_t>(j) * D;
+                d = VEC ? sqdist_rows(r, qp, D) : sqdist_nd(r, qp, D);
             }
             if (FINITE_ONLY) valid = isfinite(d);
         }
@@ -165,6 +164,16 @@ __device__ __forceinline__ void scan_refs(const float* __restrict__ qp, const fl
             list_tail<SLOTS>(ld, li, K, td, ti);
         }
     }
+}
+
+template <int SLOTS, bool DIM3, bool FINITE_ONLY>
+__device__ __forceinline__ void scan_refs(const float* __restrict__ qp, const float* __restrict__ rp,
+                                          int n, int D, int K, int lane, float (&ld)[SLOTS],
+                                          int (&li)[SLOTS]) {
+    if (!DIM3 && D % 4 == 0 && (reinterpret_cast<uintptr_t>(rp) | reinterpret_cast<uintptr_t>(qp)) % 16 == 0)
+        scan_refs_by<SLOTS, DIM3, FINITE_ONLY, true>(qp, rp, n, D, K, lane, ld, li);
+    else
+        scan_refs_by<SLOTS, DIM3, FINITE_ONLY, false>(qp, rp, n, D, K, lane, ld, li);
 }
 
 }  // namespace
