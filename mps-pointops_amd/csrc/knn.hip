@@ -2,8 +2,8 @@
 //
 // Three designs.  Most searches are screened on the matrix cores
 // (knn_screen.hip).  Of the others, dense 3-D queries with K <= 32 use
-// knn3_lane_kernel (one lane per query, described with the kernel below), and
-// the rest (K up to 256, D != 3, flat/ragged batches) the wave-per-query
+// knn3_lane_kernel (one lane per query, described with the kernel below), as
+// do small clouds of 64 or 128 features (knn_feat_lane_kernel), and the rest (K up to 256, D != 3, flat/ragged batches) the wave-per-query
 // kernels:
 //
 // One wave per query.  Lane l scans reference j = 64*c + l of chunk c; the
@@ -346,6 +346,142 @@ __global__ __launch_bounds__(NW * kWave) void knn3_lane_kernel(
                                  out_idx, static_cast<int64_t>(0xFFFFFFFFu));
 }
 
+// Feature-space kNN of small clouds, K <= KMAX <= 32, D = 64 or 128: one lane
+// per query, the scheme of knn3_lane_kernel (4 waves split the references into
+// 4 contiguous ranges, per-lane sorted lists, shared admission limits).  The
+// query stays in VGPRs; each wave streams its range through a wave-private
+// 4 KiB LDS tile (the next tile is loaded into registers while the current
+// one is scanned) and reads each reference with broadcast LDS loads.
+// Semantics of kernels/feature_knn.metal:51-164: a non-finite query matches
+// nothing, non-finite distances never match (keys below the bits of +inf
+// only), unfilled slots are (inf, -1).  The distance is the sequential
+// s = d0^2; s = s + dt^2 with dt = r - q.
+constexpr int kFeatTileFloats = 1024;
+constexpr uint32_t kInfKey = 0x7F800000u;
+
+template <int KMAX, int D>
+__global__ __launch_bounds__(kLaneThreads) void knn_feat_lane_kernel(
+    const float* __restrict__ query, const float* __restrict__ ref, float* __restrict__ out_dist,
+    int64_t* __restrict__ out_idx, int64_t M, int64_t N, int K) {
+    static_assert(D % 4 == 0 && D <= 128, "feature width");
+    constexpr int TR = kFeatTileFloats / D;                // references per tile
+    constexpr int PER_LANE = kFeatTileFloats / kWave / 4;  // float4 loads per lane per tile
+    constexpr int kGroup = 8;                              // references between drains
+    static_assert(TR % kGroup == 0, "tile holds whole groups");
+    __shared__ uint2 lds[kLaneWaves][KMAX > kLaneCap ? KMAX : kLaneCap][kWave];
+    __shared__ uint32_t taus[kLaneWaves][kWave];
+    __shared__ float4 tiles[kLaneWaves][kFeatTileFloats / 4];
+    const int lane = lane_id();
+    const int wave = uniform(threadIdx.x / kWave);
+    const CloudBlock cb = cloud_block(static_cast<uint32_t>((M + kWave - 1) / kWave));
+    const int64_t b = cb.b;
+    const int64_t m = static_cast<int64_t>(cb.x) * kWave + lane;
+    const bool active = m < M;
+    const float4* qp = reinterpret_cast<const float4*>(query + D * (b * M + (active ? m : 0)));
+    float q[D];
+    bool ok = active;
+#pragma unroll
+    for (int t = 0; t < D / 4; ++t) {
+        const float4 v = qp[t];
+        q[4 * t] = v.x;
+        q[4 * t + 1] = v.y;
+        q[4 * t + 2] = v.z;
+        q[4 * t + 3] = v.w;
+    }
+#pragma unroll
+    for (int t = 0; t < D; ++t) ok = ok && isfinite(q[t]);
+    const float* rp = ref + D * b * N;
+    uint2* buf = &lds[wave][0][0];
+    float4* tile = tiles[wave];
+    const int64_t span = (N + kLaneWaves - 1) / kLaneWaves;
+    const int64_t lo = wave * span;
+    const int64_t hi = min<int64_t>(N, lo + span);
+
+    uint32_t lk[KMAX];
+    int li[KMAX];
+#pragma unroll
+    for (int s = 0; s < KMAX; ++s) {
+        lk[s] = kInfKey;
+        li[s] = -1;
+    }
+    uint32_t tau = ok ? kInfKey : 0u;  // admits finite keys only; nothing for bad queries
+    taus[wave][lane] = tau;
+    __syncthreads();
+    auto limit = [&]() {
+        uint32_t lim = tau;
+#pragma unroll
+        for (int w = 0; w < kLaneWaves; ++w) {
+            if (w == wave) continue;
+            const uint32_t t = taus[w][lane];
+            lim = min(lim, w < wave ? t : t + 1u);
+        }
+        return lim;
+    };
+    // Load the tile of references starting at t0 into registers (zeros past hi).
+    auto fetch = [&](int64_t t0, float4 (&pf)[PER_LANE]) {
+        const int64_t valid = max<int64_t>(0, min<int64_t>(TR, hi - t0)) * D / 4;
+        const float4* src = reinterpret_cast<const float4*>(rp + D * t0);
+#pragma unroll
+        for (int i = 0; i < PER_LANE; ++i) {
+            const int e = i * kWave + lane;
+            pf[i] = e < valid ? src[e] : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    };
+    int cnt = 0;
+    float4 pf[PER_LANE];
+    if (lo < hi) fetch(lo, pf);
+    for (int64_t t0 = lo; t0 < hi; t0 += TR) {
+        // Publish the prefetched tile to this wave's LDS and fetch the next.
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < PER_LANE; ++i) tile[i * kWave + lane] = pf[i];
+        __builtin_amdgcn_wave_barrier();
+        if (t0 + TR < hi) fetch(t0 + TR, pf);
+        const int nref = static_cast<int>(min<int64_t>(TR, hi - t0));
+        for (int g0 = 0; g0 < nref; g0 += kGroup) {
+            const uint32_t lim = limit();
+#pragma unroll
+            for (int u = 0; u < kGroup; ++u) {
+                if (g0 + u >= nref) break;  // uniform
+                const float4* r = tile + (g0 + u) * (D / 4);
+                float sd = 0.f;
+#pragma unroll
+                for (int t = 0; t < D / 4; ++t) {
+                    const float4 v = r[t];  // same address in every lane: broadcast
+                    const float d0 = v.x - q[4 * t], d1 = v.y - q[4 * t + 1];
+                    const float d2 = v.z - q[4 * t + 2], d3 = v.w - q[4 * t + 3];
+                    sd = t == 0 ? d0 * d0 : sd + d0 * d0;
+                    sd = sd + d1 * d1;
+                    sd = sd + d2 * d2;
+                    sd = sd + d3 * d3;
+                }
+                const uint32_t key = static_cast<uint32_t>(f2i(sd));
+                if (key < lim) {
+                    buf[cnt * kWave + lane] = make_uint2(key, static_cast<uint32_t>(t0 + g0 + u));
+                    ++cnt;
+                }
+            }
+            if (ballot(cnt > kLaneCap - kGroup) != 0) {
+                lane_merge<KMAX>(lk, li, tau, K, buf, lane, cnt);
+                cnt = 0;
+                taus[wave][lane] = tau;
+            }
+        }
+    }
+    lane_merge<KMAX>(lk, li, tau, K, buf, lane, cnt);
+    lane_publish_and_merge<KMAX, kLaneWaves, kLaneCap>(lds, lk, li, K, wave, lane, active,
+                                                      (b * M + m) * K, out_dist, out_idx, -1);
+}
+
+template <int KMAX, int D>
+hipError_t launch_feat_lane(const float* query, const float* ref, float* dist, int64_t* idx,
+                            int64_t B, int64_t M, int64_t N, int K, hipStream_t stream) {
+    const dim3 grid(static_cast<uint32_t>((M + kWave - 1) / kWave * B));  // cloud_block order
+    hipLaunchKernelGGL((knn_feat_lane_kernel<KMAX, D>), grid, dim3(kLaneThreads), 0, stream, query,
+                       ref, dist, idx, M, N, K);
+    return hipGetLastError();
+}
+
 template <int KMAX>
 hipError_t launch_lane(const float* query, const float* ref, float* dist, int64_t* idx, int64_t B,
                        int64_t M, int64_t N, int K, hipStream_t stream) {
@@ -360,22 +496,51 @@ hipError_t launch_lane(const float* query, const float* ref, float* dist, int64_
 }
 
 constexpr int64_t kScreenMaxRefs = 16384;
+// The feature lane kernel serves many clouds of few references, where a screened
+// block's phases cost more than its scan (us, lane / wave / screened): D = 64,
+// k = 8 over 16384 x 64 x 16 558 / 1767 / 1436, 8192 x 64 x 32 363 / 1025 / 725,
+// 1024 x 256 x 64 284 / 695 / 343, 455 x 384 x 96 268 / 557 / 248; D = 128, k = 16
+// over 4096 x 128 x 32 650 / 1673 / 1349.  Fewer queries than 24 of a block's 64 leave
+// its lanes idle (16384 x 16 x 16, D = 128 824 / 733 / 1682; not where all blocks fit
+// the chip at once: 256 x 16 x 16 12.6 / 18), as fewer blocks than 128 do the
+// chip: 16 x 64 x 64, D = 64 19 / 14.
+constexpr int64_t kFeatLaneMaxRefs = 127;
+constexpr int64_t kFeatLaneMinBlocks = 128;
+constexpr int64_t kFeatLaneMinRows = 24;
+constexpr int64_t kFeatLaneFewBlocks = 512;
+constexpr int64_t kFeatLaneFewRows = 12;
 
 template <bool DIM3>
 hipError_t launch_dense(const float* query, const float* ref, float* dist, int64_t* idx, int64_t B,
                         int64_t M, int64_t N, int D, int K, hipStream_t stream) {
     const bool lane_grid_ok = (M + kWave - 1) / kWave * B <= INT32_MAX;
     // Small and middling clouds: the screened search (knn_screen.hip) without
-    // a workspace.  Below 256 references (512 for short lists) its phases cost
-    // more than a scan: 128 queries x 256 references, k = 4 16.5 against 11.7
-    // us, 16 x 256 x 384, k = 32 26 against 53 us.  Its screen loosens with
-    // the cloud's extent against its spacing, so large clouds are scanned.
+    // a workspace.  Below 256 references (512 or 768 for short lists) its phases
+    // cost more than a scan: 128 queries x 256 references, k = 4 16.5 against 11.7
+    // us, 32 x 8192 x 512, k = 3 126 against 123, k = 1 103 against 97, but x 768
+    // 129 against 148 and 106 against 119, 16 x 256 x 384, k = 32 26 against 53.
+    // Above 16384 each block would make every reference's operands itself, twice;
+    // the callers with a workspace (pointops_knn_screen) have no such limit.
     if (DIM3 && N >= (K <= 8 ? 512 : 256) && N <= kScreenMaxRefs && K <= 64 && lane_grid_ok)
         return knn3_screen_rows(query, ref, dist, idx, nullptr, B, M, N, K, stream);
     if (DIM3 && K <= 32 && lane_grid_ok) {
         if (K <= 8) return launch_lane<8>(query, ref, dist, idx, B, M, N, K, stream);
         if (K <= 16) return launch_lane<16>(query, ref, dist, idx, B, M, N, K, stream);
         return launch_lane<32>(query, ref, dist, idx, B, M, N, K, stream);
+    }
+    const int64_t lane_blocks = (M + kWave - 1) / kWave;  // a cloud
+    if (!DIM3 && (D == 64 || D == 128) && K <= 32 && N <= kFeatLaneMaxRefs && lane_grid_ok &&
+        lane_blocks * B >= kFeatLaneMinBlocks &&
+        M >= lane_blocks * (lane_blocks * B <= kFeatLaneFewBlocks ? kFeatLaneFewRows : kFeatLaneMinRows) &&
+        (reinterpret_cast<uintptr_t>(query) | reinterpret_cast<uintptr_t>(ref)) % 16 == 0) {
+        if (D == 64) {
+            if (K <= 8) return launch_feat_lane<8, 64>(query, ref, dist, idx, B, M, N, K, stream);
+            if (K <= 16) return launch_feat_lane<16, 64>(query, ref, dist, idx, B, M, N, K, stream);
+            return launch_feat_lane<32, 64>(query, ref, dist, idx, B, M, N, K, stream);
+        }
+        if (K <= 8) return launch_feat_lane<8, 128>(query, ref, dist, idx, B, M, N, K, stream);
+        if (K <= 16) return launch_feat_lane<16, 128>(query, ref, dist, idx, B, M, N, K, stream);
+        return launch_feat_lane<32, 128>(query, ref, dist, idx, B, M, N, K, stream);
     }
     const int64_t rows = B * M;
     const dim3 grid(static_cast<uint32_t>((rows + kKnnWaves - 1) / kKnnWaves));

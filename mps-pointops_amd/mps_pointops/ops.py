@@ -56,15 +56,27 @@ def _screened(B: int, M: int, N: int, D: int, k: int) -> bool:
     """Whether a dense search takes the screened entry point with its own
     workspace.  D = 3 does where neither the windowed entry nor pointops_knn3
     (which screens clouds of up to 16384 references without one) serves it
-    better.  Other D, measured against the scan: 2 x 512 x 512 (D = 33, k = 10)
-    39 against 35 us, 8 x 256 x 256 (D = 68, k = 20) 38 against 28, 8 x 600 x
-    600 (D = 40, k = 20) 44 against 53, 4 x 1000 x 1000 (D = 100, k = 40) 79
-    against 129."""
-    if D > _KNN_SCREEN_MAX_D or k > _KNN_SCREEN_MAX_K or B * N > SCREEN_MAX_ROWS:
-        return False
+    better.
+
+    Other D: a block of the screen costs the same for one query as for 64, a
+    scan as much per query, so it takes enough queries a block.  Screened
+    against scanned, at many clouds (us): D = 8 over 512 references with 8, 16, 32
+    and 64 queries a cloud 299 / 159 / 87 / 53 against 100; D = 64 over 1024 with 1, 8
+    and 16 176 / 93 / 201 against 51 / 119 / 457, over 128 with 8, 16 and 32 328 / 737 /
+    358 against 131 / 481 / 469, over 64 with 32 and 64 671 / 366 against 701 / 697; D =
+    16 over 32 with 64 24 against 31, with 32 37 against 31.  Few queries of a large
+    cloud are a single wave's work each when scanned: 16 x 20000, D = 64 0.55 ms
+    against 2.9.  Clouds of fewer than 96 references with 64 or 128 features are
+    the lane kernel's (pointops_knn_feat)."""
     if D == 3:
-        return N >= _KNN_WINDOW_MIN_N
-    return B * M * N >= _KNN_SCREEN_MIN_PAIRS
+        return N >= _KNN_WINDOW_MIN_N and k <= _KNN_SCREEN_MAX_K and B * N <= SCREEN_MAX_ROWS
+    if (B * M * N < _KNN_SCREEN_MIN_PAIRS or N < 32 or D > _KNN_SCREEN_MAX_D
+            or k > _KNN_SCREEN_MAX_K or B * N > SCREEN_MAX_ROWS
+            or (N < 96 and k <= 32 and D in (64, 128))):
+        return False
+    if N >= 8192 and B * M <= 1024:
+        return True
+    return M >= (48 if N < 64 else 24 if N * D < 1 << 14 else 8) * ((M + 63) // 64)
 
 
 def _check_large_status(workspace: Tensor) -> None:

@@ -35,3 +35,17 @@ def test_nearest_search_takes_the_grid_where_close_clouds_need_it(monkeypatch, B
     q, r = torch.empty(1, 1, 3).expand(B, M, 3), torch.empty(1, 1, 3).expand(B, N, 3)
     chamfer._nearest_device(q, r, None, None, 2, full=True)
     assert taken == [route]
+
+
+@pytest.mark.parametrize("B,M,N,D,k,screened", [
+    (4096, 16, 16, 8, 4, False), (65536, 16, 16, 8, 4, False), (16384, 8, 32, 8, 4, False),
+    (1024, 32, 32, 8, 8, False), (1024, 64, 32, 16, 8, True), (1024, 64, 64, 8, 8, True),
+    (1000, 1, 2000, 8, 8, False), (1024, 16, 1024, 8, 8, False), (1024, 24, 1024, 8, 8, True),
+    (1024, 16, 1024, 64, 8, True), (2048, 1, 1024, 64, 8, False), (64, 1, 20000, 16, 8, True),
+    (512, 64, 64, 64, 16, False), (512, 64, 96, 64, 16, True), (512, 64, 64, 64, 33, True),
+    (8, 2048, 2048, 64, 20, True), (1, 2048, 500, 33, 10, False),
+])
+def test_feature_searches_are_screened_where_a_block_has_queries_enough(B, M, N, D, k, screened):
+    from mps_pointops import ops
+
+    assert ops._screened(B, M, N, D, k) is screened

@@ -141,3 +141,28 @@ def test_queries_left_over_take_no_longer_than_a_scan(cuda_device, shape, kind):
     r = kind(r, torch.Generator().manual_seed(7)).contiguous()
     q = r[:, pick].contiguous()
     assert _best(lambda: mp.knn(q, r, k)) < _best(lambda: _scan(q, r, k))
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,M,N,k", [(128, 24, 1, 1), (128, 24, 33, 8), (64, 90, 95, 9), (3, 3000, 127, 16),
+                                     (130, 64, 64, 17), (128, 63, 32, 32), (200, 12, 31, 8)])
+@pytest.mark.parametrize("kind", ["normal", "copies", "bad"])
+def test_small_feature_clouds_match_oracle(cuda_device, D, B, M, N, k, kind):
+    """The lane kernel's range: the edges of its rule, one to its largest number
+    of references, ties and rows that are not finite."""
+    import numpy as np
+
+    import mps_pointops as mp
+    from oracle import oracle as O
+
+    g = torch.Generator().manual_seed(N + k)
+    r, q = torch.randn(B, N, D, generator=g), torch.randn(B, M, D, generator=g)
+    if kind == "copies":
+        r[:, ::2] = q[:, :1]
+    elif kind == "bad":
+        r[:, 0] = float("nan")
+        q[:, 1, 3] = float("inf")
+    dist, idx = mp.knn(q.cuda(), r.cuda(), k)
+    want_d, want_i = O.knn_feat(q, r, k)
+    np.testing.assert_array_equal(idx.cpu().numpy(), want_i)
+    np.testing.assert_array_equal(dist.cpu().numpy().view(np.int32), np.asarray(want_d).view(np.int32))
