@@ -521,7 +521,7 @@ hipError_t launch_dense(const float* query, const float* ref, float* dist, int64
     // 129 against 148 and 106 against 119, 16 x 256 x 384, k = 32 26 against 53.
     // Above 16384 each block would make every reference's operands itself, twice;
     // the callers with a workspace (pointops_knn_screen) have no such limit.
-    if (DIM3 && N >= (K <= 8 ? 512 : 256) && N <= kScreenMaxRefs && K <= 64 && lane_grid_ok)
+    if (DIM3 && N >= (K <= 3 ? 768 : K <= 8 ? 512 : 256) && N <= kScreenMaxRefs && K <= 64 && lane_grid_ok)
         return knn3_screen_rows(query, ref, dist, idx, nullptr, B, M, N, K, stream);
     if (DIM3 && K <= 32 && lane_grid_ok) {
         if (K <= 8) return launch_lane<8>(query, ref, dist, idx, B, M, N, K, stream);
