@@ -42,9 +42,23 @@ _SCREEN_MIN_PAIRS = 1 << 20
 
 
 def _screened(rows_x: int, rows_y: int, clouds: int, D: int, k: int) -> bool:
-    mean = rows_x / max(clouds, 1)
-    return (D <= _SCREEN_MAX_D and k <= _SCREEN_MAX_K and rows_x <= SCREEN_MAX_ROWS and mean >= (64 if D == 3 else 128)
-            and rows_y * mean >= _SCREEN_MIN_PAIRS)
+    """A block of the screen costs the same for one query as for 64, a scan as
+    much per query, so it takes enough queries a cloud, but for large clouds,
+    whose scan by one wave is long.  Screened against scanned at 2**22 pairs
+    (us): 4096 queries of 1024 clouds of 1024 59 / 26 (k = 8), 64 / 35 (k = 16), of
+    256 clouds 28 / 26 and less, 16384 of 2048 of 256 81 / 50, D = 16, k = 8 over 4096
+    of 256 with 4, 8 and 16 a cloud 296 / 181 / 115 against 120, D = 64, k = 8 over 128
+    with 2, 4 and 8 1262 / 664 / 340 against 988 / 583 / 350; k = 1 needs more pairs
+    than two launches cost (2**20: 16 against 12)."""
+    if (rows_x > SCREEN_MAX_ROWS or D > _SCREEN_MAX_D or k > _SCREEN_MAX_K
+            or rows_x < (64 if D == 3 else 128) * clouds):
+        return False
+    pairs = rows_y * rows_x // max(clouds, 1)
+    if pairs < _SCREEN_MIN_PAIRS * (4 if k < 4 and D == 3 else 1):
+        return False
+    if rows_x >= 8192 * clouds:
+        return True
+    return rows_y >= (8 if D >= 64 else 16 if D == 3 and k >= 16 else 24) * clouds
 
 
 _MAX_CLOUD = (1 << 32) - 1  # longest cloud a ragged FPS launch indexes
