@@ -72,14 +72,16 @@ def _screen_eligible(query: Tensor, ref: Tensor, norm: int, full: bool) -> bool:
 def _grid_pays(batch: int, query_count: int, ref_count: int) -> bool:
     """Whether the grid search is the faster one for clouds that lie close to
     each other, whose few far queries it leaves to the screen: about 10 + 85 ns
-    a million pairs for the screen against 45 us + 0.32 ns a query + 0.13 ns a
-    reference.  Measured, grid (clouds close / a tenth of the queries far) and
-    screen: 32 x 8192 x 8192 169 / 260 and 220 us, 8 x 16384 x 16384 121 / 200 and 190,
-    4 x 32768 x 32768 119 / 248 and 347, 1 x 32768 x 32768 64 / 154 and 98; the
-    other way 16 x 8192 x 8192 103 / 180 and 114, 12 x 8192 x 8192 91 / 155 and 90,
-    32 x 4096 x 8192 113 / 194 and 119."""
-    pairs = batch * query_count * ref_count
-    return 10 + 8.5e-8 * pairs > 45 + batch * (3.2e-4 * query_count + 1.3e-4 * ref_count)
+    a million pairs (or, with few queries, the 1.5 ns a reference that one block
+    takes) for the screen against 45 us + 0.32 ns a query + 0.13 ns a reference.
+    Measured, grid (clouds close / a tenth of the queries far) and screen: 32 x
+    8192 x 8192 169 / 260 and 220 us, 8 x 16384 x 16384 121 / 200 and 190, 4 x 32768 x
+    32768 119 / 248 and 347, 1 x 32768 x 32768 64 / 154 and 98, 1 x 4096 x 32768 49 to
+    61 / 140 and 60; the other way 16 x 8192 x 8192 103 / 180 and 114, 12 x 8192 x
+    8192 91 / 155 and 90, 32 x 4096 x 8192 113 / 194 and 119, 1 x 16384 x 16384 57 / 150
+    and 38."""
+    screen = 10 + max(8.5e-8 * batch * query_count * ref_count, 1.5e-3 * ref_count)
+    return screen > 45 + batch * (3.2e-4 * query_count + 1.3e-4 * ref_count)
 
 
 def _nearest_screen(query: Tensor, ref: Tensor) -> tuple[Tensor, Tensor]:

@@ -18,7 +18,8 @@ def test_searches_beyond_the_screens_limits_are_scanned(rows):
 
 @pytest.mark.parametrize("B,M,N,route", [
     (32, 8192, 8192, "grid"), (8, 16384, 16384, "grid"), (1, 32768, 32768, "grid"),
-    (4, 32768, 32768, "grid"), (1, 100_000, 100_000, "grid"), (8, 4096, 32768, "grid"),
+    (4, 32768, 32768, "grid"), (1, 100_000, 100_000, "grid"), (8, 4096, 32768, "grid"), (1, 4096, 32768, "grid"),
+    (1, 16384, 16384, "screen"),
     (8, 8192, 8192, "screen"), (16, 4096, 4096, "screen"), (1, 1000, 32768, "screen"),
     (32, 4096, 8192, "screen"), (32, 8192, 512, "scan"), (4, 300, 300, "scan"),
 ])
@@ -49,3 +50,16 @@ def test_feature_searches_are_screened_where_a_block_has_queries_enough(B, M, N,
     from mps_pointops import ops
 
     assert ops._screened(B, M, N, D, k) is screened
+
+
+@pytest.mark.parametrize("clouds,x,y,D,k,screened", [
+    (16384, 64, 1, 3, 8, False), (1024, 256, 8, 3, 8, False), (1024, 256, 24, 3, 8, True),
+    (1024, 1024, 4, 3, 16, False), (256, 1024, 16, 3, 16, True), (53, 20000, 1, 3, 16, True),
+    (32, 1024, 32, 3, 1, False), (128, 1024, 32, 3, 1, True), (4096, 128, 8, 16, 8, False),
+    (512, 256, 24, 16, 8, True), (8192, 128, 4, 64, 16, False), (2048, 128, 8, 64, 16, True),
+    (3, 20000, 20000, 3, 16, True), (32, 1000, 1000, 3, 16, True), (5000, 16, 16, 3, 8, False),
+])
+def test_ragged_searches_are_screened_where_a_cloud_has_queries_enough(clouds, x, y, D, k, screened):
+    from mps_pointops import flat
+
+    assert flat._screened(clouds * x, clouds * y, clouds, D, k) is screened
