@@ -1154,16 +1154,17 @@ size_t screen_workspace(int64_t rows, int64_t batch, int64_t D, ScreenLayout* L 
 }
 
 // The references' fragments (into a.L), which depend on the references alone.
+// `lds`: bytes the blocks take without using them.
 template <bool FLAT>
-hipError_t launch_prep(const ScreenArgs& a, int64_t ref_rows, hipStream_t stream) {
+hipError_t launch_prep(const ScreenArgs& a, int64_t ref_rows, hipStream_t stream, size_t lds = 0) {
     const int64_t tiles = FLAT ? screen_tiles(ref_rows, a.batch) : a.batch * ((a.N + kTileRefs - 1) / kTileRefs);
     constexpr int kPrepWaves = kPrepThreads / kWave;
     const dim3 grid(static_cast<uint32_t>((tiles + kPrepWaves - 1) / kPrepWaves));
     if (a.D == 3)
-        hipLaunchKernelGGL((screen_prep_kernel<true, FLAT>), grid, dim3(kPrepThreads), 0, stream, a.ref,
+        hipLaunchKernelGGL((screen_prep_kernel<true, FLAT>), grid, dim3(kPrepThreads), lds, stream, a.ref,
                            a.ptr_x, a.list_count, a.L, a.batch, a.N, tiles, a.D, 1);
     else
-        hipLaunchKernelGGL((screen_prep_kernel<false, FLAT>), grid, dim3(kPrepThreads), 0, stream, a.ref,
+        hipLaunchKernelGGL((screen_prep_kernel<false, FLAT>), grid, dim3(kPrepThreads), lds, stream, a.ref,
                            a.ptr_x, a.list_count, a.L, a.batch, a.N, tiles, a.D, screen_kernel_steps(a.D));
     return hipGetLastError();
 }
@@ -1211,7 +1212,9 @@ hipError_t knn3_screen_prepare(const float* ref, void* workspace, int64_t B, int
     a.N = N;
     a.D = 3;
     screen_workspace(B * N, B, 3, &a.L, workspace);
-    return launch_prep<false>(a, B * N, stream);
+    // Beside a pipelined FPS, which reserves the LDS of its CUs so that no other
+    // block takes issue slots there: this kernel has none of its own.
+    return launch_prep<false>(a, B * N, stream, 1024);
 }
 
 hipError_t knn3_screen_rows(const float* query, const float* ref, float* dist, int64_t* idx,
