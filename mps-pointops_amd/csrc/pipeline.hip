@@ -14,11 +14,10 @@
 // queries of that chunk follow on the free CUs while FPS goes on, every
 // radius in one scan (ball_query_multi_kernel: each distance computed once,
 // each radius's first-K list as its own search would build it).  kNN runs
-// once, over all centres, after the last chunk: its lane kernel gives each
-// workgroup 64 queries against the whole cloud, so its duration does not
-// shrink with the number of queries (measured at config 2: about 62 us for
-// 128 centres per cloud, 86 us for 1024), and per-chunk launches would
-// serialise that cost.  Results are those of the separate calls, bit for
+// once, over all centres, after the last chunk, screened on the matrix cores
+// (41 us at config 2), its references' operands made first, beside FPS: each
+// workgroup takes 64 queries against the whole cloud, so a launch per chunk
+// would last as long as one over all centres that fit the chip at once.  Results are those of the separate calls, bit for
 // bit: each query's distances and tests are the same.
 //
 // The only waiting is the gates' bounded poll of the progress words; FPS

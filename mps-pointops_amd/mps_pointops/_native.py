@@ -165,7 +165,9 @@ def stream(device: torch.device) -> int:
 
 
 def call(name: str, *args) -> None:
-    """Enqueue an operator's entry point; RuntimeError on a non-zero status."""
+    """Enqueue an entry point that computes an operator's results; RuntimeError
+    on a non-zero status.  (The argument checks below go to _enqueue directly,
+    so that replacing ``call`` shows which kernels a result came from.)"""
     _enqueue(name, *args)
 
 

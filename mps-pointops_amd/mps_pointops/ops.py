@@ -34,7 +34,8 @@ _KNN_GRID_MAX_K = 32
 _KNN_GRID_MIN_N = 32_768
 _KNN_GRID_MIN_PAIRS = 1 << 26
 # 3-D kNN with at most 32 neighbours over clouds of 2048 to 8192 references
-# (and at most 16384 queries per cloud) goes to pointops_knn3_windowed: same
+# (and at most 16384 queries per cloud) goes to pointops_knn3_windowed, the
+# screened search under the limits that entry point has always had: same
 # results; below 2048 references the launch that prepares them does not pay.
 _KNN_WINDOW_MAX_K = 32
 _KNN_WINDOW_MIN_N = 2048

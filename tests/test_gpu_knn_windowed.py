@@ -1,9 +1,9 @@
-"""GPU parity of the Morton-window 3-D kNN (pointops_knn3_windowed) against
+"""GPU parity of pointops_knn3_windowed (screened on the matrix cores) against
 the oracle.
 
-The starting limit only decides which references are buffered; indices must
-equal the brute-force answer of kernels/knn.metal:32-140 bit for bit, and the
-distances (sqrt of the same fl32 squared distance) bit for bit as well.
+The screen only decides which references are ranked; indices must equal the
+brute-force answer of kernels/knn.metal:32-140 bit for bit, and the distances
+(sqrt of the same fl32 squared distance) bit for bit as well.
 Cases cover the shapes the entry point accepts (N <= 8192, M <= 16384,
 K <= 32), the template boundaries of K (8, 16, 32), ties and duplicates,
 points outside the references' box, degenerate extents and non-finite
@@ -47,6 +47,19 @@ def knn3_windowed(query: torch.Tensor, ref: torch.Tensor, k: int):
     _native.call("pointops_knn3_windowed", q.data_ptr(), r.data_ptr(), dist.data_ptr(),
                  idx.data_ptr(), ws.data_ptr(), B, M, N, k, _native.stream(q.device))
     return host(dist), host(idx)
+
+
+def scanned(query: torch.Tensor, ref: torch.Tensor, k: int):
+    """The first k of 65 neighbours, which pointops_knn3 scans for instead of
+    screening."""
+    from mps_pointops import _native
+
+    B, M, _ = query.shape
+    dist = torch.empty(B, M, 65, device="cuda")
+    idx = torch.empty(B, M, 65, dtype=torch.long, device="cuda")
+    _native.library().pointops_knn3(query.data_ptr(), ref.data_ptr(), dist.data_ptr(), idx.data_ptr(),
+                                    B, M, ref.shape[1], 65, _native.stream(query.device))
+    return host(dist)[..., :k], host(idx)[..., :k]
 
 
 def _case(name: str):
@@ -164,23 +177,18 @@ def test_knn3_windowed_random_sweep(cuda_device, seed, k):
 
 def test_knn3_windowed_config2_full_equals_lane_kernel(cuda_device):
     """Config 2 at full size (B=32, FPS centres as queries, K=16): the
-    windowed search equals the plain kernel, twice in a row on one workspace
-    (nothing carried over between calls)."""
+    windowed search equals the scan, twice in a row (nothing carried over
+    between calls)."""
     import mps_pointops as mp
-    from mps_pointops import _native
 
     x = bench.make_c2().cuda()
     centres = x.gather(1, mp.furthest_point_sample(x, 1024)[..., None].expand(-1, -1, 3))
     centres = centres.contiguous()
-    B, M, N, K = 32, 1024, 4096, 16
-    bd = torch.empty(B, M, K, device="cuda")
-    bi = torch.empty(B, M, K, dtype=torch.long, device="cuda")
-    _native.call("pointops_knn3", centres.data_ptr(), x.data_ptr(), bd.data_ptr(), bi.data_ptr(),
-                 B, M, N, K, _native.stream(x.device))
+    bd, bi = scanned(centres, x, 16)
     for _ in range(2):
-        d, i = knn3_windowed(centres, x, K)
-        np.testing.assert_array_equal(i, host(bi))
-        same_bits(d, host(bd))
+        d, i = knn3_windowed(centres, x, 16)
+        np.testing.assert_array_equal(i, bi)
+        same_bits(d, bd)
 
 
 def test_knn3_windowed_rejects_out_of_range(cuda_device):
@@ -203,7 +211,7 @@ def test_knn3_windowed_rejects_out_of_range(cuda_device):
 
 def test_public_knn_takes_windowed_path(cuda_device, monkeypatch):
     """ops.knn sends config-2-sized clouds to the windowed entry point and
-    smaller ones (config 1) to the plain kernel; both equal the plain kernel."""
+    smaller ones (config 1) to the plain one; both equal the scan."""
     import mps_pointops as mp
     from mps_pointops import _native
 
@@ -222,9 +230,6 @@ def test_public_knn_takes_windowed_path(cuda_device, monkeypatch):
         calls.clear()
         d, i = mp.knn(query, ref, 16)
         assert calls == [want]
-        bd = torch.empty_like(d)
-        bi = torch.empty_like(i)
-        real_call("pointops_knn3", query.data_ptr(), ref.data_ptr(), bd.data_ptr(), bi.data_ptr(),
-                  4, 300, n, 16, _native.stream(query.device))
-        np.testing.assert_array_equal(host(i), host(bi))
-        same_bits(host(d), host(bd))
+        bd, bi = scanned(query, ref, 16)
+        np.testing.assert_array_equal(host(i), bi)
+        same_bits(host(d), bd)

@@ -719,10 +719,10 @@ def test_knn_feat_matches_oracle(cuda_device, dim, k):
 @pytest.mark.parametrize("m,n,k", [(1, 1, 1), (63, 15, 8), (65, 17, 9), (130, 100, 16),
                                    (70, 1000, 17), (64, 2049, 32), (3, 40, 33)])
 def test_knn_feat_lane_path(cuda_device, m, n, k, dim):
-    """D=64 and D=128 with K<=32 run one lane per query with LDS reference
-    tiles: ragged tiles and wave ranges, duplicate references (ties),
-    non-finite queries and references, and K=33 (wave-per-query path)
-    against the oracle."""
+    """D=64 and D=128 around the tiles, wave ranges and list lengths of their
+    kernels (few clouds: scanned or screened; the lane kernel's own range is
+    in test_gpu_knn_awkward.py): duplicate references (ties), non-finite
+    queries and references, against the oracle."""
     import mps_pointops as mp
 
     if k > n:
