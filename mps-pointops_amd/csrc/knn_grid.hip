@@ -720,10 +720,12 @@ __device__ __forceinline__ float box_bound(const GridParams& P, float h, const f
     return b;
 }
 
-template <int S>
+// NEAREST (S = 1, K = 1): squared distances, and the limits after which a query
+// is left to the screen (max_scan 0: after max_grow faces only).
+template <int S, bool NEAREST>
 __global__ __launch_bounds__(kGridSearchWaves * kWave) void knn3_grid_kernel(
     const float* __restrict__ query, GridLayout L, float* __restrict__ out_dist,
-    int64_t* __restrict__ out_idx, int64_t B, int64_t M, int64_t N, int K, int nearest, int max_grow, int max_scan) {
+    int64_t* __restrict__ out_idx, int64_t B, int64_t M, int64_t N, int K, int max_grow, int max_scan) {
     constexpr int KMAX = 4 * S;
     __shared__ uint2 bufs[kGridSearchWaves][kGridCap][kWave];
     const int lane = lane_id();
@@ -832,7 +834,8 @@ __global__ __launch_bounds__(kGridSearchWaves * kWave) void knn3_grid_kernel(
                     done = true;
                 } else if (qc != 0) {
                     want = true;  // merge first, then check again
-                } else if (grow == max_grow || (max_scan != 0 && tau == ~0ull)) {
+                } else if (grow == (NEAREST ? max_grow : kGridMaxGrow) ||
+                           (NEAREST && max_scan != 0 && tau == ~0ull)) {
                     listed = true;
                     done = true;
                 } else {
@@ -865,7 +868,7 @@ __global__ __launch_bounds__(kGridSearchWaves * kWave) void knn3_grid_kernel(
             for (int u = 0; u < 8; ++u) rv[u] = srt[min(base + 4 * u, last)];
             admit8s(rv, has ? e - base : 0);
             if (has) p += 32;
-            if (max_scan != 0 && has && (scanned += 32) > max_scan) {
+            if (NEAREST && max_scan != 0 && has && (scanned += 32) > max_scan) {
                 listed = done = true;
                 p = e;
             }
@@ -894,7 +897,7 @@ __global__ __launch_bounds__(kGridSearchWaves * kWave) void knn3_grid_kernel(
         if (r >= 0) {
             const uint32_t key = static_cast<uint32_t>(slot[s] >> 32);
             const float d2 = i2f(static_cast<int>(key));
-            out_dist[row + r] = slot[s] == ~0ull ? INFINITY : (nearest ? d2 : sqrtf(d2));
+            out_dist[row + r] = slot[s] == ~0ull ? INFINITY : (NEAREST ? d2 : sqrtf(d2));
             out_idx[row + r] = static_cast<int64_t>(static_cast<uint32_t>(slot[s]));
         }
     }
@@ -1513,13 +1516,13 @@ hipError_t pointops_knn3_grid(const float* query, const float* ref, float* dist,
     const dim3 block(kGridSearchWaves * kWave);
     const int k = static_cast<int>(K);
     if (K <= 4)
-        hipLaunchKernelGGL((knn3_grid_kernel<1>), grid, block, 0, stream, query, L, dist, idx, B, M, N, k, 0, kGridMaxGrow, 0);
+        hipLaunchKernelGGL((knn3_grid_kernel<1, false>), grid, block, 0, stream, query, L, dist, idx, B, M, N, k, 0, 0);
     else if (K <= 8)
-        hipLaunchKernelGGL((knn3_grid_kernel<2>), grid, block, 0, stream, query, L, dist, idx, B, M, N, k, 0, kGridMaxGrow, 0);
+        hipLaunchKernelGGL((knn3_grid_kernel<2, false>), grid, block, 0, stream, query, L, dist, idx, B, M, N, k, 0, 0);
     else if (K <= 16)
-        hipLaunchKernelGGL((knn3_grid_kernel<4>), grid, block, 0, stream, query, L, dist, idx, B, M, N, k, 0, kGridMaxGrow, 0);
+        hipLaunchKernelGGL((knn3_grid_kernel<4, false>), grid, block, 0, stream, query, L, dist, idx, B, M, N, k, 0, 0);
     else
-        hipLaunchKernelGGL((knn3_grid_kernel<8>), grid, block, 0, stream, query, L, dist, idx, B, M, N, k, 0, kGridMaxGrow, 0);
+        hipLaunchKernelGGL((knn3_grid_kernel<8, false>), grid, block, 0, stream, query, L, dist, idx, B, M, N, k, 0, 0);
     grid_list(L, B, M, N, true, stream);
     const dim3 listed(static_cast<uint32_t>(B * ((M + kWave - 1) / kWave)));
     const dim3 lblock(kListedWaves * kWave);
@@ -1547,8 +1550,8 @@ hipError_t pointops_nearest3_grid(const float* query, const float* ref, float* d
     grid_build(query, ref, L, B, M, N, 1, 0.f, 1, stream);
     grid_list_zero(L, B, stream);
     const bool quit = N <= kGridQuitRefs;
-    hipLaunchKernelGGL((knn3_grid_kernel<1>), grid, dim3(kGridSearchWaves * kWave), 0, stream, query,
-                       L, dist2, idx, B, M, N, 1, 1, quit ? kGridQuitGrow : kGridNearestGrow, quit ? kGridQuitScan : 0);
+    hipLaunchKernelGGL((knn3_grid_kernel<1, true>), grid, dim3(kGridSearchWaves * kWave), 0, stream, query,
+                       L, dist2, idx, B, M, N, 1, quit ? kGridQuitGrow : kGridNearestGrow, quit ? kGridQuitScan : 0);
     grid_list(L, B, M, N, false, stream);
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
