@@ -166,3 +166,54 @@ def test_small_feature_clouds_match_oracle(cuda_device, D, B, M, N, k, kind):
     want_d, want_i = O.knn_feat(q, r, k)
     np.testing.assert_array_equal(idx.cpu().numpy(), want_i)
     np.testing.assert_array_equal(dist.cpu().numpy().view(np.int32), np.asarray(want_d).view(np.int32))
+
+
+@pytest.mark.parametrize("kind", [_copies, _clusters, _lattice])
+@pytest.mark.parametrize("D,k", [(3, 1), (3, 64), (20, 16)])
+@pytest.mark.parametrize("sizes_x,sizes_y", [([9000, 31, 0, 4064], [70, 3, 5, 130]), ([12097], [700])])
+def test_ragged_queries_left_over(cuda_device, kind, D, k, sizes_x, sizes_y):
+    """The same over ragged clouds, of one and several ranges of tiles."""
+    from mps_pointops import _native
+
+    g = torch.Generator().manual_seed(k + D)
+    x = kind(torch.rand(1, sum(sizes_x), D, generator=g).cuda(), g)[0].contiguous()
+    y = x[torch.randint(0, len(x), (sum(sizes_y),), generator=g).cuda()].contiguous()
+    px, py = (torch.tensor([0, *s]).cumsum(0).cuda() for s in (sizes_x, sizes_y))
+    want, got = (torch.full((len(y), k), f, dtype=torch.long, device="cuda") for f in (-7, -8))
+    st = _native.stream(x.device)
+    args = (y.data_ptr(), x.data_ptr(), py.data_ptr(), px.data_ptr())
+    _native.call("pointops_knn_flat", *args, want.data_ptr(), len(y), len(sizes_x), D, k, st)
+    ws = torch.empty(_native.size_query("pointops_knn_flat_screen_workspace_bytes", len(x), len(sizes_x), D),
+                     dtype=torch.uint8, device="cuda")
+    _native.call("pointops_knn_flat_screen", *args, got.data_ptr(), ws.data_ptr(), len(y), len(x),
+                 len(sizes_x), D, k, st)
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("B,M,N", [(2, 4096, 9000), (1, 5000, 32768), (1, 4100, 33000)])
+@pytest.mark.parametrize("kind", ["stray", "shift", "far", "copies", "lattice"])
+def test_nearest_by_the_grid_and_the_screen(cuda_device, B, M, N, kind):
+    """Queries that the grid leaves to the screen (none, some, all of them, and
+    those of crowded cells), on both sides of its limits' line, against the scan."""
+    from mps_pointops import chamfer
+
+    g = torch.Generator().manual_seed(N)
+    r = torch.randn(B, N, 3, generator=g)
+    r = r / r.norm(dim=-1, keepdim=True)
+    q = r[:, torch.randint(0, N, (M,), generator=g)] + 0.01 * torch.randn(B, M, 3, generator=g)
+    if kind == "stray":
+        r[:, 7] = 50.0
+    elif kind == "shift":
+        q = q + 0.4
+    elif kind == "far":
+        q[:, ::10] = 2 * torch.rand(B, len(range(0, M, 10)), 3, generator=g) - 1
+    elif kind == "copies":
+        r[:, N // 2:], q[:, M // 2:] = 0.0, 0.0
+    elif kind == "lattice":
+        r, q = (r * 10).round(), (q * 10).round() + 0.5
+    q, r = q.cuda().contiguous(), r.cuda().contiguous()
+    lengths = [torch.full((B,), n, dtype=torch.int64, device=q.device) for n in (M, N)]
+    d, i = chamfer._nearest_grid(q, r)
+    want_d, want_i = chamfer._nearest_scan(q, r, *lengths, 2)
+    assert torch.equal(i, want_i)
+    assert torch.equal(d.view(torch.int32), want_d.view(torch.int32))
